@@ -164,3 +164,42 @@ def test_template_tables_are_kept_and_follow_their_source(hip):
     check_status()
     twice = torch.cat([k[:, :, :768], k[:, :, :256]], dim=2), torch.cat([v[:, :, :768], v[:, :, :256]], dim=2)
     assert _rel(o, numerics.sdpa_fp32(q, *twice, 0.1)) <= 1.2e-2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["explicit", "auto", "causal auto", "producer"])
+def test_same_tables_with_another_number_of_waves(hip, form):
+    """What the launcher worked out for the first NUM_WAVES rows of a set of tables is not taken for another number of
+    rows: eight waves that share their q rows, then the same table objects with eight more over other rows."""
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.attn import attention_forward
+
+    H, half, chunk, causal = 8, 1024, 256 if form == "causal auto" else 1024, form == "causal auto"
+    Sq = 2 * half
+    Skv = Sq if causal else 8 * chunk
+    if form == "producer":
+        offsets = [[0, 0, i * 128 * 2, 0] for i in range(8)]
+        sizes = [[1, H, 256, Skv]] * 8
+        steps, signals = (4, 8, 4), list(range(8))
+    else:
+        offsets = [[0, 0, rows, i * chunk] for rows in (0, half) for i in range(8)]
+        sizes = [[1, H, half, chunk]] * 16
+        steps, signals = (8, 16, 8), [-1] * 16
+    cums = [sum(s[0] * s[1] * s[2] for s in sizes[:i + 1]) for i in range(len(sizes))]
+    q, k, v, _ = _inputs(1, H, Sq, Skv, torch.bfloat16)
+    want = numerics.sdpa_fp32(q, k, v, 0.1, causal=causal)
+    table = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    tables = dict(wave_offsets=table(offsets), wave_sizes=table(sizes), cum_wave_sizes=table(cums), signal_offsets=table(signals))
+    qd, kd, vd = q.cuda(), k.cuda(), v.cuda()
+    for waves in steps:
+        out = torch.full_like(qd, float("nan"))
+        kw = dict(form="auto") if "auto" in form else {}
+        if form == "producer":
+            kw = dict(counter_ptr=torch.zeros(8, dtype=torch.int32, device="cuda"))
+        attention_forward(qd, kd, vd, 0.1, NUM_WAVES=waves, cum_tiles=cums[waves - 1], out=out, causal=causal,
+                          signal_ptr=torch.zeros(8, dtype=torch.int64, device="cuda"), **kw, **tables)
+        check_status()
+        rows = max(o[2] + s[2] for o, s in zip(offsets[:waves], sizes))
+        # one rounding of the result and of the probabilities, three times that; see test_parts_add_up
+        assert _rel(out[:, :, :rows], want[:, :, :rows]) <= 1.2e-2
+        assert bool(out[:, :, rows:].isnan().all())
