@@ -76,6 +76,9 @@ extern "C" {
                                        gemm/template.py:92-97,121-128); callers that cannot promise (1) and (2)
                                        set this bit. */
 
+#define SYN_GEMM_CUT_TILE 128u      /* cut_m and cut_n hold; without it they are not read (a descriptor may
+                                       then end behind `options`, as it did before version 200)   */
+
 typedef void* syn_stream_t;        /* hipStream_t */
 
 /*
@@ -107,8 +110,9 @@ typedef struct syn_gemm_desc {
     int64_t cum_tiles;              /* sum rows*cols over waves (elements); 0 = M*N        */
     int64_t spin_timeout_us;        /* <=0: default (2 s); flag waits give up after this   */
     uint32_t options;               /* SYN_GEMM_* bits                                     */
-    int32_t cut_m, cut_n;           /* where block_m x block_n is a piece of a larger tile whose result is wanted
-                                       bit for bit: log2 of the pieces along m and n (0: it is the tile)   */
+    int32_t cut_m, cut_n;           /* with SYN_GEMM_CUT_TILE, else not read: block_m x block_n is a piece of a larger
+                                       tile whose result is wanted bit for bit: log2 of the pieces along m and n,
+                                       0 to 4                                                            */
 } syn_gemm_desc;
 
 /*
@@ -309,7 +313,8 @@ typedef struct syn_attn_desc {
                                        tests/test_all2all_attn_all2all.py:192-210)                    */
     const int32_t* work_list;       /* with SYN_ATTN_WORK_LIST, else NULL: device int32: num_programs + 1 entry
                                        offsets, then the entries (see SYN_ATTN_WORK_LIST)              */
-    int32_t split_parts;            /* with SYN_ATTN_SPLIT_KV, else ignored: most parts a pair is cut into  */
+    int32_t split_parts;            /* the split_* fields: with SYN_ATTN_SPLIT_KV, else not read (a descriptor may then
+                                       end behind work_list, as before version 200); most parts a pair is cut into  */
     int32_t split_blocks;           /* kv blocks a part should have                                         */
     int32_t* split_nodes;           /* split_parts > 1: device int32[pairs * split_parts], zeroed            */
     void* split_partials;           /* split_parts > 1: device, 16-byte aligned, SYN_ATTN_SPLIT_SLOT_BYTES for each

@@ -196,7 +196,8 @@ def _launch(
         | (_lib.SYN_GEMM_RING_PIPE if ring_pipe else 0) | (0 if k_stagger else _lib.SYN_GEMM_NO_K_STAGGER)
         | (_lib.SYN_GEMM_TWO_STAGE if two_stage else 0) | (_lib.SYN_GEMM_MFMA_32X32 if mfma_32x32 else 0)
         | (_lib.SYN_GEMM_ACQUIRE_ALWAYS
-           if acquire_always(wait_signal_buffer if wait_signal_buffer is not None else signal_buffer) else 0),
+           if acquire_always(wait_signal_buffer if wait_signal_buffer is not None else signal_buffer) else 0)
+        | (_lib.SYN_GEMM_CUT_TILE if cut != (0, 0) else 0),
         cut_m=cut[0], cut_n=cut[1],
     )
     with device_scope(dev):

@@ -230,7 +230,8 @@ def gemm_remote(
         dtype=_lib.dtype_code(b.dtype), block_m=BLOCK_SIZE_M, block_n=BLOCK_SIZE_N, block_k=BLOCK_SIZE_K,
         group_m=GROUP_SIZE_M, num_sms=num_gemm_sms, cum_tiles=int(cum_tiles), spin_timeout_us=0,
         options=(_lib.SYN_GEMM_XCD_REMAP if xcd_remap else 0) | (_lib.SYN_GEMM_EIGHT_WAVES if eight_waves else 0)
-        | (_lib.SYN_GEMM_ACQUIRE_ALWAYS if signal_ptr is not None and acquire_always(signal_ptr) else 0),
+        | (_lib.SYN_GEMM_ACQUIRE_ALWAYS if signal_ptr is not None and acquire_always(signal_ptr) else 0)
+        | (_lib.SYN_GEMM_CUT_TILE if cut != (0, 0) else 0),
         cut_m=cut[0], cut_n=cut[1],
     )
     with device_scope(dev):

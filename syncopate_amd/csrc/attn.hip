@@ -1877,10 +1877,15 @@ int syn_attn_fwd(const syn_attn_desc* d, syn_stream_t stream) {
     p.xcd_remap = (d->options & SYN_ATTN_XCD_REMAP) ? 1 : 0;
     p.acquire_always = (d->options & SYN_ATTN_ACQUIRE_ALWAYS) ? 1 : 0;
     p.work_list = d->work_list;
-    p.split_parts = d->split_parts;
-    p.split_blocks = d->split_blocks;
-    p.split_nodes = d->split_nodes;
-    p.split_partials = reinterpret_cast<unsigned char*>(d->split_partials);
+    p.split_parts = p.split_blocks = 0;
+    p.split_nodes = nullptr;
+    p.split_partials = nullptr;
+    if (d->options & SYN_ATTN_SPLIT_KV) {         // (without the bit the descriptor may end in front of these fields)
+        p.split_parts = d->split_parts;
+        p.split_blocks = d->split_blocks;
+        p.split_nodes = d->split_nodes;
+        p.split_partials = reinterpret_cast<unsigned char*>(d->split_partials);
+    }
     p.qk_scale = d->sm_scale * 1.44269504f;
     {
         // all-zero strides: contiguous [Z, H, S, D]

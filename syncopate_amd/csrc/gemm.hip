@@ -28,6 +28,8 @@
 // the flag word, then the whole workgroup takes an acquire fence (template.py:121-128).
 // Producer form: after the C tile is stored the workgroup bumps counters[wave] and the last
 // tile of the wave publishes the flag (template.py:343-348).
+#include <cstddef>
+#include <cstring>
 #include <mutex>
 
 #include "common.h"
@@ -1458,9 +1460,12 @@ static int gemm_entry(const syn_gemm_desc* d, hipStream_t stream, int mode,
     p.c_ld = c_remote ? remote->c_ld : 0;
     p.c_atomic = (remote && remote->c_atomic_add) ? 1 : 0;
     p.wave_k = remote ? remote->k_ranges : nullptr;
-    if (d->cut_m < 0 || d->cut_m > 4 || d->cut_n < 0 || d->cut_n > 4) return SYN_EINVAL;
-    p.cut_m = d->cut_m;
-    p.cut_n = d->cut_n;
+    p.cut_m = p.cut_n = 0;
+    if (d->options & SYN_GEMM_CUT_TILE) {         // (without the bit the descriptor may end in front of these fields)
+        if (d->cut_m < 0 || d->cut_m > 4 || d->cut_n < 0 || d->cut_n > 4) return SYN_EINVAL;
+        p.cut_m = d->cut_m;
+        p.cut_n = d->cut_n;
+    }
     const bool eight = (d->options & SYN_GEMM_EIGHT_WAVES) != 0;
     // the ring needs whole groups of four 32-deep slabs (and does not exist for 224-wide tiles)
     const bool ring = (d->options & SYN_GEMM_RING_PIPE) && d->K % 128 == 0 && d->block_n != 224;
@@ -1539,7 +1544,8 @@ int syn_gemm_producer_static(const syn_gemm_desc* desc, syn_stream_t stream) {
     const int rc = scratch_address(&counters);
     if (rc != 0) return rc;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    syn_gemm_desc d = *desc;
+    syn_gemm_desc d = {};
+    std::memcpy(&d, desc, (desc->options & SYN_GEMM_CUT_TILE) ? sizeof d : offsetof(syn_gemm_desc, cut_m));
     d.counters = counters;
     // the array keeps the last call's counts: the words this launch uses are zeroed in front of the kernel,
     // behind every check of the descriptor

@@ -544,6 +544,6 @@ int syn_where_async(uint32_t* out, int32_t workgroups, int32_t dwell, syn_stream
     return (int)hipGetLastError();
 }
 
-int syn_version(void) { return 100; }
+int syn_version(void) { return 200; }
 
 }  // extern "C"

@@ -127,3 +127,41 @@ def test_launch_entry_points_reject_null_descriptors_without_a_gpu(lib):
     assert lib.syn_delay_us(-1, None) == _lib.SYN_EINVAL
     desc = _lib.GemmDesc()
     assert lib.syn_gemm_consumer(ctypes.byref(desc), None) == _lib.SYN_EINVAL
+
+
+@pytest.mark.parametrize("behind", [0, 7, -1, 0x7F7F7F7F])
+def test_descriptors_that_end_in_front_of_the_optional_fields(lib, behind):
+    """What lies behind `options` (GEMM) and `work_list` (attention) in a caller's memory is none of the library's
+    business without the option bits: a descriptor of the older, shorter structure gets as far as the missing device."""
+    import torch
+    from syncopate_amd import _lib
+
+    if torch.cuda.is_available():
+        pytest.skip("the addresses are not a GPU's")
+    somewhere = (ctypes.c_char * 4096)()
+    address = ctypes.addressof(somewhere) + 15 & ~15
+
+    def cut_off(mirror, last, values):
+        """The fields up to `last`, and `behind` in every word after it."""
+        end = getattr(mirror, last).offset + getattr(mirror, last).size
+        desc = mirror(**values)
+        raw = (ctypes.c_char * (ctypes.sizeof(mirror) + 64))()
+        ctypes.memset(raw, 0, len(raw))
+        words = ctypes.cast(raw, ctypes.POINTER(ctypes.c_int32))
+        for i in range(end // 4, len(raw) // 4):
+            words[i] = behind
+        ctypes.memmove(raw, ctypes.byref(desc), end)
+        return ctypes.cast(raw, ctypes.POINTER(mirror)), raw
+
+    pointers = {n: address for n, t in _lib.GemmDesc._fields_ if t is ctypes.c_void_p and n != "visit_log"}
+    desc, keep = cut_off(_lib.GemmDesc, "options", dict(pointers, num_waves=1, M=256, N=256, K=128, dtype=0, block_m=128, block_n=128,
+                                                        block_k=64, group_m=8, num_sms=256))
+    no_device = lib.syn_delay_us(1, None)
+    assert no_device > 0
+    assert lib.syn_gemm_consumer(desc, None) == no_device
+    assert lib.syn_gemm_producer(desc, None) == no_device
+    pointers = {n: address for n in ("q", "k", "v", "o", "lse", "lock", "first", "flags", "wave_offsets", "wave_sizes",
+                                     "cum_wave_sizes", "signal_offsets")}
+    desc, keep = cut_off(_lib.AttnDesc, "work_list", dict(pointers, num_waves=1, Z=1, H=1, Sq=256, Skv=256, D=128, dtype=0, block_m=128,
+                                                          block_n=128, sm_scale=1.0, cum_tiles=256))
+    assert lib.syn_attn_fwd(desc, None) == no_device
