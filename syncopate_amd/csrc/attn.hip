@@ -952,17 +952,20 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
         if (tid == 0) report_status(p.status, SYN_STATUS_BAD_CHAIN, 0, (int)blockIdx.x, pairs_per_wave);
         return;
     }
-    const int program = logical_program_id((int)blockIdx.x, (int)gridDim.x, p.xcd_remap != 0);
+    const int program = kSplitChain ? (int)blockIdx.x
+                                    : logical_program_id((int)blockIdx.x, (int)gridDim.x, p.xcd_remap != 0);
 
     // where the program stands: the next pair of the table (kPairTiles, kPairChainWaves) or the entry of its list
     int pair = program;
     // The split forms: the program's part, how many the pair has, kv blocks of the part behind the visit being entered.  Chained
-    // waves: all pairs' first parts, then the second ones (an early chunk's programs come first); else a pair's parts
-    // side by side (pairs finish, and are counted, in the order of the table).
+    // waves: all pairs' first parts, then the second ones, each part's pairs dealt to the XCDs by themselves - an early
+    // chunk's programs come first, and the units of those that end while others still wait, which kernels that raise the
+    // flags may need, lie on all XCDs (a kernel's workgroups go to the XCDs in turn).  Else a pair's parts side by
+    // side.
     int part = 0, parts = 1, part_left = 0;
     if constexpr (kSplit) {
         part = kSplitChain ? program / num_pairs : program % p.split_parts;
-        pair = kSplitChain ? program % num_pairs : program / p.split_parts;
+        pair = kSplitChain ? logical_program_id(program % num_pairs, num_pairs, p.xcd_remap != 0) : program / p.split_parts;
     }
     int e = 0, e_end = 0, e_begin = 0;
     const int32_t* entries = nullptr;

@@ -203,3 +203,43 @@ def test_same_tables_with_another_number_of_waves(hip, form):
         # one rounding of the result and of the probabilities, three times that; see test_parts_add_up
         assert _rel(out[:, :, :rows], want[:, :, :rows]) <= 1.2e-2
         assert bool(out[:, :, rows:].isnan().all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,Sq,chunk,form,cut", [
+    (8, 1024, 1024, "explicit", True),           # 256 programs, of which 224 wait
+    (2, 512, 2048, "auto", True),
+])
+def test_flags_that_kernels_raise_while_parts_wait(hip, monkeypatch, H, Sq, chunk, form, cut):
+    """The chunks' flags go up one after the other, in another order than the waves', raised by kernels that are launched
+    behind the attention kernel: whatever form runs, its waiting programs leave room for them."""
+    from syncopate_amd import _lib
+    from syncopate_amd.communication.comm_runtime.streams import pick_side_streams
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.attn import attention_forward, template
+
+    chunks = 8
+    plans, planner = [], plan_kv_split
+    monkeypatch.setattr(template, "plan_kv_split", lambda *a, **kw: plans.append(planner(*a, **kw)) or plans[-1])
+    offsets, sizes, cums, signals, Skv = _chain_tables(1, H, Sq, [chunk] * chunks, [-1] + list(range(chunks - 1)))
+    q, k, v, _ = _inputs(1, H, Sq, Skv, torch.bfloat16)
+    table = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    tables = dict(wave_offsets=table(offsets), wave_sizes=table(sizes), cum_wave_sizes=table(cums), signal_offsets=table(signals),
+                  cum_tiles=cums[-1])
+    qd, kd, vd = q.cuda(), k.cuda(), v.cuda()
+    lib, side = _lib.load(), pick_side_streams(1)[0]
+    flags = torch.ones(chunks, dtype=torch.int64, device="cuda")
+    resident = attention_forward(qd, kd, vd, 128 ** -0.5, signal_ptr=flags, form=form, **tables)
+    assert len(plans) == 1 and (plans[0] is not None) == cut
+    for first in (0, 3):
+        flags.zero_()
+        torch.cuda.synchronize()
+        o = attention_forward(qd, kd, vd, 128 ** -0.5, signal_ptr=flags, form=form, **tables)
+        for i in range(chunks - 1):
+            _lib.check("syn_delay_us", lib.syn_delay_us(30, _lib.stream_handle(side)))
+            _lib.check("syn_flag_set", lib.syn_flag_set(flags.data_ptr() + 8 * ((first + 2 * i) % 7), 1, _lib.stream_handle(side)))
+        check_status()
+        if cut:                                  # (the other form merges in the order in which visits end)
+            assert torch.equal(o, resident)
+        # one rounding of the result and of the probabilities, three times that, and one of the result per merge
+        assert _rel(o[:, :2], numerics.sdpa_fp32(q[:, :2], k[:, :2], v[:, :2], 128 ** -0.5)) <= (1.2e-2 if cut else 2e-2)
