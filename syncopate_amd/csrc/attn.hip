@@ -861,6 +861,7 @@ __device__ __forceinline__ void add_partial(const unsigned char* slot, f32x4_t (
 //                    which is 136 KB through memory and three trips for the words that hand it over.
 constexpr int kPairTiles = 0, kPairChainWaves = 1, kPairWorkList = 2, kPairSplitChain = 3, kPairSplitVisit = 4;
 constexpr int32_t kWorkPairMask = SYN_ATTN_WORK_PAIR_MASK;
+constexpr int kUnits = 256;              // compute units of the chip, each of which runs one workgroup of this kernel
 constexpr int kPairLdsWaves = 256, kPairLdsEntries = 512;
 
 template <typename T, int MODE, bool CAUSAL>
@@ -953,6 +954,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
         return;
     }
     const int program = kSplitChain ? (int)blockIdx.x
+                        : kSplit    ? logical_program_id_by_rounds((int)blockIdx.x, (int)gridDim.x, kUnits, p.xcd_remap != 0)
                                     : logical_program_id((int)blockIdx.x, (int)gridDim.x, p.xcd_remap != 0);
 
     // where the program stands: the next pair of the table (kPairTiles, kPairChainWaves) or the entry of its list
@@ -961,7 +963,9 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
     // waves: all pairs' first parts, then the second ones, each part's pairs dealt to the XCDs by themselves - an early
     // chunk's programs come first, and the units of those that end while others still wait, which kernels that raise the
     // flags may need, lie on all XCDs (a kernel's workgroups go to the XCDs in turn).  Else a pair's parts side by
-    // side.
+    // side, dealt to the XCDs by rounds of kUnits: pairs finish, and are counted, in the order of the table, round by round
+    // (12 heads x 8192 rows x 32 kv blocks in eight chunks, 768 programs in 280 us: the first flags go up at 201, dealt over
+    // the whole grid every chunk was one XCD's and all eight went up at 300; one tile per program: 201 and 290).
     int part = 0, parts = 1, part_left = 0;
     if constexpr (kSplit) {
         part = kSplitChain ? program / num_pairs : program % p.split_parts;

@@ -74,6 +74,15 @@ __host__ __device__ __forceinline__ int logical_program_id(int hw_id, int grid, 
     return start + slot;
 }
 
+// The same for a grid of several rounds of `round` workgroups (a multiple of kNumXcd): the remap stays within a round, so
+// the first `round` workgroups to start are the first logical programs, the next ones the next.  Over the whole grid the
+// programs that should come first would all be one XCD's, and wait there for each other while the other XCDs take late ones.
+__host__ __device__ __forceinline__ int logical_program_id_by_rounds(int hw_id, int grid, int round, bool remap) {
+    const int first = hw_id / round * round;
+    const int count = grid - first < round ? grid - first : round;
+    return first + logical_program_id(hw_id - first, count, remap);
+}
+
 // 16 bytes stored through the XCD's L2 to memory (the agent-scope form of a store: what a relaxed
 // atomic store at that scope compiles to, which exists for 8 bytes at most).  A vector store.
 // A store of more than 8 bytes reads its data registers for two more issue slots; the compiler

@@ -243,3 +243,47 @@ def test_flags_that_kernels_raise_while_parts_wait(hip, monkeypatch, H, Sq, chun
             assert torch.equal(o, resident)
         # one rounding of the result and of the probabilities, three times that, and one of the result per merge
         assert _rel(o[:, :2], numerics.sdpa_fp32(q[:, :2], k[:, :2], v[:, :2], 128 ** -0.5)) <= (1.2e-2 if cut else 2e-2)
+
+
+@pytest.mark.gpu
+def test_producer_of_several_rounds_announces_its_waves_in_order(hip):
+    """More programs than compute units: the flags of the table's first waves go up rounds before the last one's."""
+    import time
+
+    from syncopate_amd.communication.comm_runtime.streams import pick_side_streams
+    from syncopate_amd.computation._launch import check_status, compute_units
+    from syncopate_amd.computation.attn import attention_forward
+
+    H, Sq, Skv, chunks = 12, 8192, 8192, 8
+    rows = Sq // chunks
+    offsets, sizes = [[0, 0, i * rows, 0] for i in range(chunks)], [[1, H, rows, Skv]] * chunks
+    cums = [(i + 1) * H * rows for i in range(chunks)]
+    plan = plan_kv_split(offsets, sizes, cums, list(range(chunks)), causal=False, producer=True, units=256, always=True)
+    assert plan.programs > 2 * 256 >= 2 * compute_units(0)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q, k, v = (torch.randn(1, H, s, 128, device="cuda", generator=g).bfloat16() for s in (Sq, Skv, Skv))
+    table = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    tables = dict(wave_offsets=table(offsets), wave_sizes=table(sizes), cum_wave_sizes=table(cums),
+                  signal_offsets=table(list(range(chunks))), cum_tiles=cums[-1])
+    flags = torch.zeros(chunks, dtype=torch.int64, device="cuda")
+    counters = torch.zeros(chunks, dtype=torch.int32, device="cuda")
+    side, seen = pick_side_streams(1)[0], torch.zeros(chunks, dtype=torch.int64).pin_memory()
+    shares = []
+    for _ in range(5):
+        flags.zero_()
+        counters.zero_()
+        torch.cuda.synchronize()
+        start, when = time.perf_counter(), {}
+        attention_forward(q, k, v, 128 ** -0.5, signal_ptr=flags, counter_ptr=counters, **tables)
+        while len(when) < chunks and time.perf_counter() - start < 10:
+            with torch.cuda.stream(side):
+                seen.copy_(flags, non_blocking=True)
+            side.synchronize()
+            for i in range(chunks):
+                if int(seen[i]):
+                    when.setdefault(i, time.perf_counter() - start)
+        check_status()
+        assert counters.tolist() == [H * rows // BLOCK] * chunks
+        shares.append(when[0] / when[chunks - 1])
+    # 48 of 384 pairs of the first wave end with the first of three rounds; all at the end if a wave is one XCD's
+    assert sorted(shares)[2] < 0.7, shares
