@@ -72,10 +72,11 @@ def plan_kv_split(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Se
     lengths = [s[3] // BLOCK for _, s in waves]
     total = sum(lengths)
     gated = [int(signal_offsets[w]) >= 0 for w in range(len(waves))]
-    # Programs that wait hold their compute unit.  Where the uncut form leaves units free while it waits, the copies that
-    # raise the flags may need them: the cut one then leaves some free, too.
-    waiting_tiles = sum(2 * pairs for g in gated if g)
-    room = any(gated) and (waiting_tiles < 2 * units if always else pairs < units)
+    # Programs that wait hold their compute unit with all its registers (eight wavefronts of 256), so that nothing else runs
+    # there, a copy kernel that raises the flags among them.  Uncut pairs in fewer programs than units leave some free, and
+    # the kernel with one tile per program room beside it however many tiles wait (two wavefronts of 232 registers per SIMD
+    # of 512): what takes the place of either does not fill the chip with programs that wait.
+    room = any(gated) and (always or pairs < units)
 
     def waiting_parts(parts: int) -> int:
         count, first = 0, 0
@@ -88,8 +89,9 @@ def plan_kv_split(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Se
     best, best_us, whole_us = None, None, None
     for parts in range(1, min(MAX_PARTS, total) + 1):
         programs = pairs * parts
-        if parts > 1 and (pairs * (parts - 1) > MAX_SLOTS or
-                          (room and (programs > units or pairs * waiting_parts(parts) > units - RESERVED_UNITS))):
+        if pairs * (parts - 1) > MAX_SLOTS:
+            continue
+        if room and (always or parts > 1) and (programs > units or pairs * waiting_parts(parts) > units - RESERVED_UNITS):
             continue
         us = -(-programs // units) * (-(-total // parts) * BLOCK_US + SEGMENT_US + STEP_US * _steps(parts))
         whole_us = whole_us or us
@@ -99,7 +101,7 @@ def plan_kv_split(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Se
         tiles = 2 * pairs * len(waves)
         # visits to a q block that end at the same time are merged one after the other
         merges = min(len(waves), units // pairs) - 1 if tiles <= 2 * units else 0
-        if best_us >= _tiles_us(tiles, -(-total // len(waves)), units) + MERGE_US * merges:
+        if best is None or best_us >= _tiles_us(tiles, -(-total // len(waves)), units) + MERGE_US * merges:
             return None
         if best == 1 and 8 * pairs < 7 * units:         # whole pairs that leave units idle: 135 of 28 blocks 102 us, as tiles 89
             return None

@@ -35,9 +35,18 @@ def test_plans():
     free_first = plan(1, 8, 1024, [1024] * 8, [-1] + list(range(7)), always=True)
     assert free_first.programs <= 256 and free_first.pairs == 32
     assert free_first.programs - free_first.pairs <= 224
-    # enough pairs: stay whole where they would be chained, one part where they would be single tiles
+    # enough pairs: stay whole where they would be chained, one part where they would be single tiles - but not where
+    # they wait, on every compute unit and with all its registers, for flags that a kernel may have to raise
     assert plan(1, 32, 4096, [4096] * 8, [-1] + list(range(7))) is None
-    assert plan(1, 32, 4096, [4096] * 8, [-1] + list(range(7)), always=True).parts == 1
+    assert plan(1, 32, 4096, [4096] * 8, [-1] * 8, always=True).parts == 1
+    assert plan(1, 32, 4096, [4096] * 8, [-1] + list(range(7)), always=True) is None
+    for heads in range(1, 66):
+        for signals in ([-1] + list(range(7)), [-1] * 7 + [0], list(range(8))):
+            for sq in (256, 1024, 3072):
+                got = plan(1, heads, sq, [1024] * 8, signals, always=True)
+                assert got is None or (got.programs <= 256 and got.pairs * sum(
+                    any(s >= 0 and 8 * w < 64 * (p + 1) // got.parts and 8 * (w + 1) > 64 * p // got.parts
+                        for w, s in enumerate(signals)) for p in range(got.parts)) <= 224)
     # too little to gain: ten pairs of 14 blocks as 40 tiles, 64 pairs of 40 as 1024
     assert plan(1, 5, 512, [896] * 2, [-1, 0], always=True) is None
     assert plan(1, 8, 2048, [640] * 8, [-1] + list(range(7)), always=True) is None
@@ -209,6 +218,8 @@ def test_same_tables_with_another_number_of_waves(hip, form):
 @pytest.mark.parametrize("H,Sq,chunk,form,cut", [
     (8, 1024, 1024, "explicit", True),           # 256 programs, of which 224 wait
     (2, 512, 2048, "auto", True),
+    (20, 1024, 1024, "explicit", False),         # more tiles than run at a time, all but the first wave's waiting
+    (24, 3072, 512, "explicit", False),
 ])
 def test_flags_that_kernels_raise_while_parts_wait(hip, monkeypatch, H, Sq, chunk, form, cut):
     """The chunks' flags go up one after the other, in another order than the waves', raised by kernels that are launched
