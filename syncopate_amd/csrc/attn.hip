@@ -1119,6 +1119,12 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
             if constexpr (kSplitChain) {
                 while (begin >= s_row[w][6]) begin -= s_row[w++][6];
                 w = __builtin_amdgcn_readfirstlane(w);
+                // (a part that begins in a later wave reads that wave's kv range for wave 0's q blocks: they have to be the same)
+                if (__builtin_amdgcn_ballot_w64(s_cum[w] != 2 * (w + 1) * pairs_per_wave ||
+                                                (lane < 5 && s_row[w][lane] != s_row[0][lane])) != 0) {
+                    if (tid == 0) report_status(p.status, SYN_STATUS_BAD_CHAIN, w, (int)blockIdx.x, tile_id);
+                    return;
+                }
                 kv_lo = __builtin_amdgcn_readfirstlane(s_row[w][5]);
                 kv_len = __builtin_amdgcn_readfirstlane(s_row[w][6]);
                 sig = __builtin_amdgcn_readfirstlane(s_row[w][7]);

@@ -298,3 +298,21 @@ def test_producer_of_several_rounds_announces_its_waves_in_order(hip):
         shares.append(when[0] / when[chunks - 1])
     # 48 of 384 pairs of the first wave end with the first of three rounds; all at the end if a wave is one XCD's
     assert sorted(shares)[2] < 0.7, shares
+
+
+@pytest.mark.gpu
+def test_part_that_begins_in_a_wave_of_other_rows(hip, monkeypatch):
+    """The kernel compares the wave in which a part begins with the first one, whose q blocks it takes, and says so."""
+    from syncopate_amd import _lib
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.attn import attention_forward, template
+
+    q, k, v, _ = _inputs(1, 1, 512, 512, torch.bfloat16)
+    monkeypatch.setattr(template, "plan_kv_split", lambda *args, **kwargs: KvSplit(True, 1, 2, 2))
+    monkeypatch.setattr(template, "already_checked", lambda *args: True)
+    table = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    attention_forward(q.cuda(), k.cuda(), v.cuda(), 0.1, wave_offsets=table([[0, 0, 0, 0], [0, 0, 256, 256]]),
+                      wave_sizes=table([[1, 1, 256, 256]] * 2), cum_wave_sizes=table([256, 512]), signal_offsets=table([-1, -1]),
+                      signal_ptr=torch.ones(1, dtype=torch.int64, device="cuda"), cum_tiles=512)
+    with pytest.raises(RuntimeError, match=rf"kernel status \[{_lib.SYN_STATUS_BAD_CHAIN}, 1, "):
+        check_status()
