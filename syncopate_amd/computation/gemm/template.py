@@ -162,8 +162,9 @@ def _launch(
         elif waiting is None:
             waiting = recall_note(tables, "waiting share")
             waiting = 1.0 if waiting is None else waiting
+        units = compute_units(dev.index)
         bm, bn = choose_kernel_tile(num_tiles, num_gemm_sms, K, BLOCK_SIZE_M, BLOCK_SIZE_N, waiting=waiting,
-                                    room=compute_units(dev.index) - RESERVED_UNITS)
+                                    room=units - RESERVED_UNITS, units=units)
         cut = ((BLOCK_SIZE_M // bm).bit_length() - 1, (BLOCK_SIZE_N // bn).bit_length() - 1)
         GROUP_SIZE_M *= BLOCK_SIZE_M // bm
         BLOCK_SIZE_M, BLOCK_SIZE_N = bm, bn

@@ -216,8 +216,9 @@ def gemm_remote(
     cut = (0, 0)
     if visit_log is None and not eight_waves and BLOCK_SIZE_M > 0 and BLOCK_SIZE_N > 0:
         # few tiles: a smaller kernel tile (the tables, offsets and destinations are in elements)
+        units = compute_units(dev.index)
         bm, bn = choose_kernel_tile((int(cum_tiles) or M * N) // (BLOCK_SIZE_M * BLOCK_SIZE_N), num_gemm_sms, K, BLOCK_SIZE_M,
-                                    BLOCK_SIZE_N, waiting=float(signal_offsets is not None), room=compute_units(dev.index) - RESERVED_UNITS)
+                                    BLOCK_SIZE_N, waiting=float(signal_offsets is not None), room=units - RESERVED_UNITS, units=units)
         cut = ((BLOCK_SIZE_M // bm).bit_length() - 1, (BLOCK_SIZE_N // bn).bit_length() - 1)
         GROUP_SIZE_M *= BLOCK_SIZE_M // bm
         BLOCK_SIZE_M, BLOCK_SIZE_N = bm, bn

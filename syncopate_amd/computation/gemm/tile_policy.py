@@ -73,11 +73,13 @@ TILE_US = 3.0
 
 
 def choose_kernel_tile(tiles: int, programs: int, k: int, bm: int, bn: int, *, waiting: float = 0.0,
-                       room: Optional[int] = None) -> Tuple[int, int]:
+                       room: Optional[int] = None, units: Optional[int] = None) -> Tuple[int, int]:
     """The tile a launch of `tiles` tiles of (bm, bn) runs on: itself, or one that divides it where the tiles do not
     fill the programs.  42 tiles of 256x256 keep 42 programs busy for 1.27 us a slab; as 168 tiles of 128x128 they keep 168
     busy for 0.53.  Only launches of one round are cut, and into one round: every wave's last tile then ends earlier
-    too, so that a consumer whose chunks arrive slowly gains as well as one whose chunks are there.
+    too, so that a consumer whose chunks arrive slowly gains as well as one whose chunks are there.  A round is as many
+    programs as the device has compute units (`units`), however many the caller allows: 200 tiles of 256x256 on 1024
+    programs would be four rounds of 128x128 where they are one.
 
     `waiting`: the share of the tiles that wait for a flag; a launch that cuts them keeps at most `room` programs
     waiting, the others stay with the copies that raise the flags."""
@@ -91,6 +93,6 @@ def choose_kernel_tile(tiles: int, programs: int, k: int, bm: int, bn: int, *, w
         if bm % shape[0] or bn % shape[1]:
             return False
         cut = tiles * (bm // shape[0]) * (bn // shape[1])
-        return cut <= programs and (room is None or cut * waiting <= room)
+        return cut <= programs and (units is None or cut <= units) and (room is None or cut * waiting <= room)
 
     return min([(bm, bn)] + [shape for shape in SLAB_US if fits(shape)], key=cost)

@@ -15,6 +15,8 @@ def test_rule():
     assert choose_kernel_tile(128, 256, 512, 128, 256, waiting=0.75, room=224) == (128, 128)
     assert choose_kernel_tile(16, 256, 512, 256, 224) == (256, 224)         # no tile divides it
     assert choose_kernel_tile(16, 0, 512, 256, 256) == (256, 256)           # the library names the error
+    assert choose_kernel_tile(200, 1024, 2048, 256, 256, units=256) == (256, 256)     # more programs than run at a time
+    assert choose_kernel_tile(60, 1024, 2048, 256, 256, units=256) == (128, 128)
     for tiles in range(1, 257, 5):
         for shape in SLAB_US:
             bm, bn = choose_kernel_tile(tiles, 224, 1024, *shape, waiting=0.5, room=192)
