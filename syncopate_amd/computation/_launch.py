@@ -7,7 +7,7 @@ import ctypes
 import functools
 import inspect
 import weakref
-from typing import Dict, Optional, Sequence, Tuple, Union
+from typing import Dict, List, Optional, Sequence, Tuple, Union
 
 import torch
 
@@ -134,6 +134,12 @@ def as_device_table(table: TableLike, device: torch.device, width: Optional[int]
 
 def host_copy(t: torch.Tensor) -> torch.Tensor:
     return t.detach().to("cpu", copy=True).contiguous()
+
+
+def host_copies(tables: Sequence[torch.Tensor]) -> List[torch.Tensor]:
+    """CPU copies of int32 device tables, read back together: one wait for the stream instead of one per table."""
+    flat = torch.cat([t.detach().reshape(-1) for t in tables]).cpu()
+    return [part.view(t.shape) for t, part in zip(tables, flat.split([t.numel() for t in tables]))]
 
 
 # Tables that passed the host-side check are remembered per tensor OBJECT (weak

@@ -152,8 +152,8 @@ def test_part_of_minus_infinity(hip, monkeypatch):
 
 @pytest.mark.gpu
 def test_template_tables_are_kept_and_follow_their_source(hip):
-    """The hand-written template's call keeps its converted tables with the caller's: again on another stream, and after
-    the caller has changed its tables in place, in which case they are converted anew."""
+    """The hand-written template's call keeps its converted tables: again on another stream, and after the caller has
+    changed its tables in place, by whatever means; tables on the host, and a call that keeps no versions."""
     from syncopate_amd.computation._launch import check_status
     from syncopate_amd.computation.attn import attention, build_waves_and_signals_divisible
 
@@ -168,11 +168,40 @@ def test_template_tables_are_kept_and_follow_their_source(hip):
         torch.cuda.synchronize()
         check_status()
         assert _rel(o, want) <= 1.2e-2
-    waves["wave_offsets"].view(4, 4)[:, 3] = torch.tensor([0, 2, 4, 0], dtype=torch.int32)       # the last wave: the first again
-    o = attention(qd, kd, vd, 0.1, waves)
-    check_status()
+    other = torch.tensor([0, 2, 4, 0], dtype=torch.int32, device="cuda")          # the last wave: the first again
     twice = torch.cat([k[:, :, :768], k[:, :, :256]], dim=2), torch.cat([v[:, :, :768], v[:, :, :256]], dim=2)
+    for blocks, kv in ((other, twice), (torch.tensor([0, 2, 4, 6], dtype=torch.int32, device="cuda"), (k, v)), (other, twice)):
+        if blocks is other:
+            waves["wave_offsets"].data.view(4, 4)[:, 3] = blocks        # a write that the tensor's version does not count
+        else:
+            waves["wave_offsets"].view(4, 4)[:, 3] = blocks
+        o = attention(qd, kd, vd, 0.1, waves)
+        check_status()
+        assert _rel(o, numerics.sdpa_fp32(q, *kv, 0.1)) <= 1.2e-2
+    on_host = {n: t.tolist() if n in ("wave_offsets", "wave_sizes", "cum_wave_sizes", "signal_offsets") else t for n, t in waves.items()}
+    on_host["wave_offsets"] = [on_host["wave_offsets"][i:i + 4] for i in range(0, 16, 4)]
+    with torch.inference_mode():
+        o = attention(qd, kd, vd, 0.1, on_host)
+    check_status()
     assert _rel(o, numerics.sdpa_fp32(q, *twice, 0.1)) <= 1.2e-2
+
+
+@pytest.mark.gpu
+def test_template_call_is_not_captured(hip):
+    """Its tables are read on every call, so that a captured launch would go on with what they held (and where they lay)."""
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.attn import attention, build_waves_and_signals_divisible
+
+    q, k, v, _ = _inputs(1, 2, 512, 1024, torch.bfloat16)
+    qd, kd, vd = q.cuda(), k.cuda(), v.cuda()
+    waves = build_waves_and_signals_divisible(1, 2, 512, 1024, w=4)
+    attention(qd, kd, vd, 0.1, waves)
+    check_status()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        with pytest.raises(RuntimeError, match="cannot be captured"):
+            attention(qd, kd, vd, 0.1, waves)
+        qd.add_(0)                                  # (an empty graph is warned about)
 
 
 @pytest.mark.gpu
