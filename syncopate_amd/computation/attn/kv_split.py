@@ -50,40 +50,48 @@ def plan_kv_split(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Se
 
     `always`: the launch would otherwise take the kernel with one tile per program (uncut pairs may beat that too); else
     it would chain the uncut pairs, and None means that they stay whole."""
-    waves = []
-    for w, cum in enumerate(cum_wave_sizes):
-        if int(cum) == 0:
+    if len(cum_wave_sizes) > MAX_WAVES or (causal and not producer):
+        return None
+    waves, align = [], 2 * BLOCK if causal else BLOCK
+    for cum, off, size in zip(cum_wave_sizes, wave_offsets, wave_sizes):
+        if cum == 0:
             break
-        off, size = [int(x) for x in wave_offsets[w]], [int(x) for x in wave_sizes[w]]
-        if min(size) <= 0 or min(off) < 0 or size[2] % (2 * BLOCK) or size[3] % BLOCK or off[2] % BLOCK or off[3] % BLOCK:
+        if not producer and waves and (off[:3] != waves[0][0][:3] or size[:3] != waves[0][1][:3]):
             return None
-        if causal and (off[2] % (2 * BLOCK) or off[3] % (2 * BLOCK)):
+        if min(size) <= 0 or min(off) < 0 or size[2] % (2 * BLOCK) or size[3] % BLOCK or off[2] % align or off[3] % align:
             return None
         waves.append((off, size))
-    if not waves or len(cum_wave_sizes) > MAX_WAVES:
+    if not waves:
         return None
     if producer:
         return _split_visits(waves, causal, units)
-    if causal or any(off[:3] != waves[0][0][:3] or size[:3] != waves[0][1][:3] for off, size in waves):
-        return None
 
     size = waves[0][1]
     pairs = size[0] * size[1] * size[2] // (2 * BLOCK)
     lengths = [s[3] // BLOCK for _, s in waves]
     total = sum(lengths)
-    gated = [int(signal_offsets[w]) >= 0 for w in range(len(waves))]
+    gated = [signal >= 0 for _, signal in zip(waves, signal_offsets)]
     # Programs that wait hold their compute unit with all its registers (eight wavefronts of 256), so that nothing else runs
     # there, a copy kernel that raises the flags among them.  Uncut pairs in fewer programs than units leave some free, and
     # the kernel with one tile per program room beside it however many tiles wait (two wavefronts of 232 registers per SIMD
     # of 512): what takes the place of either does not fill the chip with programs that wait.
     room = any(gated) and (always or pairs < units)
 
+    # runs of blocks behind flags
+    runs, start = [], 0
+    for waits, length in zip(gated, lengths):
+        if waits and runs and runs[-1][1] == start:
+            runs[-1][1] = start + length
+        elif waits:
+            runs.append([start, start + length])
+        start += length
+
     def waiting_parts(parts: int) -> int:
-        count, first = 0, 0
-        edges = [total * p // parts for p in range(parts + 1)]
-        starts = [sum(lengths[:w]) for w in range(len(lengths))]
-        for lo, hi in zip(edges, edges[1:]):
-            count += any(g and s < hi and s + n > lo for g, s, n in zip(gated, starts, lengths))
+        count, counted = 0, 0                    # part p has the blocks from total * p // parts on
+        for lo, hi in runs:
+            first, last = ((lo + 1) * parts - 1) // total, (hi * parts - 1) // total
+            count += max(last + 1 - max(first, counted), 0)
+            counted = max(counted, last + 1)
         return count
 
     best, best_us, whole_us = None, None, None
@@ -113,9 +121,14 @@ def plan_kv_split(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Se
 def _split_visits(waves, causal: bool, units: int) -> Optional[KvSplit]:
     if len(waves) > 64:
         return None
-    for i, (a, sa) in enumerate(waves):         # every pair of q blocks in one wave only
-        for b, sb in waves[:i]:
-            if all(a[x] < b[x] + sb[x] and b[x] < a[x] + sa[x] for x in range(3)):
+    by_rows = sorted((off[2], off[2] + size[2], i) for i, (off, size) in enumerate(waves))
+    for at, (_, end, i) in enumerate(by_rows):  # every pair of q blocks in one wave only
+        (za, ha, *_), (nza, nha, *_) = waves[i]
+        for start, _, j in by_rows[at + 1:]:
+            if start >= end:
+                break
+            (zb, hb, *_), (nzb, nhb, *_) = waves[j]
+            if za < zb + nzb and zb < za + nza and ha < hb + nhb and hb < ha + nha:
                 return None
     walks: Dict[int, int] = {}                  # pairs that walk so many kv blocks
     for off, size in waves:

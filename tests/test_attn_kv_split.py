@@ -345,3 +345,35 @@ def test_part_that_begins_in_a_wave_of_other_rows(hip, monkeypatch):
                       signal_ptr=torch.ones(1, dtype=torch.int64, device="cuda"), cum_tiles=512)
     with pytest.raises(RuntimeError, match=rf"kernel status \[{_lib.SYN_STATUS_BAD_CHAIN}, 1, "):
         check_status()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["split", "auto split", "auto chain", "auto list", "causal auto", "producer"])
+def test_new_tables_are_read_back_once(hip, monkeypatch, kind):
+    """Tables that the launcher has not seen cost one read-back, whatever it works out from them; tables it has seen and
+    tables on the host cost none."""
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.attn import attention_forward, template
+
+    rows = 512 if kind in ("auto list", "producer") else 256
+    offsets = [[0, 0, i * 256 if rows == 512 else 0, 256 * i] for i in range(2)]
+    sizes, cums, signals = [[1, 2, 256, 256]] * 2, [512, 1024], [0, 1]
+    causal = kind == "causal auto"
+    q, k, v, _ = _inputs(1, 2, 512 if causal else rows, 512, torch.bfloat16)
+    q, k, v = q.cuda(), k.cuda(), v.cuda()
+    read, copies = [], template.host_copies
+    monkeypatch.setattr(template, "host_copies", lambda tables: read.append(len(tables)) or copies(tables))
+    monkeypatch.setattr(template, "host_copy", lambda table: pytest.fail("read back by itself"))
+    table = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    kw = dict(form="auto" if "auto" in kind else "explicit", causal=causal, signal_ptr=torch.ones(2, dtype=torch.int64, device="cuda"))
+    if "split" in kind:
+        monkeypatch.setattr(template, "plan_kv_split", lambda *args, **kwargs: KvSplit(True, 2, 2, 2))
+    for given, count in ((table, 1), (lambda x: x, 0)):
+        tables = dict(wave_offsets=given(offsets), wave_sizes=given(sizes), cum_wave_sizes=given(cums), signal_offsets=given(signals))
+        read.clear()
+        for _ in range(2):
+            if kind == "producer":
+                kw["counter_ptr"] = torch.zeros(2, dtype=torch.int32, device="cuda")
+            attention_forward(q, k, v, 0.1, cum_tiles=1024, **kw, **tables)
+        assert read == [4] * count
+    check_status()
