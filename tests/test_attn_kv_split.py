@@ -50,6 +50,11 @@ def test_plans():
     # too little to gain: ten pairs of 14 blocks as 40 tiles, 64 pairs of 40 as 1024
     assert plan(1, 5, 512, [896] * 2, [-1, 0], always=True) is None
     assert plan(1, 8, 2048, [640] * 8, [-1] + list(range(7)), always=True) is None
+    # tiles that need little more than a round, and whole pairs that gain as little (560 of 22 blocks: 259 us, as tiles 225)
+    assert plan(1, 70, 2048, [1408] * 2, [-1, -1], always=True) is None
+    assert plan(1, 40, 512, [4352] * 4, [-1, 0, 1, 2], always=True) is None
+    visits = ([[0, 0, i * 1024, 0] for i in range(2)], [[1, 38, 1024, 2816]] * 2, [38 * 1024 * (i + 1) for i in range(2)], [0, 1])
+    assert plan_kv_split(*visits, causal=False, producer=True, units=256, always=True) is None
     # odd q blocks, unequal q ranges, a causal consumer, a q block visited twice by a producer: not cut
     assert plan(1, 2, 384, [512] * 2, [-1, 0]) is None
     assert plan(1, 2, 512, [512] * 2, [-1, 0], causal=True) is None
