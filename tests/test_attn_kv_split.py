@@ -382,3 +382,60 @@ def test_new_tables_are_read_back_once(hip, monkeypatch, kind):
             attention_forward(q, k, v, 0.1, cum_tiles=1024, **kw, **tables)
         assert read == [4] * count
     check_status()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("producer", [False, True])
+def test_captured_split(hip, producer):
+    """A planned split under graph capture: every replay starts from zeroed words of its own, with eager launches of the
+    same tables between the replays."""
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.attn import attention_forward
+
+    H, chunks, scale = 8, 8, 128 ** -0.5
+    Sq, Skv = (2048, 4096) if producer else (1024, 8192)
+    rows = Sq // chunks
+    if producer:
+        offsets, sizes = [[0, 0, i * rows, 0] for i in range(chunks)], [[1, H, rows, Skv]] * chunks
+        cums = [(i + 1) * H * rows for i in range(chunks)]
+    else:
+        offsets, sizes, cums, _, _ = _chain_tables(1, H, Sq, [Skv // chunks] * chunks, None)
+    signals = list(range(chunks))
+    plan = plan_kv_split(offsets, sizes, cums, signals, causal=False, producer=producer, units=256, always=True)
+    assert plan.parts > 1 and plan.chain != producer
+    table = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    tables = dict(wave_offsets=table(offsets), wave_sizes=table(sizes), cum_wave_sizes=table(cums), signal_offsets=table(signals),
+                  cum_tiles=cums[-1])
+    flags = torch.full((chunks,), 0 if producer else 1, dtype=torch.int64, device="cuda")
+    counters = torch.zeros(chunks, dtype=torch.int32, device="cuda") if producer else None
+    q, k, v = (t.cuda() for t in _inputs(1, H, Sq, Skv, torch.bfloat16)[:3])
+    out = torch.zeros_like(q)
+
+    def launch(into):
+        if producer:
+            flags.zero_()
+            counters.zero_()
+        return attention_forward(q, k, v, scale, signal_ptr=flags, counter_ptr=counters, out=into, **tables)
+
+    launch(out)                                          # warm-up: tables planned and checked
+    check_status()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph):
+            launch(out)
+    torch.cuda.current_stream().wait_stream(side)
+    for replay in range(4):
+        nq, nk, nv, _ = _inputs(1, H, Sq, Skv, torch.bfloat16, seed=40 + replay)
+        q.copy_(nq.cuda()); k.copy_(nk.cuda()); v.copy_(nv.cuda())
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        for _ in range(2):                               # again at once: behind the first one's words
+            graph.replay()
+        torch.cuda.synchronize()
+        check_status()
+        assert flags.tolist() == [1] * chunks
+        assert _rel(out, numerics.sdpa_fp32(nq, nk, nv, scale)) <= 1.2e-2, f"replay {replay}"
+        assert torch.equal(out, launch(torch.empty_like(q))), f"replay {replay}"
+        check_status()

@@ -146,6 +146,13 @@ def test_allgather_attention_4096x32768_double_ring_order(hip):
     for h in (5, 22):
         s = (q[0, h].float() @ k[0, h].float().t()) * scale
         assert _rel(o2[0, h], torch.softmax(s, dim=-1) @ v[0, h].float()) <= REL_TOL
+    # a workgroup per tile, every tile's visit merged in memory
+    o3 = attention_forward(q, k, v, scale, signal_ptr=flags, num_programs=ring["cum_tiles"] // 128, **ring)
+    check_status()
+    assert _rel(o3, o) <= 2 * REL_TOL
+    for h in (0, 31):
+        s = (q[0, h].float() @ k[0, h].float().t()) * scale
+        assert _rel(o3[0, h], torch.softmax(s, dim=-1) @ v[0, h].float()) <= REL_TOL
 
 
 def test_all2all_attention_16384_causal(hip):

@@ -76,3 +76,43 @@ def test_few_tiles(hip, form, world, rows, n, k, bm, bn, programs, dtype):
     ref = a.double() @ b.double().t()
     # one rounding of the result (2^-9, 2^-12 of a value, at most that of the largest); the sums are 32-bit
     assert ((c.double() - ref).abs().max() / ref.abs().max()).item() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("world,rows,n,k,bm,bn", [(4, 512, 768, 320, 256, 256), (2, 384, 1280, 1984, 128, 256), (3, 256, 640, 2112, 256, 128)])
+@pytest.mark.parametrize("form", ["producer", "direct", "gathered", "split k"])
+def test_same_bits_as_on_the_whole_tiles(hip, monkeypatch, form, world, rows, n, k, bm, bn):
+    """The cut changes no bit of any form's result: the K phase is that of the caller's tile (each sum of an adding form
+    goes to a zero; split K adds twice, and the sum of two does not depend on their order)."""
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.gemm import (gemm_ag_direct_read, gemm_producer, gemm_rs_producer_persistent, gemm_splitk, template,
+                                                template_remote)
+
+    g = torch.Generator(device="cuda").manual_seed(k + n)
+    m = world * rows
+    a = (0.05 * torch.randn(m, k, device="cuda", generator=g)).bfloat16()
+    b = (0.05 * torch.randn(n, k, device="cuda", generator=g)).bfloat16()
+    order = [(i + 1) % world for i in range(world)]
+    sizes, offsets, ranks = _table([[rows, n]] * world), _table([[i * rows, 0] for i in order]), _table(order)
+    rule, taken, results = choose_kernel_tile, [], []
+    for cut in (True, False):
+        choose = lambda *args, **kw: taken.append((args[3:5], rule(*args, **kw) if cut else args[3:5])) or taken[-1][1]
+        monkeypatch.setattr(template, "choose_kernel_tile", choose)
+        monkeypatch.setattr(template_remote, "choose_kernel_tile", choose)
+        c = torch.zeros(world, rows, n, dtype=torch.bfloat16, device="cuda")
+        if form == "producer":
+            flags = torch.zeros(world, dtype=torch.int64, device="cuda")
+            gemm_producer(a, b, c.view(m, n), flags, sizes, offsets, ranks, 256, bm, bn, 64, 8, cum_tiles=m * n)
+            assert flags.tolist() == [1] * world
+        elif form == "direct":
+            gemm_rs_producer_persistent(a, b, list(c), sizes, offsets, ranks, world, world, 256, bm, bn, 64, 8)
+        elif form == "gathered":
+            gemm_ag_direct_read(list(a.view(world, rows, k)), b, c.view(m, n), sizes, offsets, ranks, world, world, 256, True, bm, bn, 64, 8)
+        else:
+            half = k // 128 * 64
+            gemm_splitk(a, b, c.view(m, n), world, 256, bm, bn, 64, 8, cur_wave_sizes=_table([[m, n, half], [m, n, k - half]]),
+                        wave_offsets=_table([[0, 0, 0], [0, 0, half]]), cum_tiles=2 * m * n)
+        check_status()
+        results.append(c)
+    assert taken[0][0] != taken[0][1] and len(taken) == 2
+    assert torch.equal(*results)
