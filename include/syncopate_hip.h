@@ -368,7 +368,11 @@ typedef struct syn_attn_desc {
  * (under its conditions) the kv blocks are those of all waves in a row and every program waits for the flags of its
  * own part; else every pair of q blocks has to be visited once in the whole table (the caller vouches), and with
  * `counters` the launch is a producer: no flag is waited for, every finished pair counts two tiles.
- * num_programs = pairs * split_parts.  No counterpart in the reference. */
+ * num_programs = pairs * split_parts.  Workgroup b works on part b / pairs where the waves are chained (with
+ * SYN_ATTN_XCD_REMAP the pairs of each part are dealt to the XCDs by themselves), else on part b % split_parts of pair
+ * b / split_parts (dealt to the XCDs within rounds of 256 workgroups), so the first workgroups take the first chunks, or
+ * the table's first pairs.  A workgroup takes all registers of its compute unit: where kernels on the same device
+ * raise the flags, leave units without one that waits.  No counterpart in the reference. */
 #define SYN_ATTN_SPLIT_KV 32u
 #define SYN_ATTN_SPLIT_MAX_PARTS 16
 #define SYN_ATTN_SPLIT_SLOT_BYTES 139264
