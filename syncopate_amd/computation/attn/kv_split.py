@@ -26,6 +26,10 @@ BLOCK_US, SEGMENT_US, STEP_US = 3.6, 14.0, 8.0
 MERGE_US = 5.0
 MIN_GAIN_US = 10.0        # (the words and slots of the parts cost the host 3 us a launch, which small ones wait for)
 RESERVED_UNITS = 32       # compute units that waiting programs leave to the copies which raise their flags
+# Units that a producer does not count on: kernels that wait for its flags, one workgroup per side stream of an exchange, each
+# keep a unit from a workgroup that wants all registers, and a program too many for its XCD costs a round.  128 pairs
+# of 32 blocks as 256 programs: 85 us alone, 133 beside one such kernel; as single tiles, which share units with it, 96 and 95.
+EXCHANGE_UNITS = 16
 
 
 class KvSplit(NamedTuple):
@@ -143,6 +147,7 @@ def _split_visits(waves, causal: bool, units: int) -> Optional[KvSplit]:
             walks[walked] = walks.get(walked, 0) + size[0] * size[1]
     longest, pairs = max(walks), sum(walks.values())
     best, best_us = None, None
+    tile_units, units = units, units - EXCHANGE_UNITS
     for parts in range(1, min(MAX_PARTS, max(longest, 1)) + 1):
         if pairs * (parts - 1) > MAX_SLOTS or (len(walks) > 1 and parts > 1 and pairs * parts > units):
             break
@@ -161,7 +166,7 @@ def _split_visits(waves, causal: bool, units: int) -> Optional[KvSplit]:
     # blocks 96 us against 85, 672 causal ones of up to 32 328 against 258).  So do causal pairs cut into more programs than
     # units (152 pairs of up to 16 blocks, two parts: 87 against 55) and short ones (up to 8 blocks: 42 against 37); 48
     # pairs of up to 24 blocks as four parts take 48 against 67.
-    if best[0] == 1 or (longest < 16 if len(walks) > 1 else best_us >= _tiles_us(2 * pairs, longest, units)):
+    if best[0] == 1 or (longest < 16 if len(walks) > 1 else best_us >= _tiles_us(2 * pairs, longest, tile_units)):
         return None
     return KvSplit(False, pairs, best[0], best[1])
 
