@@ -25,7 +25,7 @@ MAX_SLOTS = 1024          # partial results in memory at a time: 136 KB each
 BLOCK_US, SEGMENT_US, STEP_US = 3.6, 14.0, 8.0
 MERGE_US = 5.0
 MIN_GAIN_US = 10.0        # (the words and slots of the parts cost the host 3 us a launch, which small ones wait for)
-RESERVED_UNITS = 32       # compute units that waiting programs leave to the copies which raise their flags
+RESERVED_UNITS = 32       # compute units that launches which wait leave to the copies that raise their flags
 # Units that a producer does not count on: kernels that wait for its flags, one workgroup per side stream of an exchange, each
 # keep a unit from a workgroup that wants all registers, and a program too many for its XCD costs a round.  128 pairs
 # of 32 blocks as 256 programs: 85 us alone, 133 beside one such kernel; as single tiles, which share units with it, 96 and 95.
@@ -74,36 +74,17 @@ def plan_kv_split(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Se
     pairs = size[0] * size[1] * size[2] // (2 * BLOCK)
     lengths = [s[3] // BLOCK for _, s in waves]
     total = sum(lengths)
-    gated = [signal >= 0 for _, signal in zip(waves, signal_offsets)]
     # Programs that wait hold their compute unit with all its registers (eight wavefronts of 256), so that nothing else runs
     # there, a copy kernel that raises the flags among them.  Uncut pairs in fewer programs than units leave some free, and
     # the kernel with one tile per program room beside it however many tiles wait (two wavefronts of 232 registers per SIMD
-    # of 512): what takes the place of either does not fill the chip with programs that wait.
-    room = any(gated) and (always or pairs < units)
-
-    # runs of blocks behind flags
-    runs, start = [], 0
-    for waits, length in zip(gated, lengths):
-        if waits and runs and runs[-1][1] == start:
-            runs[-1][1] = start + length
-        elif waits:
-            runs.append([start, start + length])
-        start += length
-
-    def waiting_parts(parts: int) -> int:
-        count, counted = 0, 0                    # part p has the blocks from total * p // parts on
-        for lo, hi in runs:
-            first, last = ((lo + 1) * parts - 1) // total, (hi * parts - 1) // total
-            count += max(last + 1 - max(first, counted), 0)
-            counted = max(counted, last + 1)
-        return count
-
+    # of 512): what takes the place of either leaves units free, too, and from the start - with 256 programs of which 32 have
+    # nothing to wait for the copies start when those end (8 heads x 1024 rows, eight chunks of 1024 that copies of 16
+    # workgroups bring: 178 us, with 224 programs 148, single tiles 158; with 20 us between the copies 320, 290, 272).
+    room = (always or pairs < units) and any(signal >= 0 for _, signal in zip(waves, signal_offsets))
     best, best_us, whole_us = None, None, None
     for parts in range(1, min(MAX_PARTS, total) + 1):
         programs = pairs * parts
-        if pairs * (parts - 1) > MAX_SLOTS:
-            continue
-        if room and (always or parts > 1) and (programs > units or pairs * waiting_parts(parts) > units - RESERVED_UNITS):
+        if pairs * (parts - 1) > MAX_SLOTS or (room and (always or parts > 1) and programs > units - RESERVED_UNITS):
             continue
         us = -(-programs // units) * (-(-total // parts) * BLOCK_US + SEGMENT_US + STEP_US * _steps(parts))
         whole_us = whole_us or us
