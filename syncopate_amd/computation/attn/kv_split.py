@@ -80,11 +80,18 @@ def plan_kv_split(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Se
     # of 512): what takes the place of either leaves units free, too, and from the start - with 256 programs of which 32 have
     # nothing to wait for the copies start when those end (8 heads x 1024 rows, eight chunks of 1024 that copies of 16
     # workgroups bring: 178 us, with 224 programs 148, single tiles 158; with 20 us between the copies 320, 290, 272).
-    room = (always or pairs < units) and any(signal >= 0 for _, signal in zip(waves, signal_offsets))
+    flagged = [n for n, signal in zip(lengths, signal_offsets) if signal >= 0]
+    room = (always or pairs < units) and bool(flagged)
     best, best_us, whole_us = None, None, None
     for parts in range(1, min(MAX_PARTS, total) + 1):
         programs = pairs * parts
         if pairs * (parts - 1) > MAX_SLOTS or (room and (always or parts > 1) and programs > units - RESERVED_UNITS):
+            continue
+        # What is left to do when the last chunk arrives late: its blocks, on the one part of a pair that has them, and the
+        # steps whose other sides are long there, against one round of its tiles.  (8 heads x 1024 rows, a chunk of 8 blocks
+        # every 10 us: as 7 parts 41 us behind the last flag, as tiles 25; 2 heads, 16 blocks, as 16 parts 49 and 40.)
+        if always and flagged and (min(-(-total // parts), flagged[-1]) * BLOCK_US + SEGMENT_US + 2.0 * _steps(parts) >
+                                   _tiles_us(2 * pairs, flagged[-1], units)):
             continue
         us = -(-programs // units) * (-(-total // parts) * BLOCK_US + SEGMENT_US + STEP_US * _steps(parts))
         whole_us = whole_us or us

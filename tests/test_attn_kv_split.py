@@ -32,8 +32,13 @@ def test_plans():
     # nothing to wait for: no unit kept back
     assert plan(2, 4, 1536, [6144] * 4, [-1] * 4).programs > 224 >= plan(2, 4, 1536, [6144] * 4, [0] * 4).programs
     # only the first wave's programs do not wait; they hold units as long as they run
-    free_first = plan(1, 8, 1024, [1024] * 8, [-1] + list(range(7)), always=True)
+    free_first = plan(1, 8, 1024, [1024] * 8, [-1] + list(range(7)))
     assert free_first.programs <= 224 and free_first.pairs == 32
+    # what would be single tiles is cut only if it ends as early behind the last flag, too: parts shorter than a chunk
+    assert plan(1, 8, 1024, [1024] * 8, [-1] + list(range(7)), always=True) is None
+    assert plan(1, 2, 1024, [2048] * 8, [-1] + list(range(7)), always=True) is None
+    assert plan(1, 2, 512, [4096] * 8, [-1] + list(range(7)), always=True).parts == 16
+    assert plan(1, 8, 1024, [1024] * 8, [-1] * 8, always=True).parts == 8
     # enough pairs: stay whole where they would be chained, one part where they would be single tiles - but not where
     # they wait, on every compute unit and with all its registers, for flags that a kernel may have to raise
     assert plan(1, 32, 4096, [4096] * 8, [-1] + list(range(7))) is None
@@ -250,7 +255,8 @@ def test_same_tables_with_another_number_of_waves(hip, form):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,Sq,chunk,form,cut", [
-    (8, 1024, 1024, "explicit", True),
+    (2, 512, 4096, "explicit", True),
+    (8, 1024, 1024, "auto", True),
     (2, 512, 2048, "auto", True),
     (20, 1024, 1024, "explicit", False),         # more tiles than run at a time, all but the first wave's waiting
     (24, 3072, 512, "explicit", False),
@@ -401,7 +407,7 @@ def test_captured_split(hip, producer):
         cums = [(i + 1) * H * rows for i in range(chunks)]
     else:
         offsets, sizes, cums, _, _ = _chain_tables(1, H, Sq, [Skv // chunks] * chunks, None)
-    signals = list(range(chunks))
+    signals = list(range(chunks)) if producer else [-1] * chunks
     plan = plan_kv_split(offsets, sizes, cums, signals, causal=False, producer=producer, units=256, always=True)
     assert plan.parts > 1 and plan.chain != producer
     table = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
