@@ -70,6 +70,11 @@ def choose_xcd_remap(bm: int, bn: int) -> bool:
 # What a tile costs a program beyond and per 64-deep slab of K (RESIDENT_COST / 128), microseconds.
 SLAB_US = {shape: us / 128 for shape, us in RESIDENT_COST.items()}
 TILE_US = 3.0
+# What a launch that waits has to gain: cut, the tiles that wait for nothing use more units and the memory sooner, and copies
+# that run here begin 8 to 13 us slower (three to seven chunks by 32 workgroups).  Not cut any more: 4096 x 1024 x 512 and 1024 x
+# 2048 x 2048 on 128x256 tiles (41 -> 50 us and 64 -> 74 behind such copies), 2048 x 1536 x 1024 on 256x256 (43 -> 46); still
+# cut: 1024 x 5376 x 2752 on 256x256 (73 -> 67), 2048 x 768 x 6784 on 128x256 (105 -> 98).
+WAITING_GAIN_US = 15.0
 
 
 def choose_kernel_tile(tiles: int, programs: int, k: int, bm: int, bn: int, *, waiting: float = 0.0,
@@ -95,4 +100,5 @@ def choose_kernel_tile(tiles: int, programs: int, k: int, bm: int, bn: int, *, w
         cut = tiles * (bm // shape[0]) * (bn // shape[1])
         return cut <= programs and (units is None or cut <= units) and (room is None or cut * waiting <= room)
 
-    return min([(bm, bn)] + [shape for shape in SLAB_US if fits(shape)], key=cost)
+    best = min([(bm, bn)] + [shape for shape in SLAB_US if fits(shape)], key=cost)
+    return (bm, bn) if waiting and cost((bm, bn)) - cost(best) < WAITING_GAIN_US else best

@@ -12,7 +12,12 @@ def test_rule():
     assert choose_kernel_tile(256, 256, 8192, 256, 256) == (256, 256)       # a whole round
     assert choose_kernel_tile(129, 256, 8192, 128, 256) == (128, 256)       # twice as many would be two rounds
     assert choose_kernel_tile(128, 256, 512, 128, 256, waiting=1.0, room=224) == (128, 256)
-    assert choose_kernel_tile(128, 256, 512, 128, 256, waiting=0.75, room=224) == (128, 128)
+    assert choose_kernel_tile(128, 256, 8192, 128, 256, waiting=0.75, room=224) == (128, 128)
+    # a launch that waits gains more than its copies lose
+    assert choose_kernel_tile(128, 256, 512, 128, 256) == (128, 128)
+    assert choose_kernel_tile(128, 256, 512, 128, 256, waiting=0.75, room=224) == (128, 256)
+    assert choose_kernel_tile(48, 256, 1024, 256, 256, waiting=0.75, room=224) == (256, 256)
+    assert choose_kernel_tile(84, 256, 2752, 256, 256, waiting=0.75, room=224) == (256, 128)
     assert choose_kernel_tile(16, 256, 512, 256, 224) == (256, 224)         # no tile divides it
     assert choose_kernel_tile(16, 0, 512, 256, 256) == (256, 256)           # the library names the error
     assert choose_kernel_tile(200, 1024, 2048, 256, 256, units=256) == (256, 256)     # more programs than run at a time
