@@ -271,7 +271,7 @@ typedef struct syn_attn_desc {
     void* o;                        /* (z, h, q row, d)                                   */
     float* lse;                     /* [Z, H, Sq]                                         */
     int32_t* lock;                  /* [Z, H, Sq/block_m], zeroed; left in an unspecified state      */
-    int32_t* first;                 /* [Z, H, Sq/block_m], zeroed                         */
+    int32_t* first;                 /* [Z, H, Sq/block_m], zeroed (both: not read with SYN_ATTN_SPLIT_KV, may then be NULL) */
     uint64_t* flags;
     const int32_t* wave_offsets;    /* device, [num_waves, 4]                             */
     const int32_t* wave_sizes;      /* device, [num_waves, 4]                             */
@@ -375,6 +375,13 @@ typedef struct syn_attn_desc {
  * raise the flags, leave units without one that waits.  No counterpart in the reference. */
 #define SYN_ATTN_SPLIT_KV 32u
 #define SYN_ATTN_SPLIT_MAX_PARTS 16
+/* with SYN_ATTN_SPLIT_KV and SYN_ATTN_CHAIN_Q_BLOCKS: a pair's kv blocks are dealt to its split_parts programs one by one,
+ * block b (counted over all waves in a row) to part b % split_parts, so that every program goes through all chunks and a
+ * chunk that comes late is spread over all of them.  split_blocks and split_nodes are not read.  split_parts > 1: every part
+ * leaves its sums in a slot of its own, split_partials holds pairs * split_parts of them, and a second kernel of the same
+ * call adds them up in the order of the parts.  Workgroup b works on part b % split_parts of pair b / split_parts (dealt
+ * to the XCDs within rounds of 256 workgroups).  No counterpart in the reference. */
+#define SYN_ATTN_SPLIT_DEAL 64u
 #define SYN_ATTN_SPLIT_SLOT_BYTES 139264
 #define SYN_ATTN_WORK_PAIR_MASK 0x0fffffff
 #define SYN_ATTN_WORK_CONTINUES 0x10000000

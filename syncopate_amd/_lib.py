@@ -41,6 +41,7 @@ SYN_ATTN_CHAIN_Q_BLOCKS = 4
 SYN_ATTN_ACQUIRE_ALWAYS = 8
 SYN_ATTN_WORK_LIST = 16
 SYN_ATTN_SPLIT_KV = 32
+SYN_ATTN_SPLIT_DEAL = 64
 SYN_ATTN_SPLIT_MAX_PARTS = 16
 SYN_ATTN_SPLIT_SLOT_BYTES = 139264
 SYN_ATTN_WORK_PAIR_MASK = 0x0FFFFFFF

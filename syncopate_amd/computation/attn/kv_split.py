@@ -6,8 +6,8 @@ whose sums are added up in 32 bits at the end.  Host logic on plain integers, li
 
 Two kinds of tables can be cut:
 
-* consumer tables whose waves all list the same (z, h, q) ranges (the all-gather table): the parts are cut out of the kv
-  blocks of all waves in a row, in wave order;
+* consumer tables whose waves all list the same (z, h, q) ranges (the all-gather table): the kv blocks of all waves in a row
+  are dealt to the parts one by one, and a second kernel adds the parts up (SYN_ATTN_SPLIT_DEAL);
 * producer tables that visit every pair of q blocks once (attention that feeds an exchange), causal or not.
 """
 
@@ -19,10 +19,16 @@ BLOCK = 128
 MAX_WAVES = 256           # wave-table rows that the kernel holds in LDS
 MAX_PARTS = 16
 MAX_SLOTS = 1024          # partial results in memory at a time: 136 KB each
-# Microseconds, from kernel traces (256 programs of 8 blocks and three steps 66, 192 of 12 blocks and two steps 68, 256 of
-# 16 blocks and one step 80): a kv block of a pair, what a segment costs beyond its blocks (launch, Q, first fills,
-# epilogue), and a step of the tree that adds the parts (136 KB stored, handed over and loaded).
+# Microseconds, from kernel traces (256 programs of 16 blocks and one step 80, of 8 blocks and three steps 62): a kv block of a
+# pair, what a segment costs beyond its blocks (launch, Q, first fills, epilogue), and a step of the tree in which a
+# producer's parts are added (136 KB stored, handed over and loaded).
 BLOCK_US, SEGMENT_US, STEP_US = 3.6, 14.0, 8.0
+# The same where the blocks are dealt: a kv block on a nearly idle chip and what it takes longer where all units are busy, a
+# segment, and the second kernel (its launch, and 136 KB of every part stored and loaded; 256 parts 6.8 us, 16 4.1).
+# Measured: 32 pairs of 64 blocks as 1, 2, 4, 7, 8 parts 201, 112, 69, 54 and 51 us, 48 pairs of 48 as 2, 4, 5 90, 59 and 55.
+DEAL_BLOCK_US, DEAL_FULL_US, DEAL_SEGMENT_US, DEAL_ADD_US, DEAL_ADD_FULL_US = 2.8, 0.9, 13.0, 4.0, 5.0
+# What the host takes for a launch of two kernels and their slots: tiles that take less stay single.
+DEAL_HOST_US = 38.0
 MERGE_US = 5.0
 MIN_GAIN_US = 10.0        # (the words and slots of the parts cost the host 3 us a launch, which small ones wait for)
 RESERVED_UNITS = 32       # compute units that launches which wait leave to the copies that raise their flags
@@ -47,6 +53,14 @@ def _steps(parts: int) -> int:
     return (parts - 1).bit_length()
 
 
+def _deal_us(pairs: int, parts: int, blocks: int, units: int) -> float:
+    """What `pairs` of `blocks` kv blocks take, dealt to `parts` programs each."""
+    programs = pairs * parts
+    share = min(programs / units, 1.0)
+    us = -(-programs // units) * (-(-blocks // parts) * (DEAL_BLOCK_US + DEAL_FULL_US * share) + DEAL_SEGMENT_US)
+    return us + (DEAL_ADD_US + DEAL_ADD_FULL_US * programs / units if parts > 1 else 0.0)
+
+
 def plan_kv_split(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Sequence[int]], cum_wave_sizes: Sequence[int],
                   signal_offsets: Sequence[int], *, causal: bool, producer: bool, units: int,
                   always: bool) -> Optional[KvSplit]:
@@ -56,6 +70,24 @@ def plan_kv_split(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Se
     it would chain the uncut pairs, and None means that they stay whole."""
     if len(cum_wave_sizes) > MAX_WAVES or (causal and not producer):
         return None
+    waves = _real_waves(wave_offsets, wave_sizes, cum_wave_sizes, causal=causal, producer=producer)
+    if not waves:
+        return None
+    return _split_visits(waves, causal, units) if producer else _split_chain(waves, signal_offsets, units, always, dealt=False)
+
+
+def plan_kv_deal(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Sequence[int]], cum_wave_sizes: Sequence[int],
+                 signal_offsets: Sequence[int], *, units: int) -> Optional[KvSplit]:
+    """The split of a consumer's tables that wait for flags and that `plan_kv_split` leaves to the kernel with one tile per
+    program: there a late chunk is looked at as if its blocks were one part's, here as the parts share it."""
+    if len(cum_wave_sizes) > MAX_WAVES:
+        return None
+    waves = _real_waves(wave_offsets, wave_sizes, cum_wave_sizes, causal=False, producer=False)
+    return _split_chain(waves, signal_offsets, units, True, dealt=True) if waves else None
+
+
+def _real_waves(wave_offsets, wave_sizes, cum_wave_sizes, *, causal: bool, producer: bool):
+    """The waves in front of the padding, None where they cannot be cut."""
     waves, align = [], 2 * BLOCK if causal else BLOCK
     for cum, off, size in zip(cum_wave_sizes, wave_offsets, wave_sizes):
         if cum == 0:
@@ -65,11 +97,10 @@ def plan_kv_split(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Se
         if min(size) <= 0 or min(off) < 0 or size[2] % (2 * BLOCK) or size[3] % BLOCK or off[2] % align or off[3] % align:
             return None
         waves.append((off, size))
-    if not waves:
-        return None
-    if producer:
-        return _split_visits(waves, causal, units)
+    return waves
 
+
+def _split_chain(waves, signal_offsets: Sequence[int], units: int, always: bool, dealt: bool) -> Optional[KvSplit]:
     size = waves[0][1]
     pairs = size[0] * size[1] * size[2] // (2 * BLOCK)
     lengths = [s[3] // BLOCK for _, s in waves]
@@ -83,31 +114,40 @@ def plan_kv_split(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Se
     flagged = [n for n, signal in zip(lengths, signal_offsets) if signal >= 0]
     room = (always or pairs < units) and bool(flagged)
     best, best_us, whole_us = None, None, None
-    for parts in range(1, min(MAX_PARTS, total) + 1):
-        programs = pairs * parts
-        if pairs * (parts - 1) > MAX_SLOTS or (room and (always or parts > 1) and programs > units - RESERVED_UNITS):
-            continue
-        # What is left to do when the last chunk arrives late: its blocks, on the one part of a pair that has them, and the
-        # steps whose other sides are long there, against one round of its tiles.  (8 heads x 1024 rows, a chunk of 8 blocks
-        # every 10 us: as 7 parts 41 us behind the last flag, as tiles 25; 2 heads, 16 blocks, as 16 parts 49 and 40.)
-        if always and flagged and (min(-(-total // parts), flagged[-1]) * BLOCK_US + SEGMENT_US + 2.0 * _steps(parts) >
-                                   _tiles_us(2 * pairs, flagged[-1], units)):
-            continue
-        us = -(-programs // units) * (-(-total // parts) * BLOCK_US + SEGMENT_US + STEP_US * _steps(parts))
-        whole_us = whole_us or us
-        if best is None or us < best_us:
-            best, best_us = parts, us
+    most = min(MAX_PARTS, total)
     if always:
         tiles = 2 * pairs * len(waves)
         # visits to a q block that end at the same time are merged one after the other
         merges = min(len(waves), units // pairs) - 1 if tiles <= 2 * units else 0
         tiles_us = _tiles_us(tiles, -(-total // len(waves)), units) + MERGE_US * merges
-        if best is None or best_us >= tiles_us:
+        if tiles_us < DEAL_HOST_US:
             return None
-        # Whole pairs that leave units idle (135 of 28 blocks 102 us, as tiles 89), or whose gain is within what the two
-        # models are off (560 of 22 blocks 259 us, as tiles 225).  Over 1000 tables drawn anew (500 of them producers') four
+        if flagged:
+            last_us = _tiles_us(2 * pairs, flagged[-1], units)
+            if not dealt and min(-(-total // most), flagged[-1]) * BLOCK_US + SEGMENT_US > last_us:
+                return None                      # (however many parts)
+    for parts in range(1, most + 1):
+        programs = pairs * parts
+        if (parts > 1 and programs > MAX_SLOTS) or (room and (always or parts > 1) and programs > units - RESERVED_UNITS):
+            break
+        us = _deal_us(pairs, parts, total, units)
+        # What is left to do when the last chunk arrives late, against one round of its tiles.  Without `dealt` only tables
+        # that would end as early if one part had all its blocks; with it, the share of a part and the second kernel, and
+        # where that takes longer, the launch has to gain as much with every chunk there.
+        if always and flagged:
+            if not dealt and min(-(-total // parts), flagged[-1]) * BLOCK_US + SEGMENT_US + 2.0 * _steps(parts) > last_us:
+                continue
+            us += max(_deal_us(pairs, parts, flagged[-1], units) - last_us, 0.0) if dealt else 0.0
+        whole_us = whole_us or us
+        if best is None or us < best_us:
+            best, best_us = parts, us
+    if always:
+        if best is None:
+            return None
+        # Whole pairs that leave units idle (135 of 28 blocks 102 us, as tiles 89), a gain within what the two models are off
+        # (560 whole pairs of 22 blocks 259 us, as tiles 225; 75 of 172 as two parts 295 and 277).  Over 1000 tables drawn anew (500 of them producers') four
         # lose more than 3 %, the most 7 % (324 pairs of 28 blocks), and the medians gain 20 to 39 %.
-        if best == 1 and (8 * pairs < 7 * units or 1.05 * best_us >= tiles_us):
+        if (best == 1 and 8 * pairs < 7 * units) or 1.05 * best_us >= tiles_us:
             return None
     elif best_us > min(0.85 * whole_us, whole_us - MIN_GAIN_US):
         return None

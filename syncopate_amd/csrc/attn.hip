@@ -62,8 +62,8 @@ struct AttnParams {
     int32_t xcd_remap;    // workgroups of one XCD take consecutive tiles (see logical_program_id)
     int32_t acquire_always;   // SYN_ATTN_ACQUIRE_ALWAYS: fence behind every flag wait, not only behind a spin
     const int32_t* work_list; // SYN_ATTN_WORK_LIST: [grid + 1] entry offsets, then the entries
-    // SYN_ATTN_SPLIT_KV: parts per pair of q blocks (at most), kv blocks per part (at least, where the parts allow),
-    // one zeroed word per pair and part, and the slots of the partial results
+    // SYN_ATTN_SPLIT_KV: parts per pair of q blocks (at most; exactly with SYN_ATTN_SPLIT_DEAL), kv blocks per part (at least,
+    // where the parts allow), one zeroed word per pair and part, and the slots of the partial results
     int32_t split_parts, split_blocks;
     int32_t* split_nodes;
     unsigned char* split_partials;
@@ -792,16 +792,20 @@ constexpr int kPartialRecords = 17;
 constexpr size_t kPartialSlotBytes = (size_t)8 * kPartialRecords * 1024;
 static_assert(kPartialSlotBytes == SYN_ATTN_SPLIT_SLOT_BYTES, "the caller sizes the slots");
 
+// (THROUGH: for a reader of the same launch; a kernel behind this one finds plain stores, too.)
+template <bool THROUGH>
 __device__ __forceinline__ void store_partial(unsigned char* slot, const f32x4_t (&o_acc)[8][2], const float (&m)[2],
                                               const float (&l)[2], int wave8, int lane) {
     unsigned char* const dst = slot + ((size_t)wave8 * kPartialRecords * 64 + lane) * 16;
+    auto store16 = [](unsigned char* to, const f32x4_t x) {
+        if constexpr (THROUGH) store16_write_through(to, __builtin_bit_cast(uint4, x));
+        else *reinterpret_cast<f32x4_t*>(to) = x;
+    };
 #pragma unroll
     for (int t = 0; t < 8; ++t)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
-            store16_write_through(dst + (2 * t + b) * 1024, __builtin_bit_cast(uint4, o_acc[t][b]));
-    const f32x4_t stats = {m[0], m[1], l[0], l[1]};
-    store16_write_through(dst + 16 * 1024, __builtin_bit_cast(uint4, stats));
+        for (int b = 0; b < 2; ++b) store16(dst + (2 * t + b) * 1024, o_acc[t][b]);
+    store16(dst + 16 * 1024, f32x4_t{m[0], m[1], l[0], l[1]});
 }
 
 // The sum of two partial results.  Each product is rounded by itself (no fused multiply-add), so that a + b and b + a are
@@ -859,7 +863,13 @@ __device__ __forceinline__ void add_partial(const unsigned char* slot, f32x4_t (
 //                    per program, merged in memory: 76); 128 pairs of 32, as two: 79 (256 tiles, nothing merged: 85).
 //                    A part costs 3.6 us a kv block; the first K block, Q and the epilogue 14 us; a step of the tree 8 us,
 //                    which is 136 KB through memory and three trips for the words that hand it over.
-constexpr int kPairTiles = 0, kPairChainWaves = 1, kPairWorkList = 2, kPairSplitChain = 3, kPairSplitVisit = 4;
+//   kPairSplitDeal   (SYN_ATTN_SPLIT_DEAL) chained waves whose kv blocks are dealt to the parts one by one, block b to part
+//                    b % parts, so that all parts go through the chunks together and share the last one; a kernel behind this
+//                    one adds them up (attn_add_parts_kernel), where the tree took 8 us a step.  32 pairs of 64 kv blocks as
+//                    eight parts 61 -> 51 us, 48 pairs of 48 as five 60 -> 55.  From entry to the first products takes 6.5 us
+//                    (wave table and flags 1.3, what the part is 3, the first K block and Q 2), a block 3.4 with all units
+//                    busy (2.8 with an eighth of them; without the fills 3.3), the sums 3 to 8 on their way to memory.
+constexpr int kPairTiles = 0, kPairChainWaves = 1, kPairWorkList = 2, kPairSplitChain = 3, kPairSplitVisit = 4, kPairSplitDeal = 5;
 constexpr int32_t kWorkPairMask = SYN_ATTN_WORK_PAIR_MASK;
 constexpr int kUnits = 256;              // compute units of the chip, each of which runs one workgroup of this kernel
 constexpr int kPairLdsWaves = 256, kPairLdsEntries = 512;
@@ -868,8 +878,9 @@ template <typename T, int MODE, bool CAUSAL>
 __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnParams p) {
     typedef typename AttnMfma<T>::frag_t frag_t;
     typedef T vec4_t __attribute__((ext_vector_type(4)));
-    constexpr bool kSplitChain = MODE == kPairSplitChain, kSplit = kSplitChain || MODE == kPairSplitVisit;
-    static_assert(!(CAUSAL && (MODE == kPairChainWaves || kSplitChain)), "the waves of a causal table do not share their kv extent");
+    constexpr bool kSplitChain = MODE == kPairSplitChain, kDeal = MODE == kPairSplitDeal;
+    constexpr bool kSplit = kSplitChain || kDeal || MODE == kPairSplitVisit;
+    static_assert(!(CAUSAL && (MODE == kPairChainWaves || kSplitChain || kDeal)), "the waves of a causal table do not share their kv extent");
 
     __shared__ __attribute__((aligned(1024))) unsigned char k_lds[2 * kBlockBytes];
     __shared__ __attribute__((aligned(1024))) unsigned char v_lds[2 * kPairVBlockBytes];
@@ -885,6 +896,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
     // here: kept in registers through the loop it costs spills inside it, whose reloads wait for the fills in flight
     enum { kLatePair, kLatePart, kLateParts, kLateWave, kLateSignal, kLateZ, kLateH, kLateQ };
     __shared__ int s_late[8];
+    __shared__ int s_waves_up;           // kPairSplitDeal: the waves in front of this one need not be waited for
     auto late = [&](const int what) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane(s_late[what]); };
 
     const int tid = threadIdx.x;
@@ -906,6 +918,15 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
         s_row[w][5] = p.wave_offsets[w * 4 + 3] / kBlockN;
         s_row[w][6] = p.wave_sizes[w * 4 + 3] / kBlockN;
         s_row[w][7] = p.signal_offsets[w];
+    }
+    if constexpr (kDeal) {
+        // the first 64 waves' flags, read beside the table (see wait_for_wave)
+        if (wave8 == 0) {
+            const int sg = lane < p.num_waves && p.cum_wave_sizes[lane] != 0 ? p.signal_offsets[lane] : -1;
+            const bool up = sg < 0 || __hip_atomic_load(p.flags + sg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 1ull;
+            const unsigned long long down = ~__builtin_amdgcn_ballot_w64(up);
+            if (lane == 0) s_waves_up = down == 0 ? 64 : (int)__builtin_ctzll(down);
+        }
     }
 
     // LDS layouts of this kernel (row = kv position in the block, 16 chunks of 16 bytes per row):
@@ -944,7 +965,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
     T* __restrict__ O = reinterpret_cast<T*>(p.o);
 
     const int pairs_per_wave = p.cum_wave_sizes[0] / kBlockM / 2;
-    const int num_pairs = MODE == kPairChainWaves || kSplitChain ? pairs_per_wave : p.num_tiles / 2;
+    const int num_pairs = MODE == kPairChainWaves || kSplitChain || kDeal ? pairs_per_wave : p.num_tiles / 2;
     if (kSplit && (int)gridDim.x != num_pairs * p.split_parts) {
         if (tid == 0) report_status(p.status, SYN_STATUS_BAD_CHAIN, 0, (int)blockIdx.x, num_pairs);
         return;
@@ -967,6 +988,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
     // (12 heads x 8192 rows x 32 kv blocks in eight chunks, 768 programs in 280 us: the first flags go up at 201, dealt over
     // the whole grid every chunk was one XCD's and all eight went up at 300; one tile per program: 201 and 290).
     int part = 0, parts = 1, part_left = 0;
+    int dealt_on = 0;            // kPairSplitDeal: where in the next wave the part's next block lies
     if constexpr (kSplit) {
         part = kSplitChain ? program / num_pairs : program % p.split_parts;
         pair = kSplitChain ? logical_program_id(program % num_pairs, num_pairs, p.xcd_remap != 0) : program / p.split_parts;
@@ -1061,6 +1083,76 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
         __syncthreads();       // s_spun may be written again only when everyone has read it
         return ok;
     };
+    // kPairSplitDeal: a part enters a wave every few blocks.  The flags of the next 64 waves are read at once, one per lane, and
+    // those in a row that are up are not looked at again (a flag goes up once per launch).
+    int waves_up = 0, real_waves = 0;
+    auto wait_for_wave = [&](const int wv) __attribute__((always_inline)) -> bool {
+        if (wv < waves_up) return true;
+        if (wave8 == 0) {
+            const int idx = wv + lane;
+            const int sg = idx < real_waves ? s_row[idx][7] : -1;
+            const bool up = sg < 0 || __hip_atomic_load(p.flags + sg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 1ull;
+            const unsigned long long down = ~__builtin_amdgcn_ballot_w64(up);
+            if (lane == 0) {
+                s_spun = (int)(down & 1);
+                s_waves_up = wv + (down == 0 ? 64 : max((int)__builtin_ctzll(down), 1));
+                if (s_spun && !spin_until_equal(p.flags + sg, 1ull, p.timeout_ticks)) {
+                    report_status(p.status, SYN_STATUS_SPIN_TIMEOUT, wv, (int)blockIdx.x, sg);
+                    s_abort = 1;
+                }
+            }
+        }
+        __syncthreads();
+        waves_up = __builtin_amdgcn_readfirstlane(s_waves_up);
+        // see attn_fwd_kernel.  One wavefront's fence drops the lines of the compute unit's L1 and the XCD's L2 for all eight,
+        // which load behind the barrier below.  (All programs pass here at every chunk that comes late, and the fences of
+        // all their wavefronts held up the kernels that raise the next flags: 32 pairs, seven flags 5 and 20 us apart,
+        // the last went up at 82 and 189 us instead of 62 and 170.)
+        if (wave8 == 0 && (__builtin_amdgcn_readfirstlane(s_spun) || p.acquire_always)) {
+            acquire_fence_agent();
+            __builtin_amdgcn_s_waitcnt(attn_vmcnt(0));
+        }
+        const bool ok = __builtin_amdgcn_readfirstlane(s_abort) == 0;
+        __syncthreads();       // the words may be written again only when everyone has read them
+        return ok;
+    };
+    // kPairSplitDeal: what the program's part is, worked out from the table with a lane per wave
+    int first_wave = 0;
+    if constexpr (kDeal) {
+        // (every wave has to list wave 0's q blocks: a part reads each wave's kv range for them)
+        int before = 0, other = -1;
+        for (int base = 0; base < p.num_waves; base += 64) {
+            const int idx = base + lane;
+            const int cum = idx < p.num_waves ? s_cum[idx] : 0;
+            bool same = cum == 0 || cum == 2 * (idx + 1) * pairs_per_wave;
+#pragma unroll
+            for (int f = 0; f < 5; ++f) same = same && (cum == 0 || s_row[idx][f] == s_row[0][f]);
+            const unsigned long long differ = __builtin_amdgcn_ballot_w64(!same);
+            if (differ != 0 && other < 0) other = base + __builtin_ctzll(differ);
+            int blocks = cum != 0 ? s_row[idx][6] : 0;      // kv blocks of the waves of `base` .. idx
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int below = __shfl_up(blocks, d);
+                blocks += lane >= d ? below : 0;
+            }
+            const int here = __builtin_amdgcn_readlane(blocks, 63);
+            if (before <= part && part < before + here) {
+                const int ahead = __builtin_popcountll(__builtin_amdgcn_ballot_w64(before + blocks <= part));
+                first_wave = base + ahead;
+                dealt_on = part - before - (ahead == 0 ? 0 : __builtin_amdgcn_readlane(blocks, ahead - 1));
+            }
+            before += here;
+            real_waves += __builtin_popcountll(__builtin_amdgcn_ballot_w64(cum != 0));
+        }
+        if (other >= 0) {
+            if (tid == 0) report_status(p.status, SYN_STATUS_BAD_CHAIN, other, (int)blockIdx.x, 2 * pair);
+            return;
+        }
+        parts = p.split_parts;
+        part_left = before > part ? (before - part + parts - 1) / parts : 0;
+        waves_up = __builtin_amdgcn_readfirstlane(s_waves_up);
+        if (p.acquire_always && waves_up > 0) acquire_fence_agent();
+    }
 
     for (; pending(); advance()) {
         // ---- the segment's first visit: tile id -> wave -> (z, h, q block, kv range); the two tiles of a pair
@@ -1071,7 +1163,21 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
         const bool sole_writer = MODE == kPairChainWaves || (MODE == kPairWorkList && (entry & SYN_ATTN_WORK_SOLE_WRITER));
         const int tile_id = 2 * pair_id + grp;
         Where first;
-        if (!locate(tile_id, first)) return;
+        if constexpr (kDeal) {
+            int row[8];
+#pragma unroll
+            for (int f = 0; f < 8; ++f) row[f] = __builtin_amdgcn_readfirstlane(s_row[0][f]);
+            first.w = 0;
+            first.z = tile_id / (row[1] * row[0]) + row[2];
+            first.h = (tile_id / row[1]) % row[0] + row[3];
+            first.qb = tile_id % row[1] + row[4];
+            first.kv_lo = row[5];
+            first.kv_len = row[6];
+            first.sig = row[7];
+            first.paired = !(row[1] & 1);
+        } else {
+            if (!locate(tile_id, first)) return;
+        }
         const int z = first.z, h = first.h, qb = first.qb;
         int w = first.w, kv_lo = first.kv_lo, kv_len = first.kv_len, sig = first.sig;
         // the caller promised an even number of q blocks per wave (and, under a causal mask, q ranges and kv
@@ -1112,10 +1218,28 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
             // begins at or below the lower q block, so that every row finds an unmasked position in its first block.
             constexpr int kUnit = CAUSAL ? 2 : 1;
             const int units = total / kUnit;
-            parts = min(min(p.split_parts, (total + p.split_blocks - 1) / p.split_blocks), max(units, 1));
-            if (part >= parts) continue;
-            int begin = units * part / parts * kUnit;
-            part_left = (part + 1 == parts ? total : units * (part + 1) / parts * kUnit) - begin;
+            int begin = 0;
+            if constexpr (kDeal) {
+                if (part_left == 0) {                   // more parts than blocks: sums of nothing
+                    const f32x4_t none[8][2] = {};
+                    const float no_max[2] = {-FLT_MAX, -FLT_MAX}, no_sum[2] = {0.f, 0.f};
+                    store_partial<false>(p.split_partials + ((size_t)pair * parts + part) * kPartialSlotBytes, none, no_max, no_sum,
+                                         wave8, lane);
+                    continue;
+                }
+                w = first_wave;
+                kv_lo = __builtin_amdgcn_readfirstlane(s_row[w][5]) + dealt_on;
+                kv_len = __builtin_amdgcn_readfirstlane(s_row[w][6]);
+                sig = __builtin_amdgcn_readfirstlane(s_row[w][7]);
+                const int here = (kv_len - dealt_on + parts - 1) / parts;
+                dealt_on += here * parts - kv_len;
+                kv_len = here;
+            } else {
+                parts = min(min(p.split_parts, (total + p.split_blocks - 1) / p.split_blocks), max(units, 1));
+                if (part >= parts) continue;
+                begin = units * part / parts * kUnit;
+                part_left = (part + 1 == parts ? total : units * (part + 1) / parts * kUnit) - begin;
+            }
             if constexpr (kSplitChain) {
                 while (begin >= s_row[w][6]) begin -= s_row[w++][6];
                 w = __builtin_amdgcn_readfirstlane(w);
@@ -1130,8 +1254,10 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
                 sig = __builtin_amdgcn_readfirstlane(s_row[w][7]);
                 begin = __builtin_amdgcn_readfirstlane(begin);
             }
-            kv_lo += begin;
-            kv_len = min(kv_len - begin, part_left);
+            if constexpr (!kDeal) {
+                kv_lo += begin;
+                kv_len = min(kv_len - begin, part_left);
+            }
             part_left -= kv_len;
             if (tid == 0) {
                 s_late[kLatePair] = pair;
@@ -1148,11 +1274,24 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
         const int nkv = CAUSAL ? min(kv_len, diag_hi + 1 - kv_lo) : kv_len;
         if (CAUSAL && nkv <= 0) continue;               // wholly above the diagonal: visited, nothing to add
 
-        if (sig >= 0 && !(MODE == kPairSplitVisit && p.counters != nullptr) && !wait_for_flag(sig, w)) return;
-
-        const size_t head = (size_t)z * p.H + h;
+        // Q^T operands of the two 16-row halves of the slice: [b][ks] = Q[q_row + 16 b][32 ks + 8 g .. + 8]
         const int q_row = qb * kBlockM + wave * 32 + c16;          // and q_row + 16
         const T* q_src = Q + z * p.q_st[0] + h * p.q_st[1] + q_row * p.q_st[2] + 8 * g;
+        frag_t qf[2][4];
+        auto load_q = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks) qf[b][ks] = *reinterpret_cast<const frag_t*>(q_src + 16 * b * p.q_st[2] + 32 * ks);
+        };
+        if constexpr (kDeal) {
+            load_q();                                   // (no flag covers Q)
+            if (!wait_for_wave(w)) return;
+        } else {
+            if (sig >= 0 && !(MODE == kPairSplitVisit && p.counters != nullptr) && !wait_for_flag(sig, w)) return;
+        }
+
+        const size_t head = (size_t)z * p.H + h;
         const unsigned char* const k_head = K + (z * p.k_st[0] + h * p.k_st[1]) * (int64_t)sizeof(T);
         const unsigned char* const v_head = V + (z * p.v_st[0] + h * p.v_st[1]) * (int64_t)sizeof(T);
 
@@ -1172,6 +1311,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
 
         // ---- the walk: the K fills run one block ahead of the V fills; both step through the visit's blocks
         //      (rotated) and the K walk enters the segment's next visit when its own is used up ----
+        const int k_apart = kDeal ? parts : 1;           // blocks from one of the walk to the next
         int k_lo = kv_lo, k_nkv = nkv, k_next = 1, k_rot = rotation(kv_lo, kv_len, nkv);
         int v_nkv = nkv, v_next = 0, v_rot = k_rot;
         const unsigned char* k_walk = k_head + (size_t)kv_lo * kBlockN * k_pitch;
@@ -1209,7 +1349,21 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
         // the K walk enters the segment's next visit: 1 entered, 0 the segment ends here, -1 give up
         auto enter_next_visit = [&]() __attribute__((always_inline)) -> int {
             int next_tile;
-            if constexpr (MODE == kPairTiles) {
+            if constexpr (kDeal) {
+                if (part_left == 0) return 0;          // (while there are blocks left, there is a wave that has them)
+                int blocks;
+                while (blocks = __builtin_amdgcn_readfirstlane(s_row[++k_wave][6]), dealt_on >= blocks) dealt_on -= blocks;
+                const int here = (blocks - dealt_on + parts - 1) / parts;
+                if (!wait_for_wave(k_wave)) return -1;
+                k_lo = __builtin_amdgcn_readfirstlane(s_row[k_wave][5]) + dealt_on;
+                k_nkv = here;
+                k_rot = rotation(k_lo, here, here);
+                k_next = 0;
+                k_walk = k_head + (size_t)k_lo * kBlockN * k_pitch;
+                dealt_on += here * parts - blocks;
+                part_left -= here;
+                return 1;
+            } else if constexpr (MODE == kPairTiles) {
                 return 0;
             } else if constexpr (MODE == kPairChainWaves) {
                 if (k_wave + 1 >= p.num_waves || p.cum_wave_sizes[k_wave + 1] == 0) return 0;
@@ -1259,14 +1413,9 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
         };
         look_ahead();
         // every wavefront has passed the barrier that ended the previous segment: all four buffers are free
-        dma_kv_block8(k_lds, k_walk + (size_t)k_rot * kBlockN * k_pitch, k_pitch, k_fill_off, wave8);
+        dma_kv_block8(k_lds, k_walk + (size_t)(k_rot * k_apart) * kBlockN * k_pitch, k_pitch, k_fill_off, wave8);
 
-        // Q^T operands of the two 16-row halves of the slice: [b][ks] = Q[q_row + 16 b][32 ks + 8 g .. + 8]
-        frag_t qf[2][4];
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) qf[b][ks] = *reinterpret_cast<const frag_t*>(q_src + 16 * b * p.q_st[2] + 32 * ks);
+        if constexpr (!kDeal) load_q();
         // O^T: [t][b] = columns 16 t + 4 g + 0..3 of q row 16 b + c16
         f32x4_t o_acc[8][2];
 #pragma unroll
@@ -1319,7 +1468,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
             }
             int b = v_next + v_rot;
             b = b >= v_nkv ? b - v_nkv : b;
-            v_src_pending = v_walk + (size_t)b * kBlockN * v_pitch;       // for group 0's fill_v, one slot on
+            v_src_pending = v_walk + (size_t)(b * k_apart) * kBlockN * v_pitch;       // for group 0's fill_v, one slot on
             v_buf_pending = m & 1;
             ++v_next;
             int more = 1;
@@ -1328,7 +1477,8 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
                 b = k_next + k_rot;
                 b = b >= k_nkv ? b - k_nkv : b;
                 if (grp == 1)
-                    dma_kv_block4(k_lds + ((m + 1) & 1) * kBlockBytes, k_walk + (size_t)b * kBlockN * k_pitch, k_pitch, k_fill_off, wave);
+                    dma_kv_block4(k_lds + ((m + 1) & 1) * kBlockBytes, k_walk + (size_t)(b * k_apart) * kBlockN * k_pitch, k_pitch, k_fill_off,
+                                  wave);
                 ++k_next;
                 if constexpr (CAUSAL) m2 = beyond(k_lo + b);
             }
@@ -1451,10 +1601,10 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
             typedef short s16x8_t __attribute__((ext_vector_type(8)));
             __builtin_amdgcn_s_setprio(3);
             const unsigned char* v_blk = v_lds + (n & 1) * kPairVBlockBytes;
-            // (kSplitChain, which has the most to carry: three of the four addresses are made here from the first - the
+            // (the chained split forms, which have the most to carry: three of the four addresses are made here from the first - the
             // exclusive-or of v_rd - and not carried around the loop, where they would be spilled)
             int rd[4] = {v_rd[0], v_rd[1], v_rd[2], v_rd[3]};
-            if constexpr (kSplitChain) {
+            if constexpr (kSplitChain || kDeal) {
                 asm volatile("" : "+v"(rd[0]));
 #pragma unroll
                 for (int t = 1; t < 4; ++t) rd[t] = rd[0] ^ (32 * t);
@@ -1587,6 +1737,13 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
             const int late_lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
             const int own_pair = late(kLatePair), own_parts = late(kLateParts);
             int at = late(kLatePart);
+            if constexpr (kDeal) {
+                if (own_parts > 1) {
+                    store_partial<false>(p.split_partials + ((size_t)own_pair * own_parts + at) * kPartialSlotBytes, o_acc, m_i, l_row,
+                                         wave8, late_lane);
+                    return;
+                }
+            }
             for (int step = 1; step < own_parts; step <<= 1) {
                 const int right = (at & step) ? at : at + step;
                 if (right >= own_parts) continue;
@@ -1595,7 +1752,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
                 if (tid == 0) s_spun = __hip_atomic_fetch_add(node, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 1;
                 __syncthreads();
                 if (__builtin_amdgcn_readfirstlane(s_spun) == 0) {
-                    store_partial(slot, o_acc, m_i, l_row, wave8, late_lane);
+                    store_partial<true>(slot, o_acc, m_i, l_row, wave8, late_lane);
                     __builtin_amdgcn_s_waitcnt(attn_vmcnt(0));       // every lane's stores acknowledged, then the barrier
                     __syncthreads();
                     if (tid == 0) {
@@ -1696,10 +1853,78 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
     }
 }
 
+// What follows kPairSplitDeal: the sum of a pair's parts, in the order of the parts, written as whole rows.  A workgroup per
+// wavefront of the pair (32 q rows); each of its own eight wavefronts takes the 16 rows of one half and 32 columns, reads the
+// parts' statistics and two records of each part, four parts at a time, and writes 64 bytes of a row.
+template <typename T>
+__global__ void __launch_bounds__(kPairThreads) attn_add_parts_kernel(const AttnParams p) {
+    typedef T vec4_t __attribute__((ext_vector_type(4)));
+    constexpr int kAtOnce = 4;
+    const int lane = threadIdx.x & 63, job = threadIdx.x >> 6;
+    const int pair = blockIdx.x >> 3, wave8 = blockIdx.x & 7;
+    const int b = job & 1, t0 = job & ~1;
+    const int c16 = lane & 15, g = lane >> 4;
+    const int parts = p.split_parts;
+    const unsigned char* const src = p.split_partials + (size_t)pair * parts * kPartialSlotBytes +
+                                     ((size_t)wave8 * kPartialRecords * 64 + lane) * 16;
+
+    float top = -FLT_MAX, l = 0.f;
+    f32x4_t sum[2] = {};
+    for (int first = 0; first < parts; first += kAtOnce) {
+        f32x4_t stats[kAtOnce], x[kAtOnce][2];
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i) {
+            const unsigned char* const slot = src + (size_t)min(first + i, parts - 1) * kPartialSlotBytes;
+            stats[i] = *reinterpret_cast<const f32x4_t*>(slot + 16 * 1024);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) x[i][t] = *reinterpret_cast<const f32x4_t*>(slot + (2 * (t0 + t) + b) * 1024);
+        }
+        float m[kAtOnce], new_top = top;
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i) {
+            m[i] = stats[i][b];
+            new_top = fmaxf(new_top, m[i]);
+        }
+        const float w_old = fast_exp2(top - new_top);
+        l *= w_old;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) sum[t] *= w_old;
+        top = new_top;
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i) {
+            if (first + i >= parts) break;
+            const float w = fast_exp2(m[i] - top);
+            l += stats[i][2 + b] * w;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) sum[t] += x[i][t] * w;
+        }
+    }
+
+    const int size_h = p.wave_sizes[1], nq = p.wave_sizes[2] / kBlockM;
+    const int tile = 2 * pair + (wave8 >> 2);
+    const int z = tile / (nq * size_h) + p.wave_offsets[0], h = (tile / nq) % size_h + p.wave_offsets[1];
+    const int row = (tile % nq + p.wave_offsets[2] / kBlockM) * kBlockM + (wave8 & 3) * 32 + 16 * b + c16;
+    const float inv_l = 1.0f / l;
+    T* const out = reinterpret_cast<T*>(p.o) + z * p.o_st[0] + h * p.o_st[1] + row * p.o_st[2] + 16 * t0 + 4 * g;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        vec4_t v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (T)(sum[t][i] * inv_l);
+        *reinterpret_cast<vec4_t*>(out + 16 * t) = v;
+    }
+    if (t0 == 0 && g == 0) p.lse[((size_t)z * p.H + h) * p.Sq + row] = top + fast_log2(l);
+}
+
 template <typename T>
 static int launch_attn_pairs(const AttnParams& p, int grid, int mode, bool causal, hipStream_t stream) {
     const dim3 g(grid), b(kPairThreads);
-    if (mode == kPairSplitChain)
+    if (mode == kPairSplitDeal) {
+        hipLaunchKernelGGL((attn_pair_kernel<T, kPairSplitDeal, false>), g, b, 0, stream, p);
+        const hipError_t err = hipGetLastError();
+        if (err != hipSuccess || p.split_parts == 1) return (int)err;
+        hipLaunchKernelGGL((attn_add_parts_kernel<T>), dim3(grid / p.split_parts * 8), b, 0, stream, p);
+    } else if (mode == kPairSplitChain)
         hipLaunchKernelGGL((attn_pair_kernel<T, kPairSplitChain, false>), g, b, 0, stream, p);
     else if (mode == kPairSplitVisit && causal)
         hipLaunchKernelGGL((attn_pair_kernel<T, kPairSplitVisit, true>), g, b, 0, stream, p);
@@ -1844,7 +2069,8 @@ int syn_attn_check_work_list(const int32_t* wave_offsets, const int32_t* wave_si
 int syn_attn_fwd(const syn_attn_desc* d, syn_stream_t stream) {
     using namespace syn;
     if (d == nullptr) return SYN_EINVAL;
-    if (!d->q || !d->k || !d->v || !d->o || !d->lse || !d->lock || !d->first) return SYN_EINVAL;
+    if (!d->q || !d->k || !d->v || !d->o || !d->lse) return SYN_EINVAL;
+    if ((!d->lock || !d->first) && !(d->options & SYN_ATTN_SPLIT_KV)) return SYN_EINVAL;     // (the split forms take no locks)
     if (!d->wave_offsets || !d->wave_sizes || !d->cum_wave_sizes || !d->signal_offsets || !d->flags)
         return SYN_EINVAL;
     if (d->num_waves <= 0 || d->Z <= 0 || d->H <= 0 || d->Sq <= 0 || d->Skv <= 0) return SYN_EINVAL;
@@ -1934,9 +2160,11 @@ int syn_attn_fwd(const syn_attn_desc* d, syn_stream_t stream) {
             if (d->split_parts < 1 || d->split_parts > SYN_ATTN_SPLIT_MAX_PARTS || d->split_blocks < 1) return SYN_EINVAL;
             if (d->num_programs <= 0 || d->num_programs % d->split_parts) return SYN_EINVAL;
             if (!chain && d->num_programs / d->split_parts != tiles / 2) return SYN_EINVAL;
-            if (d->split_parts > 1 && (!d->split_nodes || !d->split_partials)) return SYN_EINVAL;
+            const bool deal = (d->options & SYN_ATTN_SPLIT_DEAL) != 0;
+            if (deal && !chain) return SYN_EINVAL;
+            if (d->split_parts > 1 && ((!d->split_nodes && !deal) || !d->split_partials)) return SYN_EINVAL;
             if (!aligned16(d->split_partials)) return SYN_EALIGN;
-            const int form = chain ? kPairSplitChain : kPairSplitVisit;
+            const int form = deal ? kPairSplitDeal : chain ? kPairSplitChain : kPairSplitVisit;
             return d->dtype == SYN_DTYPE_BF16 ? launch_attn_pairs<__bf16>(p, d->num_programs, form, d->causal != 0, s)
                                               : launch_attn_pairs<_Float16>(p, d->num_programs, form, d->causal != 0, s);
         }
@@ -1946,7 +2174,7 @@ int syn_attn_fwd(const syn_attn_desc* d, syn_stream_t stream) {
         return d->dtype == SYN_DTYPE_BF16 ? launch_attn_pairs<__bf16>(p, grid, mode, d->causal != 0, s)
                                           : launch_attn_pairs<_Float16>(p, grid, mode, d->causal != 0, s);
     }
-    if (d->options & (SYN_ATTN_CHAIN_Q_BLOCKS | SYN_ATTN_WORK_LIST | SYN_ATTN_SPLIT_KV)) return SYN_EINVAL;
+    if (d->options & (SYN_ATTN_CHAIN_Q_BLOCKS | SYN_ATTN_WORK_LIST | SYN_ATTN_SPLIT_KV | SYN_ATTN_SPLIT_DEAL)) return SYN_EINVAL;
     if (d->work_list != nullptr) return SYN_EINVAL;
     int grid = d->num_programs > 0 ? d->num_programs : (int)tiles;
     if (grid > tiles) grid = (int)tiles;

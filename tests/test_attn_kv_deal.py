@@ -1,0 +1,104 @@
+"""Pairs of q blocks whose kv blocks are dealt to several programs one by one (SYN_ATTN_SPLIT_DEAL): the plan of tables that
+wait for flags (host), and launches at the sizes where the deal goes round differently."""
+
+import pytest
+import torch
+
+from oracle import numerics
+from syncopate_amd.computation.attn.kv_split import BLOCK, KvSplit, plan_kv_deal
+
+
+def _tables(Z, H, Sq, lengths, signals):
+    offsets, sizes, cums, lo = [], [], [], 0
+    for i, n in enumerate(lengths):
+        offsets.append([0, 0, 0, lo])
+        sizes.append([Z, H, Sq, n])
+        cums.append((i + 1) * Z * H * Sq)
+        lo += n
+    return offsets, sizes, cums, signals
+
+
+def test_plans_of_tables_that_wait():
+    plan = lambda Z, H, Sq, lengths, signals: plan_kv_deal(*_tables(Z, H, Sq, lengths, signals), units=256)
+    gated = lambda waves: [-1] + list(range(waves - 1))
+    # the last chunk's blocks are shared by seven parts; 32 units stay free for the kernels that raise the flags
+    assert plan(1, 8, 1024, [1024] * 8, gated(8)) == KvSplit(True, 32, 7, 10)
+    for heads in range(1, 66):
+        for sq in (256, 1024, 3072):
+            got = plan(1, heads, sq, [1024] * 8, gated(8))
+            assert got is None or (got.programs <= 224 and got.chain)
+    # short launches, which the host bounds; enough tiles to fill the device; q blocks that do not pair up or differ
+    assert plan(1, 2, 512, [128] * 2, gated(2)) is None
+    assert plan(1, 32, 4096, [4096] * 8, gated(8)) is None
+    assert plan(1, 8, 1152, [1024] * 8, gated(8)) is None
+    assert plan_kv_deal([[0, 0, 0, 0], [0, 0, 256, 0]], [[1, 2, 256, 4096]] * 2, [512, 1024], [-1, 0], units=256) is None
+    assert plan_kv_deal([[0, 0, 0, 0]], [[1, 1, 256, 128]], [0], [-1], units=256) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["bhsd", "bshd"])
+@pytest.mark.parametrize("Z,H,Sq,lengths,parts", [
+    (1, 1, 256, [128], 3),                       # fewer blocks than parts: two parts of nothing
+    (1, 3, 256, [128 * 5, 128, 128 * 9], 4),     # waves that some parts have no block of
+    (2, 1, 512, [128] * 70, 16),                 # more waves than are looked at at a time
+    (1, 9, 1024, [128 * 3] * 4, 7),              # programs dealt to the XCDs unevenly
+    (1, 75, 1024, [128, 256], 2),                # more programs than compute units
+])
+def test_dealt_blocks_add_up(hip, monkeypatch, Z, H, Sq, lengths, parts, layout):
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.attn import attention_forward
+
+    waves, Skv = len(lengths), sum(lengths)
+    # every other wave is behind a flag, and the table ends in a row of padding
+    offsets, sizes, cums, _ = _tables(Z, H, Sq, lengths, None)
+    signals = [i if i % 2 else -1 for i in range(waves)]
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(Z, H, s, 128, generator=g).bfloat16() for s in (Sq, Skv, Skv))
+    lay = lambda t: t if layout == "bhsd" else t.permute(0, 2, 1, 3).contiguous()
+    monkeypatch.setattr("syncopate_amd.computation.attn.template.plan_kv_split",
+                        lambda *args, **kwargs: KvSplit(True, Z * H * Sq // 256, parts, -(-Skv // (BLOCK * parts))))
+    flags = torch.ones(waves, dtype=torch.int64, device="cuda")
+    o, lse = attention_forward(lay(q).cuda(), lay(k).cuda(), lay(v).cuda(), 128 ** -0.5, wave_offsets=offsets + [[0] * 4],
+                               wave_sizes=sizes + [[0] * 4], cum_wave_sizes=cums + [0], signal_offsets=signals + [0],
+                               signal_ptr=flags, cum_tiles=cums[-1], layout=layout, return_lse=True)
+    check_status()
+    want = numerics.sdpa_fp32(q, k, v, 128 ** -0.5)
+    # one rounding of the result and one of the probabilities, 2^-9 each, relative to the largest value; three times that
+    assert ((o if layout == "bhsd" else o.permute(0, 2, 1, 3)).float().cpu() - want).abs().max() <= \
+        1.2e-2 * want.abs().max()
+    s = (q.float() @ k.float().transpose(-1, -2)) * 128 ** -0.5
+    assert (lse.cpu() - torch.logsumexp(s, dim=-1) / 0.6931471805599453).abs().max().item() <= 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("trusted", [True, False])
+def test_chunks_that_come_late(hip, trusted):
+    """A table that the launcher deals by itself: flags raised one after the other and out of order, by kernels that are
+    launched behind it; the same bits as with every flag up."""
+    from syncopate_amd import _lib
+    from syncopate_amd.communication.comm_runtime.streams import pick_side_streams
+    from syncopate_amd.computation._launch import check_status, compute_units, trust_flags
+    from syncopate_amd.computation.attn import attention_forward
+
+    H, Sq, chunk, chunks = 8, 1024, 1024, 8
+    offsets, sizes, cums, signals = _tables(1, H, Sq, [chunk] * chunks, [-1] + list(range(chunks - 1)))
+    assert plan_kv_deal(offsets, sizes, cums, signals, units=compute_units(0))
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q, k, v = (torch.randn(1, H, s, 128, device="cuda", generator=g).bfloat16() for s in (Sq, chunk * chunks, chunk * chunks))
+    table = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    tables = dict(wave_offsets=table(offsets), wave_sizes=table(sizes), cum_wave_sizes=table(cums), signal_offsets=table(signals),
+                  cum_tiles=cums[-1])
+    flags = torch.ones(chunks, dtype=torch.int64, device="cuda")
+    if trusted:
+        trust_flags(flags)
+    resident = attention_forward(q, k, v, 128 ** -0.5, signal_ptr=flags, **tables)
+    lib, side = _lib.load(), pick_side_streams(1)[0]
+    for first in (0, 3):
+        flags.zero_()
+        torch.cuda.synchronize()
+        o = attention_forward(q, k, v, 128 ** -0.5, signal_ptr=flags, **tables)
+        for i in range(chunks - 1):
+            _lib.check("syn_delay_us", lib.syn_delay_us(20, _lib.stream_handle(side)))
+            _lib.check("syn_flag_set", lib.syn_flag_set(flags.data_ptr() + 8 * ((first + 2 * i) % 7), 1, _lib.stream_handle(side)))
+        check_status()
+        assert torch.equal(o, resident)
