@@ -214,6 +214,8 @@ _SIGNATURES = {
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
 _lib: Optional[ctypes.CDLL] = None
+_native = None
+_NATIVE_CALLS = ("syn_gemm_consumer", "syn_gemm_producer", "syn_gemm_remote_binding", "syn_ring_reduce_strided", "syn_attn_fwd")
 
 
 def load() -> ctypes.CDLL:
@@ -233,6 +235,21 @@ def load() -> ctypes.CDLL:
         fn.argtypes = argtypes
     _lib = lib
     return lib
+
+
+def native():
+    """The extension that launches what the Python launchers have prepared before (csrc/launch.cpp), bound to the library."""
+    global _native
+    if _native is None:
+        lib = load()
+        try:
+            from . import _native as module
+        except ImportError as exc:
+            raise RuntimeError("syncopate_amd/_native.so is missing or does not fit this torch: build it with "
+                               "`python -m syncopate_amd.build`") from exc
+        module.bind(*(ctypes.cast(getattr(lib, name), c_void_p).value for name in _NATIVE_CALLS))
+        _native = module
+    return _native
 
 
 def check(fn: str, code: int) -> None:

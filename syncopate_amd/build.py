@@ -1,6 +1,6 @@
-"""Build libsyncopate_hip.so (gfx950) in-tree with hipcc.
+"""Build libsyncopate_hip.so (gfx950) in-tree with hipcc, and the _native extension with g++.
 
-    python -m syncopate_amd.build            # compile every csrc/*.hip and link
+    python -m syncopate_amd.build            # compile every csrc/*.hip and link; compile csrc/launch.cpp
 
 hipcc cross-compiles for gfx950 without a GPU.  The library is linked without
 an rpath to a ROCm tree: at run time ``syncopate_amd._lib`` imports torch first,
@@ -14,12 +14,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 CSRC = Path(__file__).resolve().parent / "csrc"
 LIB_NAME = "libsyncopate_hip.so"
 LIB_PATH = CSRC / LIB_NAME
+NATIVE_PATH = CSRC.parent / "_native.so"
 ARCH = "gfx950"
 
 # -packed-fp32-ops is off: hipcc must not form v_pk_*_f32 from scalar float code.
@@ -56,8 +58,23 @@ def _run(cmd: list[str]) -> None:
         print(err, file=sys.stderr)
 
 
+def build_native() -> Path:
+    """Compile csrc/launch.cpp, host code against torch's headers, into the extension module syncopate_amd._native."""
+    import torch
+
+    home = Path(torch.__file__).resolve().parent
+    tmp = NATIVE_PATH.with_suffix(".so.tmp")
+    _run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-isystem{home / 'include'}",
+          f"-isystem{home / 'include/torch/csrc/api/include'}", f"-isystem{Path(_hipcc()).resolve().parents[1] / 'include'}",
+          f"-I{sysconfig.get_paths()['include']}", str(CSRC / "launch.cpp"), f"-L{home / 'lib'}", "-ltorch_python", "-ltorch_cpu",
+          "-ltorch", "-lc10", "-lc10_hip", "-lamdhip64", "-o", str(tmp)])
+    os.replace(tmp, NATIVE_PATH)
+    return NATIVE_PATH
+
+
 def build_library(jobs: int = 4, verbose: bool = True) -> Path:
-    """Compile all HIP sources and link the shared library; always recompiles."""
+    """Compile all HIP sources and link the shared library, and the extension beside it; always recompiles."""
     hipcc = _hipcc()
     obj_dir = CSRC / "build"
     obj_dir.mkdir(exist_ok=True)
@@ -73,7 +90,9 @@ def build_library(jobs: int = 4, verbose: bool = True) -> Path:
         return obj
 
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as pool:
+        native = pool.submit(build_native)
         objs = list(pool.map(compile_one, srcs))
+        native.result()
 
     tmp = LIB_PATH.with_suffix(".so.tmp")
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)])

@@ -73,6 +73,17 @@ def _launch(
     wait_signal_offsets: Optional[TableLike] = None,
     mfma_32x32: bool = False,
 ) -> None:
+    steady = None
+    if visit_log is None and counter_buffer is None and wait_signal_buffer is None and wait_signal_offsets is None and k_stagger \
+            and spin_timeout_us == DEFAULT_SPIN_TIMEOUT_US and not (eight_waves or ring_pipe or two_stage or mfma_32x32):
+        # operands and tables of a launch that came this way before: launched without the interpreter
+        steady = (a, b, c, signal_buffer, cur_wave_size, wave_offset, signal_offsets, num_gemm_sms, BLOCK_SIZE_M, BLOCK_SIZE_N,
+                  BLOCK_SIZE_K, GROUP_SIZE_M, cum_tiles, -1 if xcd_remap is None else bool(xcd_remap),
+                  id(choose_kernel_tile), producer, acquire_always(signal_buffer))
+        code = _lib.native().gemm(*steady)
+        if code is not None:
+            _lib.check("syn_gemm_producer" if producer else "syn_gemm_consumer", code)
+            return
     # shape/dtype contract of the reference launchers (template.py:177-185)
     assert a.shape[1] == b.shape[1], "Incompatible dimensions"  # b is [N, K]
     assert a.dtype == b.dtype, "Incompatible dtypes"
@@ -210,6 +221,8 @@ def _launch(
         fn = lib.syn_gemm_producer if producer else lib.syn_gemm_consumer
         name = "syn_gemm_producer" if producer else "syn_gemm_consumer"
         _lib.check(name, fn(ctypes.byref(desc), _lib.stream_handle(stream)))
+    if steady is not None and caller_owned and sizes is cur_wave_size and offsets is wave_offset and signals is signal_offsets:
+        _lib.native().gemm(*steady, bytes(desc), status_words(dev))
 
 
 def gemm_consumer(

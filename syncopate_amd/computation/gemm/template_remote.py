@@ -20,6 +20,7 @@ allocations.  Everything else (tables in elements, B stored [N, K]) is as in ``t
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Optional, Sequence
 
 import torch
@@ -52,6 +53,15 @@ def _check_ranks(name: str, ranks: torch.Tensor, count: int, num_waves: int) -> 
         raise ValueError(f"{name} is shorter than the wave tables")
     if int(host[:num_waves].min()) < 0 or int(host[:num_waves].max()) >= count:
         raise ValueError(f"{name} names a rank outside 0..{count - 1}")
+
+
+@functools.lru_cache(maxsize=64)
+def _no_signals(num_waves: int, device_index: int):
+    """Signal offsets and a flag array for waves that wait for nothing, read by every such launch and written by none (copied
+    from the host, so that they are there for whichever stream launches)."""
+    with torch.inference_mode(False):
+        return (torch.tensor([-1] * num_waves, dtype=torch.int32, device=torch.device("cuda", device_index)),
+                torch.tensor([0], dtype=torch.int64, device=torch.device("cuda", device_index)))
 
 
 @launches_on_stream
@@ -154,6 +164,17 @@ def gemm_remote(
     """
     a_list = list(a) if isinstance(a, (list, tuple)) else None
     c_list = list(c) if isinstance(c, (list, tuple)) else None
+    steady = None
+    if a_list is None and c_list is not None and a_target_rank is None and k_ranges is None and signal_ptr is None \
+            and signal_offsets is None and visit_log is None and not eight_waves:
+        # operands and tables of a launch that came this way before: launched without the interpreter
+        steady = (a, b, c_list, cur_wave_sizes, wave_offsets, target_rank, dst_offsets, num_gemm_sms, BLOCK_SIZE_M, BLOCK_SIZE_N,
+                  BLOCK_SIZE_K, GROUP_SIZE_M, cum_tiles, bool(xcd_remap), M, bool(atomic_add),
+                  id(choose_kernel_tile))
+        code = _lib.native().remote(*steady)
+        if code is not None:
+            _lib.check("syn_gemm_remote_binding", code)
+            return
     if a_list is None and c_list is None:
         raise ValueError("neither a nor c is bound to peers: use gemm / gemm_consumer")
     first_a = a_list[0] if a_list is not None else a
@@ -179,8 +200,9 @@ def gemm_remote(
     if offsets.shape[0] != num_waves:
         raise ValueError("wave size and offset tables disagree on the number of waves")
     if signal_offsets is None:
-        signals = torch.full((num_waves,), -1, dtype=torch.int32, device=dev)
-        flags = torch.zeros((1,), dtype=torch.int64, device=dev) if signal_ptr is None else signal_ptr
+        signals, flags = _no_signals(num_waves, dev.index)
+        if signal_ptr is not None:
+            flags = signal_ptr
     else:
         if signal_ptr is None:
             raise ValueError("signal_offsets without signal_ptr")
@@ -238,6 +260,9 @@ def gemm_remote(
     with device_scope(dev):
         _lib.check("syn_gemm_remote_binding",
                    lib.syn_gemm_remote_binding(ctypes.byref(desc), ctypes.byref(remote), _lib.stream_handle(stream)))
+    if steady is not None and caller_owned and sizes is cur_wave_sizes and offsets is wave_offsets:
+        _lib.native().remote(*steady, bytes(desc), bytes(remote), status_words(dev),
+                             [signals, flags] + [t for t in keep if t is not target_rank and t is not dst_offsets])
     del keep, prepared
 
 

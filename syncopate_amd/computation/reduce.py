@@ -35,6 +35,11 @@ def ring_reduce(
     tensors computes (tests/test_gemm_rs.py:64-70); "fp32" rounds once at the end.
     `num_sms` is accepted for call compatibility: the launch always spans the chip.
     """
+    if acc_mode in ACC_MODES:
+        code = _lib.native().reduce(input, output, local_output, begin_idx, ACC_MODES[acc_mode])
+        if code is not None:
+            _lib.check("syn_ring_reduce_strided", code)
+            return output
     if input.dim() != 3:
         raise ValueError("input must be [num_splits, M_per_split, N]")
     num_splits, m_per_split, n = input.shape

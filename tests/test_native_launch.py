@@ -1,0 +1,196 @@
+"""The native steady-state launches (csrc/launch.cpp): taken for operands and tables that came through a launcher before, left to
+the launcher's general path for everything else."""
+
+import threading
+
+import pytest
+import torch
+
+from syncopate_amd import _lib
+
+
+def _table(rows):
+    return torch.tensor(rows, dtype=torch.int32, device="cuda")
+
+
+def test_everything_unusual_is_left_alone():
+    native = _lib.native()
+    host = torch.zeros(2, 4, 8, dtype=torch.bfloat16)
+    assert native.reduce(host, host[0], host.view(8, 8), 0, 0) is None            # not in device memory
+    assert native.reduce(None, 1, "x", 0, 0) is None and native.reduce() is None
+    assert native.gemm(*[host[0]] * 7, *[0] * 10) is None and native.gemm(host) is None
+    assert native.remote(host[0], host[0], [host[0]], *[host[0]] * 4, *[0] * 10) is None
+    assert native.attention(*[host] * 3, 0.1, *[host] * 5, *[0] * 5, None, None, 0, 0) is None
+
+
+def _gemm_case(form):
+    from syncopate_amd.computation.gemm import gemm_consumer, gemm_producer, gemm_rs_producer_persistent, template, template_remote
+
+    world, rows, n, k = 2, 256, 512, 192
+    m = world * rows
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a, b = ((0.1 * torch.randn(s, k, device="cuda", generator=g)).bfloat16() for s in (m, n))
+    sizes, offsets, signals = _table([[rows, n]] * world), _table([[rows, 0], [0, 0]]), _table([1, 0])
+    flags = torch.zeros(world, dtype=torch.int64, device="cuda")
+    c = torch.zeros(m, n, dtype=torch.bfloat16, device="cuda")
+
+    def run(sizes=sizes, a=a, n=n):
+        c.zero_()
+        flags.fill_(form == "consumer")
+        if form == "direct":
+            gemm_rs_producer_persistent(a, b, list(c.view(world, rows, n)), sizes, offsets, signals, world, world, 64, 128, 128, 64, 8)
+        elif form == "producer":
+            gemm_producer(a, b, c, flags, sizes, offsets, signals, 64, 128, 128, 64, 8, cum_tiles=m * n)
+            assert flags.tolist() == [1] * world
+        else:
+            gemm_consumer(a, b, c, flags, sizes, offsets, signals, world, 64, 128, 128, 64, 8, cum_tiles=m * n)
+        return c.clone()
+
+    want = a.float() @ b.float().T
+    if form == "direct":                       # wave 0 (the second half) goes to rank 1, wave 1 to rank 0: in place
+        want = want.view(world, rows, n).reshape(m, n)
+    return run, want, sizes, a, template_remote if form == "direct" else template
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["consumer", "producer", "direct"])
+def test_gemm_second_launch(hip, monkeypatch, form):
+    from syncopate_amd.computation._launch import check_status
+
+    run, want, sizes, a, module = _gemm_case(form)
+    first = run()
+    check_status()
+    # one rounding of the result (2^-9 relative), sums in 32 bits
+    assert (first.float() - want).abs().max() <= 4e-3 * want.abs().max()
+    general, convert = [], module.as_device_table
+    monkeypatch.setattr(module, "as_device_table", lambda *args: general.append(1) or convert(*args))
+    for _ in range(40):                        # the pool of counters is filled again on the way
+        again = run()
+    check_status()
+    assert torch.equal(again, first) and not general
+    # a write into a table: read and checked again, and refused if it does not fit any more
+    sizes.add_(0)
+    assert torch.equal(run(), first) and general
+    general.clear()
+    assert torch.equal(run(), first) and not general
+    # a subclass, an operand elsewhere, other tables with the same contents, a table that no longer fits
+    assert torch.equal(run(a=torch.nn.Parameter(a, requires_grad=False)), first) and not general
+    assert torch.equal(run(a=torch.cat([a, a])[:len(a)]), first) and not general
+    assert torch.equal(run(sizes=sizes.clone()), first) and general
+    with pytest.raises(Exception):
+        run(a=a.cpu())
+    sizes[0, 0] = 64
+    with pytest.raises(_lib.SyncopateHipError):
+        run()
+
+
+@pytest.mark.gpu
+def test_threads_and_streams(hip):
+    """Producers of two threads on streams of their own, more launches than a pool of counters has areas."""
+    from syncopate_amd.computation._launch import check_status
+
+    failed = []
+
+    def work():
+        try:
+            stream = torch.cuda.Stream()
+            stream.wait_stream(torch.cuda.default_stream())
+            with torch.cuda.stream(stream):
+                run, want, *_ = _gemm_case("producer")
+                for _ in range(50):
+                    assert (run().float() - want).abs().max() <= 4e-3 * want.abs().max()
+            stream.synchronize()
+        except BaseException as exc:                                    # noqa: BLE001
+            failed.append(exc)
+
+    threads = [threading.Thread(target=work) for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    check_status()
+    assert not failed, failed
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["bhsd", "bshd"])
+@pytest.mark.parametrize("form", ["explicit", "auto", "causal auto", "producer"])
+def test_attention_second_launch(hip, monkeypatch, form, layout):
+    from oracle import numerics
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.attn import attention_forward, template
+
+    H, S, waves = 2, 512, 2
+    causal, producer = form == "causal auto", form == "producer"
+    g = torch.Generator().manual_seed(1)
+    q, k, v = (torch.randn(1, H, S, 128, generator=g).half() for _ in range(3))
+    lay = (lambda t: t.cuda()) if layout == "bhsd" else (lambda t: t.permute(0, 2, 1, 3).contiguous().cuda())
+    qd, kd, vd = lay(q), lay(k), lay(v)
+    split_q = producer
+    offsets = _table([[0, 0, i * 256 if split_q else 0, 0 if split_q else i * 256] for i in range(waves)])
+    sizes = _table([[1, H, 256 if split_q else S, S if split_q else 256]] * waves)
+    rows = H * (256 if split_q else S)
+    cums, signals = _table([rows, 2 * rows]), _table([0, 1])
+    flags = torch.ones(waves, dtype=torch.int64, device="cuda")
+    counters = torch.zeros(waves, dtype=torch.int32, device="cuda") if producer else None
+
+    def run(scale=0.1, **kw):
+        if producer:
+            flags.zero_()
+            counters.zero_()
+        got = attention_forward(qd, kd, vd, scale, wave_offsets=offsets, wave_sizes=sizes, cum_wave_sizes=cums,
+                                signal_ptr=flags, signal_offsets=signals, NUM_WAVES=waves, cum_tiles=2 * rows, causal=causal,
+                                layout=layout, counter_ptr=counters, form="auto" if "auto" in form else "explicit", **kw)
+        check_status()
+        assert flags.tolist() == [1] * waves and (not producer or counters.tolist() == [rows // 128] * waves)
+        return got
+
+    def near(out, scale=0.1):
+        out = (out if layout == "bhsd" else out.permute(0, 2, 1, 3)).float().cpu()
+        want = numerics.sdpa_fp32(q, k, v, scale, causal=causal)
+        # roundings of the result, of the probabilities and of a merged result, 2^-12 each relative to the largest; four times that
+        return (out - want).abs().max() <= 4e-3 * want.abs().max()
+
+    first, lse = run(return_lse=True)
+    assert near(first) and near(run())         # without and with lse are two things to remember
+    general, convert = [], template.as_device_table
+    monkeypatch.setattr(template, "as_device_table", lambda *args: general.append(1) or convert(*args))
+    for _ in range(20):
+        assert near(run())
+    assert near(run(0.3), 0.3)
+    out = torch.full_like(qd, float("nan"))
+    assert run(out=out) is out and near(out)
+    again, lse2 = run(return_lse=True)
+    assert near(again) and (lse2 - lse).abs().max() <= 1e-4 and not general
+    sizes.add_(0)
+    assert near(run()) and general
+    general.clear()
+    with pytest.raises(ValueError):
+        run(out=torch.empty(1, H, S, 64, device="cuda", dtype=torch.half))
+    sizes[0, 2] = 192
+    with pytest.raises(Exception):
+        run()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("acc_mode", ["dtype", "fp32"])
+def test_reduce_is_launched_or_refused(hip, monkeypatch, acc_mode):
+    from syncopate_amd.computation import reduce as module
+
+    g = torch.Generator(device="cuda").manual_seed(1)
+    received, local = (torch.randn(s, device="cuda", generator=g).half() for s in ((3, 40, 64), (120, 64)))
+    out = torch.empty(40, 64, dtype=torch.half, device="cuda")
+    seen, ask = [], module.require_cuda
+    monkeypatch.setattr(module, "require_cuda", lambda *args: seen.append(1) or ask(*args))
+    assert module.ring_reduce(received, out, local, 1, acc_mode=acc_mode) is out and not seen
+    want = local[40:80].float()
+    for i in (2, 0):
+        want = want + received[i].float()
+        want = want.half().float() if acc_mode == "dtype" else want
+    assert torch.equal(out, want.half())
+    with pytest.raises(ValueError):
+        module.ring_reduce(received, out, local.t().contiguous().t(), 1, acc_mode=acc_mode)
+    with pytest.raises(TypeError):
+        module.ring_reduce(received, out, local.float(), 1, acc_mode=acc_mode)
+    with pytest.raises(_lib.SyncopateHipError):
+        module.ring_reduce(received, out, local, 3, acc_mode=acc_mode)
