@@ -11,18 +11,17 @@
 //
 // Pipelines over the same tile walk (the 64 fills of a 256x256 slab take the texture path of a
 // compute unit about 1400 cycles, a k16 step of MFMAs 512: where the fills are issued matters):
-//   early  2 stages of 64-deep slabs, the LDS reads of a slab bunched at its start so that its
-//          stage is refilled during three quarters of the slab's MFMAs; the default for the tiles of
-//          which only two stages fit the 160 KB of LDS (256x256, 256x224), on 16x16x32 MFMAs
-//          (which cost less energy per product on a power-limited board; same bits) or, as an
-//          option, on 32x32x16 ones.
-//   slab   3 stages of 64-deep slabs, a slab's fills spread over the four k16 steps; the default
-//          for the other tiles.  With 2 stages (an option) all fills go out in one step.
-//          Rows are whole 128-byte cache lines; any K % 64 == 0.
+//   roll   the default, on 16x16x32 MFMAs (which cost less energy per product on a power-limited board;
+//          same bits): 64-deep slabs in 3 stages, or in 2 for the tiles of which only two fit the 160 KB
+//          of LDS (256x256, 256x224), their fills spread over the slab's MFMAs, and no break between
+//          a program's tiles.  Rows are whole 128-byte cache lines; any K % 64 == 0.
+//   early, slab   (options) 2 and 3 stages on 32x32x16 MFMAs, tile by tile: early bunches the LDS reads of a
+//          slab at its start so that its stage is refilled during three quarters of its MFMAs, slab spreads the
+//          fills over the four k16 steps; with 2 stages (an option) all its fills go out in one step.
 //   ring   4 stages of 32-deep slabs, three in flight; rows are half cache lines, which costs
 //          L1 fill bandwidth.  Needs K % 128 == 0.
-// A tile's first fills are issued before the previous tile's C is stored; C leaves through a
-// per-wavefront LDS strip as whole cache lines.
+// A tile's first fills are issued before the previous tile's C is stored (roll: in its K loop); C leaves
+// through a per-wavefront LDS strip as whole cache lines.
 //
 // Consumer form: before the first tile of a wave whose signal offset is >= 0 lane 0 spins on
 // the flag word, then the whole workgroup takes an acquire fence (template.py:121-128).
@@ -109,7 +108,7 @@ struct Mfma16<__bf16> {
     //    eight MFMAs (128 cycles) apart, and always as the same whole tuple;
     //  - MFMA result -> vector ALU read or overwrite: a matrix op of N passes needs N + 3 wait states before a
     //    vector instruction may read or write its result registers (7 for the four passes of 16x16x32, 11 for
-    //    eight, 19 for sixteen).  Every K loop ends in mfma_result_wait_states() below, which idles 24 - more
+    //    eight, 19 for sixteen).  Every K loop ends in mfma_result_wait_states below, which idles 24 - more
     //    than the longest form needs - before the epilogue reads the accumulators and before the next tile's
     //    zeros are written.
     static __device__ __forceinline__ void run(bf16x8_t a, bf16x8_t b, f32x4_t& c) {
@@ -125,9 +124,17 @@ struct Mfma16<_Float16> {
 };
 
 // Wait states between the last assembly MFMA of a K loop and the first vector instruction that touches an
-// accumulator (see Mfma16): 16 + 8 idle issue slots, once per tile.
-__device__ __forceinline__ void mfma_result_wait_states() {
+// accumulator (see Mfma16): 16 + 8 idle issue slots, once per tile.  Every accumulator passes through a statement that comes
+// behind them: as a statement of its own the compiler moved copies of the accumulators in front of it.
+template <int R, int C>
+__device__ __forceinline__ void mfma_result_wait_states(f32x4_t (&acc)[R][C]) {
+    static_assert(R * C % 8 == 0, "eight accumulators at a time");
     asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+    f32x4_t* const x = &acc[0][0];
+#pragma unroll
+    for (int i = 0; i < R * C; i += 8)
+        asm volatile("" : "+a"(x[i]), "+a"(x[i + 1]), "+a"(x[i + 2]), "+a"(x[i + 3]), "+a"(x[i + 4]), "+a"(x[i + 5]), "+a"(x[i + 6]),
+                          "+a"(x[i + 7]));
 }
 
 template <typename T>
@@ -139,6 +146,15 @@ __device__ __forceinline__ uint2 pack4(float x0, float x1, float x2, float x3) {
     v[2] = (T)x2;
     v[3] = (T)x3;
     return __builtin_bit_cast(uint2, v);
+}
+
+// the value of a variable that is the same in every lane, as a scalar (what comes from tables in LDS is not one for the compiler)
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ const unsigned char* uniform(const unsigned char* ptr) {
+    const uint64_t bits = reinterpret_cast<uint64_t>(ptr);
+    const uint64_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)bits);
+    const uint64_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(bits >> 32));
+    return reinterpret_cast<const unsigned char*>(lo | hi << 32);
 }
 
 typedef __attribute__((address_space(3))) void* lds_void_ptr;
@@ -317,7 +333,7 @@ struct SlabPipe {
     static constexpr int LDS_BYTES = NST * STAGE;
     static constexpr int FILLS = (BM + BN) / (8 * NW);
     static constexpr int K_ALIGN = 64;
-    static constexpr bool kMfma16 = false;
+    static constexpr bool kMfma16 = false, kRolls = false;
     typedef typename Mfma32<T>::frag_t frag_t;
 
     static constexpr int NV = (BM > BN ? BM : BN) / (8 * NW);    // fills per wavefront and operand
@@ -591,18 +607,22 @@ struct EarlyPipe : SlabPipe<T, BM, BN, WGM, WGN, 2> {
     }
 };
 
-// early16: the early-read pipeline on 16x16x32 MFMAs.  A wavefront's 128 x 128 part of the tile is 8 x 8 accumulators
-// of 16 x 16; a slab is two k32 steps of 64 MFMAs, run as four quarters of 32 (row blocks 0-3 or 4-7 of A against all
-// eight column blocks).  A k32 step needs eight fragments of A and eight of B (one 128-bit LDS read each, lane l:
-// row l % 16, 16-byte chunk l / 16 of the step's four), so the fragments of both steps are again 128 VGPRs:
-//     quarter 3 of slab s-1: MFMAs | read the fragments of k32 step 0 of slab s
-//     quarter 0: MFMAs | read the fragments of step 1;  wait for them;  barrier: the stage is free
-//     quarter 1: MFMAs | first third of the fills of slab s+2 into that stage
-//     quarter 2: MFMAs | second third;  wait: own fills of slab s+1 landed;  barrier
-//     quarter 3: MFMAs | last third | read step 0 of slab s+1
-template <typename T, int BM, int BN, int WGM, int WGN>
-struct EarlyPipe16 : SlabPipe<T, BM, BN, WGM, WGN, 2> {
-    typedef SlabPipe<T, BM, BN, WGM, WGN, 2> Base;
+// roll: the default pipelines, on 16x16x32 MFMAs, over all tiles of a program without a break.  A wavefront's part of the tile is
+// RM x RN accumulators of 16 x 16; a slab is two k32 steps, run as four quarters (half of the row blocks of A against all column
+// blocks of B).  A k32 step needs RM fragments of A and RN of B (one 128-bit LDS read each, lane l: row l % 16, 16-byte chunk
+// l / 16 of the step's four); those of the next step are read beside the products of the first half of a step.  With two
+// stages (the tiles of which three do not fit) the reads of a slab are done after its first quarter and its stage is
+// refilled during the other three; with three the fills of a slab go out in four parts and two slabs are in flight (see main).
+// The slabs behind a tile's last one are the next tile's first ones, and the stages are taken in turn whatever the number of
+// slabs.  The form before it kept a stage per unrolled slab, fetched the last slab again past the end, drained, and
+// issued the next tile's first 27 fills per wavefront with the matrix pipes idle: 2 to 3 us a tile.  Measured on one box, M and N
+// for full rounds of 256 programs: 128x256 tiles, K = 512, 2 and 4 rounds 26.1 -> 22.5 and 48.4 -> 38.7 us, K = 2048 60.4 -> 57.0
+// and 115 -> 107; 256x256, 2 rounds of K = 2048 106.6 -> 103.6; one round the same to 1.5 %.  128x128, which ran on
+// 32x32x16 MFMAs with a k16 step (128 cycles) of look-ahead for its LDS reads: one round of K = 4096 36.2 -> 32.6, four 140.8 -> 118.8.
+// With power no limit (zeros) a 128x256 slab takes 1190 cycles for 1030 of MFMAs, with random operands 1.53 PFLOP/s.
+template <typename T, int BM, int BN, int WGM, int WGN, int NST_>
+struct RollPipe : SlabPipe<T, BM, BN, WGM, WGN, NST_> {
+    typedef SlabPipe<T, BM, BN, WGM, WGN, NST_> Base;
     using Base::TM;
     using Base::TN;
     using Base::ROW;
@@ -613,9 +633,11 @@ struct EarlyPipe16 : SlabPipe<T, BM, BN, WGM, WGN, 2> {
     using Base::WM;
     using Base::WN;
     using Base::A_BYTES;
+    using Base::STAGE;
     typedef typename Base::frag_t frag_t;
     typedef typename Base::Lane Lane;
-    static constexpr bool kMfma16 = true;
+    static constexpr bool kMfma16 = true, kRolls = true;
+    static constexpr int NST = NST_, kChainSlabs = 3;
     static constexpr int RM = 2 * TM, RN = 2 * TN;          // 16-row blocks of A and of B per wavefront
     static constexpr int PA = (FILLS + 2) / 3, PB = (FILLS - PA + 1) / 2, PC = FILLS - PA - PB;
     static_assert(RM % 2 == 0, "two quarters of row blocks");
@@ -664,165 +686,186 @@ struct EarlyPipe16 : SlabPipe<T, BM, BN, WGM, WGN, 2> {
             }
     }
 
-    // fill f of `count` goes out after MFMA g of Q when f * Q / count == g
-    template <int FIRST, int COUNT>
-    static __device__ __forceinline__ void fill_slot(int g, int q, unsigned char* dst, const unsigned char* a_k,
-                                                     const unsigned char* b_k, const Lane& ln) {
-#pragma unroll
-        for (int f = 0; f < COUNT; ++f)
-            if (f * q / COUNT == g) dma_one<BM, NW, NV>(FIRST + f, dst, a_k, b_k, ln.voff);
+    // Where a tile's slabs come from: the first rows of its panels, the number of slabs, and the one it begins with.
+    struct Source {
+        const unsigned char *a, *b;
+        int slabs, rot;
+    };
+    static __device__ __forceinline__ Source source(const unsigned char* a_panel, const unsigned char* b_panel, int K, int k_rot) {
+        const int slabs = uniform(K / BK), rot = uniform(k_rot);
+        return Source{uniform(a_panel), uniform(b_panel), slabs, rot < slabs ? rot : rot % slabs};
+    }
+    // The slabs of a tile one after the other, from slab `rot` on and around, and behind the last one those of the next tile, or
+    // the last one again.  `left` slabs are to come before something other than the next address comes.
+    struct Stream {
+        const unsigned char *a, *b;
+        int left, turn;              // turn: 0 before the end of K, 1 behind it, 2 the next tile's, 3 the last slab again
+    };
+    static __device__ __forceinline__ Stream begin(const Source& t) {
+        return Stream{t.a + (size_t)t.rot * ROW, t.b + (size_t)t.rot * ROW, t.slabs - t.rot, 0};
+    }
+    static __device__ __forceinline__ void step(Stream& at, const Source& t, const Source& next, bool chained) {
+        at.a += ROW;
+        at.b += ROW;
+        if (__builtin_expect(--at.left == 0, 0)) {
+            if (at.turn == 0 && t.rot != 0) {
+                at = Stream{t.a, t.b, t.rot, 1};
+            } else if (at.turn <= 1 && chained) {
+                at = begin(next);
+                at.turn = 2;
+            } else if (at.turn != 2) {
+                at = Stream{at.a - ROW, at.b - ROW, 1, 3};
+            } else {
+                at = Stream{next.a, next.b, next.rot, 2};
+            }
+        }
     }
 
-    static __device__ __forceinline__ void slab(f32x4_t (&acc)[RM][RN], frag_t (&fa)[2][RM], frag_t (&fb)[2][RN],
-                                                unsigned char* cur, const unsigned char* nxt,
-                                                const unsigned char* a_slab, const unsigned char* b_slab,
-                                                size_t k_refill, const Lane& ln, const Lane16& l16, int wave) {
+    // the stream that went on into tile `t` is this tile's own now
+    static __device__ __forceinline__ void enter(Stream& at, const Source& t) { at.turn = at.a - t.a >= (ptrdiff_t)((size_t)t.rot * ROW) ? 0 : 1; }
+
+    // the stages, one behind the other: which of them a slab lives in is counted at run time
+    static __device__ __forceinline__ unsigned char* stages() {
+        __shared__ __attribute__((aligned(1024))) unsigned char st[NST * STAGE];
+        return st;
+    }
+    static __device__ __forceinline__ int behind(int stage) { return stage + 1 == NST ? 0 : stage + 1; }
+
+    // Fill j of the wavefront, 16 bytes per lane from a uniform base and a 32-bit lane offset, as assembly: told of a load into
+    // LDS, the compiler would make LDS reads of the other stages wait for it, which it cannot tell from this one any more.
+    // The waits for fills are this pipeline's own.  In two statements, of which the first says where in LDS: an instruction has to
+    // stand between them, and in the K loop an MFMA does.
+    static __device__ __forceinline__ void fill_to(int j, unsigned stage_wave) {
+        asm volatile("s_add_u32 m0, %0, %1" : : "s"(stage_wave), "n"(j * NW * 1024) : "m0", "scc");
+    }
+    static __device__ __forceinline__ void fill_from(int j, const unsigned char* a, const unsigned char* b, const Lane& ln) {
+        constexpr int kAFills = BM / (8 * NW);
+        asm volatile("global_load_lds_dwordx4 %0, %1"
+                     :
+                     : "v"(j < kAFills ? ln.voff[j] : ln.voff[j - kAFills]), "s"(j < kAFills ? a : b)
+                     : "memory");
+    }
+    static __device__ __forceinline__ unsigned stage_wave(int stage, int wave) {
+        return (unsigned)(uintptr_t)(lds_void_ptr)stages() + (unsigned)(stage * STAGE + wave * 1024);
+    }
+    template <int FIRST, int LAST>
+    static __device__ __forceinline__ void fill_range(unsigned dst, const Stream& from, const Lane& ln) {
+#pragma unroll
+        for (int j = FIRST; j < LAST; ++j) {
+            fill_to(j, dst);
+            asm volatile("s_nop 0");
+            fill_from(j, from.a, from.b, ln);
+        }
+    }
+    // fills FIRST .. FIRST + COUNT beside q MFMAs: fill f of them goes out after MFMA f * q / COUNT + 1
+    template <int FIRST, int COUNT>
+    static __device__ __forceinline__ void fill_slot(int g, int q, unsigned dst, const Stream& from, const Lane& ln) {
+        static_assert(COUNT == 0 || (RM * RN / 2) / COUNT >= 2, "an MFMA between a fill's two statements");
+#pragma unroll
+        for (int f = 0; f < COUNT; ++f) {
+            if (f * q / COUNT == g) fill_to(FIRST + f, dst);
+            if (f * q / COUNT + 1 == g) fill_from(FIRST + f, from.a, from.b, ln);
+        }
+    }
+
+    // The parts of a slab's fills and the quarter they go out in.  Two stages: the thirds of slab s+2 in quarters 1, 2, 3 of slab s.
+    // Three: part 0 of slab s+3 in quarter 3 of slab s, parts 1-3 in quarters 0-2 of slab s+1.
+    static constexpr int part_begin(int q) { return NST == 3 ? FILLS * q / 4 : q == 0 ? 0 : (q == 1 ? PA : q == 2 ? PA + PB : FILLS); }
+    template <int P>
+    static constexpr int part_size() { return part_begin(P + 1) - part_begin(P); }
+
+    // Issue the fills that are under way when a tile begins: its first two slabs, and with three stages part 0 of the third.
+    // Returns the stream at the slab to be fetched next (of which part 0 is under way with three stages).
+    static __device__ __forceinline__ Stream prologue(const Source& t, int stage, size_t row_bytes, int lane, int wave) {
+        const Lane ln = Base::make_lane(row_bytes, lane, wave);
+        const int next = behind(stage);
+        Stream at = begin(t);
+        fill_range<0, FILLS>(stage_wave(stage, wave), at, ln);
+        step(at, t, t, false);
+        fill_range<0, FILLS>(stage_wave(next, wave), at, ln);
+        step(at, t, t, false);
+        if constexpr (NST == 3) fill_range<0, part_begin(1)>(stage_wave(behind(next), wave), at, ln);
+        return at;
+    }
+
+    // The K loop of a tile.  `stage` is the one of its first slab, on return the one of the slab behind its last.  `chained`: the
+    // slabs behind the last are `next`'s first ones - its prologue, issued here, where they take the place of fetching the
+    // last slab again, and nothing is waited for at the end; fa[0], fb[0] then hold the fragments of its first step, and
+    // `primed` says so to the next call.  Else every fill has landed and every wavefront has passed a barrier on return.
+    // (Both tiles have at least kChainSlabs slabs then: `at` stands at a tile's third slab when the tile begins.)
+    static __device__ __forceinline__ void main(f32x4_t (&acc)[RM][RN], frag_t (&fa)[2][RM], frag_t (&fb)[2][RN], int& stage,
+                                                Stream& at, const Source& t, const Source& next, bool chained, bool primed,
+                                                size_t row_bytes, int lane, int wave) {
         constexpr int Q = RM * RN / 2;                         // MFMAs of a quarter
         static_assert(RM + RN <= Q, "a fragment read per MFMA");
-        const unsigned char* a_k = a_slab + k_refill;
-        const unsigned char* b_k = b_slab + k_refill;
-        unsigned char* const dst = cur + wave * 1024;
-
-        quarter<0>(acc, fa[0], fb[0], [&](int g) { if (g < RM + RN) read_frag<1>(fa[1], fb[1], cur, l16, g); });
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, true));     // own reads of this stage returned
-        __builtin_amdgcn_s_barrier();                          // everyone's: the stage is free
-
-        quarter<1>(acc, fa[0], fb[0], [&](int g) { fill_slot<0, PA>(g, Q, dst, a_k, b_k, ln); });
-        quarter<0>(acc, fa[1], fb[1], [&](int g) { fill_slot<PA, PB>(g, Q, dst, a_k, b_k, ln); });
-        // own fills of slab s+1 landed (the two thirds of slab s+2 issued since may fly on)
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm(PA + PB, false));
-        __builtin_amdgcn_s_barrier();
-
-        quarter<1>(acc, fa[1], fb[1], [&](int g) {
-            if (g < RM + RN) read_frag<0>(fa[0], fb[0], nxt, l16, g);
-            fill_slot<PA + PB, PC>(g, Q, dst, a_k, b_k, ln);
-        });
-    }
-
-    static __device__ __forceinline__ void main(f32x4_t (&acc)[RM][RN], const unsigned char* a_slab,
-                                                const unsigned char* b_slab, size_t row_bytes, int K,
-                                                int k_rot, int lane, int wave) {
-        unsigned char* const stage0 = Base::template stage<0>();
-        unsigned char* const stage1 = Base::template stage<1>();
         const Lane ln = Base::make_lane(row_bytes, lane, wave);
         const Lane16 l16 = make_lane16(lane, wave);
-        const int k_steps = K / BK;
-        const int rot = k_rot % k_steps;
-
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm(FILLS, true));       // slab 0 landed; slab 1 may fly on
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        frag_t fa[2][RM], fb[2][RN];
-        read_step<0>(fa[0], fb[0], stage0, l16);
-
-        const int pairs = k_steps >> 1;
-        for (int pr = 0; pr < pairs; ++pr) {
-            slab(acc, fa, fb, stage0, stage1, a_slab, b_slab, Base::slab_off(2 * pr + 2, rot, k_steps), ln, l16, wave);
-            slab(acc, fa, fb, stage1, stage0, a_slab, b_slab, Base::slab_off(2 * pr + 3, rot, k_steps), ln, l16, wave);
+        unsigned char* const st = stages();
+        if (!primed) {
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm(FILLS + (NST == 3 ? part_begin(1) : 0), true));      // slab 0 landed
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("" ::: "memory");
+            read_step<0>(fa[0], fb[0], st + stage * STAGE, l16);
         }
-        if (k_steps & 1)
-            slab(acc, fa, fb, stage0, stage1, a_slab, b_slab, Base::slab_off(k_steps + 1, rot, k_steps), ln, l16, wave);
-        // drain the re-fetches of the last slab before anything refills the stages
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, true));
-        __builtin_amdgcn_s_barrier();
-        mfma_result_wait_states();      // the accumulators are read by vector instructions from here on
-        __builtin_amdgcn_sched_barrier(0);
-    }
-};
-
-// slab16: the three-stage pipeline on 16x16x32 MFMAs, for the tiles of which three stages fit.  The quarters and the
-// fragment reads are those of early16; a slab's fills go out in four parts as in `slab`: part 0 of slab s+3 in quarter 3
-// of slab s (into the stage slab s has left), parts 1-3 in quarters 0-2 of slab s+1; two slabs in flight.
-//     quarter 0: MFMAs (k32 step 0) | read the fragments of step 1 | part 1 of slab s+2
-//     quarter 1: MFMAs (step 0)     | part 2
-//     quarter 2: MFMAs (step 1)     | part 3;  wait: own fills of slab s+1 landed, own reads returned;  barrier
-//     quarter 3: MFMAs (step 1)     | read step 0 of slab s+1 | part 0 of slab s+3 into this slab's stage
-template <typename T, int BM, int BN, int WGM, int WGN>
-struct SlabPipe16 : SlabPipe<T, BM, BN, WGM, WGN, 3> {
-    typedef SlabPipe<T, BM, BN, WGM, WGN, 3> Base;
-    typedef EarlyPipe16<T, BM, BN, WGM, WGN> Ops;            // fragment reads and quarters
-    using Base::TM;
-    using Base::TN;
-    using Base::FILLS;
-    using Base::NW;
-    using Base::NV;
-    using Base::BK;
-    typedef typename Base::frag_t frag_t;
-    typedef typename Base::Lane Lane;
-    typedef typename Ops::Lane16 Lane16;
-    static constexpr bool kMfma16 = true;
-    static constexpr int RM = 2 * TM, RN = 2 * TN;
-
-    template <int PART>
-    static __device__ __forceinline__ void fill_slot(int g, int q, unsigned char* stage_wave, const unsigned char* a_k,
-                                                     const unsigned char* b_k, const Lane& ln) {
-        constexpr int first = Base::part_begin(PART), count = Base::part_begin(PART + 1) - first;
-#pragma unroll
-        for (int f = 0; f < count; ++f)
-            if (f * q / count == g) dma_one<BM, NW, NV>(first + f, stage_wave, a_k, b_k, ln.voff);
-    }
-
-    static __device__ __forceinline__ void slab(f32x4_t (&acc)[RM][RN], frag_t (&fa)[2][RM], frag_t (&fb)[2][RN],
-                                                unsigned char* cur, const unsigned char* nxt, unsigned char* prv,
-                                                const unsigned char* a_slab, const unsigned char* b_slab,
-                                                size_t k_refill, size_t k_prev, const Lane& ln, const Lane16& l16,
-                                                int wave) {
-        constexpr int Q = RM * RN / 2;                         // MFMAs of a quarter
-        static_assert(RM + RN <= Q, "a fragment read per MFMA");
-        unsigned char* const prv_w = prv + wave * 1024;
-        const unsigned char* a_p = a_slab + k_prev;
-        const unsigned char* b_p = b_slab + k_prev;
-
-        Ops::template quarter<0>(acc, fa[0], fb[0], [&](int g) {
-            if (g < RM + RN) Ops::template read_frag<1>(fa[1], fb[1], cur, l16, g);
-            fill_slot<1>(g, Q, prv_w, a_p, b_p, ln);
-        });
-        Ops::template quarter<1>(acc, fa[0], fb[0], [&](int g) { fill_slot<2>(g, Q, prv_w, a_p, b_p, ln); });
-        Ops::template quarter<0>(acc, fa[1], fb[1], [&](int g) { fill_slot<3>(g, Q, prv_w, a_p, b_p, ln); });
-        // own fills of slab s+1 landed (those of slab s+2, all younger, may fly on)
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm(FILLS, true));
-        __builtin_amdgcn_s_barrier();
-
-        Ops::template quarter<1>(acc, fa[1], fb[1], [&](int g) {
-            if (g < RM + RN) Ops::template read_frag<0>(fa[0], fb[0], nxt, l16, g);
-            fill_slot<0>(g, Q, cur + wave * 1024, a_slab + k_refill, b_slab + k_refill, ln);
-        });
-    }
-
-    static __device__ __forceinline__ void main(f32x4_t (&acc)[RM][RN], const unsigned char* a_slab,
-                                                const unsigned char* b_slab, size_t row_bytes, int K,
-                                                int k_rot, int lane, int wave) {
-        unsigned char* const stage0 = Base::template stage<0>();
-        unsigned char* const stage1 = Base::template stage<1>();
-        unsigned char* const stage2 = Base::template stage<2>();
-        const Lane ln = Base::make_lane(row_bytes, lane, wave);
-        const Lane16 l16 = Ops::make_lane16(lane, wave);
-        const int k_steps = K / BK;
-        const int rot = k_rot % k_steps;
-
-        // slab 0 landed; slab 1 and part 0 of slab 2 may fly on
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm(FILLS + Base::template part_size<0>(), true));
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        frag_t fa[2][RM], fb[2][RN];
-        Ops::template read_step<0>(fa[0], fb[0], stage0, l16);
-
-        auto run = [&](unsigned char* cur, const unsigned char* nxt, unsigned char* prv, int s) {
-            slab(acc, fa, fb, cur, nxt, prv, a_slab, b_slab, Base::slab_off(s + 3, rot, k_steps),
-                 Base::slab_off(s + 2, rot, k_steps), ln, l16, wave);
-        };
-        const int triples = k_steps / 3, rest = k_steps - 3 * triples;
-        for (int tr = 0; tr < triples; ++tr) {
-            run(stage0, stage1, stage2, 3 * tr);
-            run(stage1, stage2, stage0, 3 * tr + 1);
-            run(stage2, stage0, stage1, 3 * tr + 2);
+        // (two wait states between the zeros of the first accumulators and the first MFMAs)
+        asm volatile("s_nop 1" : "+a"(acc[0][0]), "+a"(acc[0][1]), "+a"(acc[0][2]), "+a"(acc[0][3]));
+        int s = 0;
+        do {
+            const int nxt_stage = behind(stage);
+            const unsigned char* const cur = st + stage * STAGE;
+            const unsigned char* const nxt = st + nxt_stage * STAGE;
+            const unsigned cur_w = stage_wave(stage, wave);
+            if constexpr (NST == 2) {
+                //     quarter 0: MFMAs | read the fragments of step 1;  wait for them;  barrier: the stage is free
+                //     quarter 1: MFMAs | first third of the fills of slab s+2 into that stage
+                //     quarter 2: MFMAs | second third;  wait: own fills of slab s+1 landed;  barrier
+                //     quarter 3: MFMAs | last third | read step 0 of slab s+1
+                quarter<0>(acc, fa[0], fb[0], [&](int g) { if (g < RM + RN) read_frag<1>(fa[1], fb[1], cur, l16, g); });
+                __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, true));     // own reads of this stage returned
+                __builtin_amdgcn_s_barrier();                          // everyone's: the stage is free
+                asm volatile("" ::: "memory");
+                quarter<1>(acc, fa[0], fb[0], [&](int g) { fill_slot<0, PA>(g, Q, cur_w, at, ln); });
+                quarter<0>(acc, fa[1], fb[1], [&](int g) { fill_slot<PA, PB>(g, Q, cur_w, at, ln); });
+                // own fills of slab s+1 landed (the two thirds of slab s+2 issued since may fly on)
+                __builtin_amdgcn_s_waitcnt(waitcnt_imm(PA + PB, false));
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                quarter<1>(acc, fa[1], fb[1], [&](int g) {
+                    if (g < RM + RN) read_frag<0>(fa[0], fb[0], nxt, l16, g);
+                    fill_slot<PA + PB, PC>(g, Q, cur_w, at, ln);
+                });
+                step(at, t, next, chained);
+            } else {
+                //     quarter 0: MFMAs (k32 step 0) | read the fragments of step 1 | part 1 of slab s+2
+                //     quarter 1: MFMAs (step 0)     | part 2
+                //     quarter 2: MFMAs (step 1)     | part 3;  wait: own fills of slab s+1 landed, own reads returned;  barrier
+                //     quarter 3: MFMAs (step 1)     | read step 0 of slab s+1 | part 0 of slab s+3 into this slab's stage
+                const unsigned prv_w = stage_wave(behind(nxt_stage), wave);
+                quarter<0>(acc, fa[0], fb[0], [&](int g) {
+                    if (g < RM + RN) read_frag<1>(fa[1], fb[1], cur, l16, g);
+                    fill_slot<part_begin(1), part_size<1>()>(g, Q, prv_w, at, ln);
+                });
+                quarter<1>(acc, fa[0], fb[0], [&](int g) { fill_slot<part_begin(2), part_size<2>()>(g, Q, prv_w, at, ln); });
+                quarter<0>(acc, fa[1], fb[1], [&](int g) { fill_slot<part_begin(3), part_size<3>()>(g, Q, prv_w, at, ln); });
+                // own fills of slab s+1 landed (those of slab s+2, all younger, may fly on)
+                __builtin_amdgcn_s_waitcnt(waitcnt_imm(FILLS, true));
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                step(at, t, next, chained);
+                quarter<1>(acc, fa[1], fb[1], [&](int g) {
+                    if (g < RM + RN) read_frag<0>(fa[0], fb[0], nxt, l16, g);
+                    fill_slot<0, part_size<0>()>(g, Q, cur_w, at, ln);
+                });
+            }
+            stage = nxt_stage;
+        } while (++s < t.slabs);
+        if (!chained) {
+            // drain the re-fetches of the last slab before anything refills the stages
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, true));
+            __builtin_amdgcn_s_barrier();
         }
-        if (rest >= 1) run(stage0, stage1, stage2, 3 * triples);
-        if (rest == 2) run(stage1, stage2, stage0, 3 * triples + 1);
-        // drain the re-fetches of the last slab before anything refills the stages
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, true));
-        __builtin_amdgcn_s_barrier();
-        mfma_result_wait_states();      // the accumulators are read by vector instructions from here on
+        mfma_result_wait_states(acc);      // the accumulators are read by vector instructions from here on
         __builtin_amdgcn_sched_barrier(0);
     }
 };
@@ -832,14 +875,11 @@ struct SlabPipe16 : SlabPipe<T, BM, BN, WGM, WGN, 3> {
 template <typename T, int BM, int BN, int WGM, int WGN,
           bool THREE = (3 * (BM + BN) * 128 + WGM * WGN * 32 * 80 + 4096 <= 160 * 1024)>
 struct DeepPipeSel {
-    // a wavefront part of 64 x 64 (the 128x128 tile) is 2 % faster on 32x32x16 MFMAs: eight MFMAs per quarter
-    // leave no room beside the fragment reads
-    typedef typename std::conditional<(BM / WGM) * (BN / WGN) <= 64 * 64, SlabPipe<T, BM, BN, WGM, WGN, 3>,
-                                      SlabPipe16<T, BM, BN, WGM, WGN>>::type type;
+    typedef RollPipe<T, BM, BN, WGM, WGN, 3> type;
 };
 template <typename T, int BM, int BN, int WGM, int WGN>
 struct DeepPipeSel<T, BM, BN, WGM, WGN, false> {
-    typedef EarlyPipe16<T, BM, BN, WGM, WGN> type;
+    typedef RollPipe<T, BM, BN, WGM, WGN, 2> type;
 };
 template <typename T, int BM, int BN, int WGM, int WGN>
 using DeepPipe = typename DeepPipeSel<T, BM, BN, WGM, WGN>::type;
@@ -870,7 +910,7 @@ using DeepPipe32 = typename DeepPipe32Sel<T, BM, BN, WGM, WGN>::type;
 template <typename T, int BM, int BN, int WGM, int WGN>
 struct RingPipe {
     static constexpr int NW = WGM * WGN;
-    static constexpr bool kMfma16 = false;
+    static constexpr bool kMfma16 = false, kRolls = false;
     static constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
     static constexpr int BK = 32, ROW = BK * 2;
     static constexpr int A_BYTES = BM * ROW, STAGE = (BM + BN) * ROW;
@@ -1008,7 +1048,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
     constexpr int TM = WM / 32, TN = WN / 32;     // 32x32 MFMA tiles per wavefront
 
     __shared__ int s_abort;
-    __shared__ int s_spun;
+    __shared__ int s_spun, s_waves_up;
     // C staging of the epilogue: 32 rows x CS_COLS columns per wavefront, 64 columns where LDS allows
     constexpr int NWAVES = WGM * WGN;
     constexpr int CS_COLS = ((BN / WGN / 32) % 2 == 0 &&
@@ -1039,7 +1079,28 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
         s_waves[w][4] = p.signal_offsets[w];
     }
     if (tid == 0) s_abort = 0;
+    // Which waves need not be waited for.  Flags are read for 64 waves at a time, a lane each - here for the first ones, beside the
+    // table, and whenever a wave has to be waited for - and those in a row that are up are not looked at again: a flag goes up
+    // once per launch, and a program visits the waves in order.  With every chunk there, no program stops at a wave.
+    // Wavefront 0: flag index per wave, -1: none.
+    auto wait_index = [&](int w) -> int {
+        if (w >= p.num_waves) return -1;
+        return PRODUCER ? (p.wait_offsets != nullptr ? p.wait_offsets[w] : -1) : p.signal_offsets[w];
+    };
+    const uint64_t* const wait_on = PRODUCER ? p.wait_flags : p.flags;
+    if (wave == 0) {
+        const int sig = wait_index(lane);
+        const bool up = sig < 0 || __hip_atomic_load(wait_on + sig, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 1ull;
+        const unsigned long long down = ~__builtin_amdgcn_ballot_w64(up), flagged = __builtin_amdgcn_ballot_w64(sig >= 0);
+        if (lane == 0) {
+            const int row = down == 0 ? 64 : (int)__builtin_ctzll(down);
+            s_waves_up = row;
+            s_spun = (flagged & (row == 64 ? ~0ull : (1ull << row) - 1)) != 0;
+        }
+    }
     __syncthreads();
+    int waves_up = uniform(s_waves_up);
+    if (p.acquire_always && uniform(s_spun)) acquire_fence_agent();
 
     // --- wave walk state (uniform across the workgroup) ---
     int cur_wave = -1, past_tiles = 0, cur_tiles = 0;
@@ -1052,11 +1113,11 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
     auto enter_wave = [&](int w) {
         cur_wave = w;
         if (w < kLdsWaves) {
-            cur_m = s_waves[w][0];
-            cur_n = s_waves[w][1];
-            off_m = s_waves[w][2];
-            off_n = s_waves[w][3];
-            cur_sig = s_waves[w][4];
+            cur_m = uniform(s_waves[w][0]);
+            cur_n = uniform(s_waves[w][1]);
+            off_m = uniform(s_waves[w][2]);
+            off_n = uniform(s_waves[w][3]);
+            cur_sig = uniform(s_waves[w][4]);
         } else {
             cur_m = p.wave_sizes[w * 2] / BM;
             cur_n = p.wave_sizes[w * 2 + 1] / BN;
@@ -1083,29 +1144,42 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
     };
     enter_wave(0);
 
-    auto wait_flag = [&](int sig) -> bool {
-        if (tid == 0) {
-            const uint64_t* flags = PRODUCER ? p.wait_flags : p.flags;
-            s_spun = __hip_atomic_load(flags + sig, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 1ull;
-            if (s_spun && !spin_until_equal(flags + sig, 1ull, p.timeout_ticks)) {
-                report_status(p.status, SYN_STATUS_SPIN_TIMEOUT, cur_wave, pid, sig);
-                s_abort = 1;
+    // wait for the flag of the wave that was entered
+    auto wait_flag = [&]() -> bool {
+        if (wave == 0) {
+            const int sig = wait_index(cur_wave + lane);
+            const bool up = sig < 0 || __hip_atomic_load(wait_on + sig, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 1ull;
+            const unsigned long long down = ~__builtin_amdgcn_ballot_w64(up);
+            if (lane == 0) {
+                s_waves_up = cur_wave + (down == 0 ? 64 : max((int)__builtin_ctzll(down), 1));
+                s_spun = (int)(down & 1);
+                if (s_spun && !spin_until_equal(wait_on + sig, 1ull, p.timeout_ticks)) {
+                    report_status(p.status, SYN_STATUS_SPIN_TIMEOUT, cur_wave, pid, sig);
+                    s_abort = 1;
+                }
             }
         }
         __syncthreads();
+        waves_up = uniform(s_waves_up);
         // No program reads a chunk's rows before its flag is up, so the XCD's L2 (emptied when the kernel
         // began) cannot hold a stale line of it.  The acquire fence drops every clean line of that L2 -
         // the panels of A and B its 28 other programs are reusing - so only a program that really had
         // to wait takes it.  That rests on the caller: nothing on the device reads the gathered buffer
         // between the start of this kernel and a chunk's flag, and no flag is raised twice during the
-        // launch.  SYN_GEMM_ACQUIRE_ALWAYS is for callers that cannot promise that.
-        if (s_spun || p.acquire_always) acquire_fence_agent();
-        return s_abort == 0;
+        // launch.  SYN_GEMM_ACQUIRE_ALWAYS is for callers that cannot promise that.  (One wavefront's fence drops the
+        // lines of the compute unit's L1 and the XCD's L2 for all, which load behind the barrier.)
+        if (wave == 0 && (uniform(s_spun) || p.acquire_always)) {
+            acquire_fence_agent();
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, true));
+        }
+        const bool ok = uniform(s_abort) == 0;
+        __syncthreads();       // the words may be written again only when everyone has read them
+        return ok;
     };
 
     // the reference's consumer waits for wave 0 before it looks at its first tile (template.py:92-97)
-    if (cur_wait >= 0) {
-        if (!wait_flag(cur_wait)) return;
+    if (cur_wait >= 0 && waves_up == 0) {
+        if (!wait_flag()) return;
     }
 
     const T* __restrict__ A = reinterpret_cast<const T*>(p.a);
@@ -1125,7 +1199,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
             enter_wave(cur_wave + 1);
             new_wave = true;
         }
-        return new_wave && cur_wait >= 0;
+        return new_wave && cur_wait >= 0 && cur_wave >= waves_up;
     };
 
     struct Tile {
@@ -1183,43 +1257,12 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
     auto panel_a = [&](const Tile& t) { return t.a_panel; };
     auto panel_b = [&](const Tile& t) { return t.b_panel; };
 
-    if (tiles_here == 0) return;
-    if (advance(pid)) {
-        if (!wait_flag(cur_wait)) return;
-    }
-    if (cur_wave < 0) return;
-    Tile tile = locate(pid);
-    Pipe::prologue(panel_a(tile), panel_b(tile), row_bytes, tile.k_len, tile.k_rot, lane, wave);
+    constexpr bool M16 = Pipe::kMfma16;                   // 16x16x32 MFMAs: 2 TM x 2 TN accumulators of four floats
+    constexpr int AR = M16 ? 2 * TM : TM, AC = M16 ? 2 * TN : TN, AE = M16 ? 4 : 16;
+    typedef typename std::conditional<M16, f32x4_t, f32x16_t>::type acc_t;
 
-    for (int it = 0; it < tiles_here; ++it) {
-        constexpr bool M16 = Pipe::kMfma16;                   // 16x16x32 MFMAs: 2 TM x 2 TN accumulators of four floats
-        constexpr int AR = M16 ? 2 * TM : TM, AC = M16 ? 2 * TN : TN, AE = M16 ? 4 : 16;
-        typename std::conditional<M16, f32x4_t, f32x16_t>::type acc[AR][AC];
-#pragma unroll
-        for (int i = 0; i < AR; ++i)
-#pragma unroll
-            for (int j = 0; j < AC; ++j)
-#pragma unroll
-                for (int e = 0; e < AE; ++e) acc[i][j][e] = 0.f;
-
-        Pipe::main(acc, panel_a(tile), panel_b(tile), row_bytes, tile.k_len, tile.k_rot, lane, wave);
-
-        // The stages are free: start the next tile's fills before this tile's C is stored, unless
-        // the next tile opens a wave whose flag is still to be waited for (nothing of a chunk may
-        // be read before its flag).
-        const bool has_next = it + 1 < tiles_here;
-        const int next_id = pid + (it + 1) * num_sms;
-        bool gated = false;
-        Tile next = tile;
-        if (has_next) {
-            gated = advance(next_id);
-            if (cur_wave < 0) return;
-            if (!gated) {
-                next = locate(next_id);
-                Pipe::prologue(panel_a(next), panel_b(next), row_bytes, next.k_len, next.k_rot, lane, wave);
-            }
-        }
-
+    // the C tile leaves, and with it the count of a producer's wave
+    auto store_tile = [&](const acc_t (&acc)[AR][AC], const Tile& tile) __attribute__((always_inline)) {
         // Epilogue.  With B as the first MFMA operand a lane holds, for column m = lane % 32 of
         // D', rows n = 8g + 4*(lane/32) + 0..3: four consecutive elements of one row of C.
         {
@@ -1322,13 +1365,98 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
                 }
             }
         }
+    };
+    auto clear = [&](acc_t (&acc)[AR][AC]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < AR; ++i)
+#pragma unroll
+            for (int j = 0; j < AC; ++j)
+#pragma unroll
+                for (int e = 0; e < AE; ++e) acc[i][j][e] = 0.f;
+    };
+
+    if (tiles_here == 0) return;
+    if (advance(pid)) {
+        if (!wait_flag()) return;
+    }
+    if (cur_wave < 0) return;
+    Tile tile = locate(pid);
+
+    if constexpr (Pipe::kRolls) {
+        auto source = [&](const Tile& t) __attribute__((always_inline)) { return Pipe::source(t.a_panel, t.b_panel, t.k_len, t.k_rot); };
+        typename Pipe::Source here = source(tile);
+        int stage = 0;
+        bool primed = false;
+        typename Pipe::frag_t fa[2][Pipe::RM], fb[2][Pipe::RN];
+        typename Pipe::Stream at = Pipe::prologue(here, stage, row_bytes, lane, wave);
+        for (int it = 0; it < tiles_here; ++it) {
+            // The next tile is worked out in front of this one's K loop, which goes on into it - unless it opens a wave whose flag
+            // was not up when flags were last read (nothing of a chunk may be read before its flag), or one of them is short.
+            bool has_next = it + 1 < tiles_here, gated = false, chained = false;
+            const int next_id = pid + (it + 1) * num_sms;
+            Tile next = tile;
+            typename Pipe::Source there = here;
+            if (has_next) {
+                gated = uniform(advance(next_id));
+                if (uniform(cur_wave) < 0) {
+                    has_next = false;
+                } else if (!gated) {
+                    next = locate(next_id);
+                    there = source(next);
+                    chained = here.slabs >= Pipe::kChainSlabs && there.slabs >= Pipe::kChainSlabs;
+                }
+            }
+            acc_t acc[AR][AC];
+            clear(acc);
+            Pipe::main(acc, fa, fb, stage, at, here, there, chained, primed, row_bytes, lane, wave);
+            if (has_next && !gated && !chained) at = Pipe::prologue(there, stage, row_bytes, lane, wave);
+            primed = chained;
+            if (chained) Pipe::enter(at, there);
+            store_tile(acc, tile);
+            if (!has_next) return;
+            if (gated) {
+                if (!wait_flag()) return;
+                next = locate(next_id);
+                there = source(next);
+                at = Pipe::prologue(there, stage, row_bytes, lane, wave);
+            }
+            tile = next;
+            here = there;
+        }
+        return;
+    } else {
+    Pipe::prologue(panel_a(tile), panel_b(tile), row_bytes, tile.k_len, tile.k_rot, lane, wave);
+
+    for (int it = 0; it < tiles_here; ++it) {
+        acc_t acc[AR][AC];
+        clear(acc);
+        Pipe::main(acc, panel_a(tile), panel_b(tile), row_bytes, tile.k_len, tile.k_rot, lane, wave);
+
+        // The stages are free: start the next tile's fills before this tile's C is stored, unless
+        // the next tile opens a wave whose flag is still to be waited for (nothing of a chunk may
+        // be read before its flag).
+        const bool has_next = it + 1 < tiles_here;
+        const int next_id = pid + (it + 1) * num_sms;
+        bool gated = false;
+        Tile next = tile;
+        if (has_next) {
+            gated = advance(next_id);
+            if (cur_wave < 0) return;
+            if (!gated) {
+                next = locate(next_id);
+                Pipe::prologue(panel_a(next), panel_b(next), row_bytes, next.k_len, next.k_rot, lane, wave);
+            }
+        }
+
+        store_tile(acc, tile);
 
         if (has_next && gated) {
-            if (!wait_flag(cur_wait)) return;
+            if (!wait_flag()) return;
             next = locate(next_id);
             Pipe::prologue(panel_a(next), panel_b(next), row_bytes, next.k_len, next.k_rot, lane, wave);
         }
         tile = next;
+    }
     }
 }
 
