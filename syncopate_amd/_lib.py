@@ -203,6 +203,7 @@ _SIGNATURES = {
     "syn_delay_us": (c_int32, [c_int64, c_void_p]),
     "syn_stream_create_cu_mask": (c_int32, [POINTER(ctypes.c_uint32), ctypes.c_uint32, POINTER(c_void_p)]),
     "syn_stream_destroy": (c_int32, [c_void_p]),
+    "syn_read_tables_async": (c_int32, [POINTER(c_void_p), POINTER(c_int32), c_int32, c_void_p, c_void_p, ctypes.c_uint64, c_void_p]),
     "syn_where_async": (c_int32, [c_void_p, c_int32, c_int32, c_void_p]),
     "syn_probe_mfma_rate": (c_int32, [c_void_p, c_int32, c_int32, c_int32, c_void_p]),
     "syn_probe_read_streams": (c_int32, [c_void_p, ctypes.c_int64, ctypes.c_int64, c_int32, c_int32, c_void_p, c_void_p]),
@@ -215,7 +216,8 @@ EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
 _lib: Optional[ctypes.CDLL] = None
 _native = None
-_NATIVE_CALLS = ("syn_gemm_consumer", "syn_gemm_producer", "syn_gemm_remote_binding", "syn_ring_reduce_strided", "syn_attn_fwd")
+_NATIVE_CALLS = ("syn_gemm_consumer", "syn_gemm_producer", "syn_gemm_remote_binding", "syn_ring_reduce_strided", "syn_attn_fwd",
+                 "syn_read_tables_async")
 
 
 def load() -> ctypes.CDLL:

@@ -37,6 +37,8 @@ gemm_fn g_consumer = nullptr, g_producer = nullptr;
 remote_fn g_remote = nullptr;
 reduce_fn g_reduce = nullptr;
 attn_fn g_attn = nullptr;
+typedef int (*read_fn)(const int32_t* const*, const int32_t*, int32_t, int32_t*, uint64_t*, uint64_t, syn_stream_t);
+read_fn g_read = nullptr;
 
 constexpr size_t kMaxRecords = 1024, kMaxPools = 64;
 constexpr int kPoolAreas = 16;
@@ -485,14 +487,75 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
     CATCH
 }
 
-// bind(addresses of syn_gemm_consumer, syn_gemm_producer, syn_gemm_remote_binding, syn_ring_reduce_strided, syn_attn_fwd)
-PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    if (n != 5) {
-        PyErr_SetString(PyExc_TypeError, "bind takes five addresses");
+// read_tables(offsets, sizes, cums, signals) -> their words as bytes, as they are at this point of the current stream, or None
+//
+// The words go to pinned memory that this call has to itself (from a bounded list that is never freed: the process may end
+// in any order) and the host looks at the word behind them.  Work in front of it that takes long is waited for asleep.
+constexpr int64_t kReadWords = 4096;
+PyObject* read_tables(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    TRY
+    NEED(n == 4 && !modes_active());
+    const at::Tensor* first = plain(args[0]);
+    NEED(first);
+    const int dev = first->device().index();
+    NEED(dev == c10::hip::current_device() && !capturing(dev));
+    const int32_t* tables[4];
+    int32_t counts[4];
+    int64_t words = 0;
+    for (int i = 0; i < 4; ++i) {
+        const at::Tensor* t = plain(args[i], dev);
+        NEED(t && t->scalar_type() == at::kInt && t->is_contiguous() && t->numel() <= kReadWords &&
+             (i < 2 ? t->numel() % 4 == 0 : t->dim() == 1));
+        tables[i] = static_cast<const int32_t*>(t->data_ptr());
+        counts[i] = (int32_t)t->numel();
+        words += counts[i];
+    }
+    NEED(words <= kReadWords);
+    static auto* const spare = new std::vector<at::Tensor>;
+    static uint64_t last = 0;
+    at::Tensor buffer;
+    if (!spare->empty()) {
+        buffer = spare->back();
+        spare->pop_back();
+    } else {
+        buffer = at::zeros({kReadWords + 16}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+    }
+    int32_t* const out = buffer.data_ptr<int32_t>();
+    uint64_t* const flag = reinterpret_cast<uint64_t*>(out + kReadWords);
+    const uint64_t seq = ++last;
+    hipStream_t stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream();
+    int rc;
+    bool there = false;
+    Py_BEGIN_ALLOW_THREADS
+    rc = g_read(tables, counts, 4, out, flag, seq, reinterpret_cast<syn_stream_t>(stream));
+    if (rc == 0) {
+        for (int i = 0; i < 20000 && !(there = __atomic_load_n(flag, __ATOMIC_ACQUIRE) == seq); ++i) __builtin_ia32_pause();
+        if (!there) {
+            rc = (int)hipStreamSynchronize(stream);
+            there = __atomic_load_n(flag, __ATOMIC_ACQUIRE) == seq;
+        }
+    }
+    Py_END_ALLOW_THREADS
+    if (rc != 0 || !there) {                 // (the buffer may still be written to: it is not used again)
+        new at::Tensor(buffer);
+        PyErr_Format(PyExc_RuntimeError, "reading the wave tables back failed: %d", rc);
         return nullptr;
     }
-    void* fn[5];
-    for (int i = 0; i < 5; ++i) {
+    PyObject* bytes = PyBytes_FromStringAndSize(reinterpret_cast<const char*>(out), words * 4);
+    if (spare->size() < 8) spare->push_back(buffer);
+    return bytes;
+    CATCH
+}
+
+// bind(addresses of syn_gemm_consumer, syn_gemm_producer, syn_gemm_remote_binding, syn_ring_reduce_strided, syn_attn_fwd,
+// syn_read_tables_async)
+PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != 6) {
+        PyErr_SetString(PyExc_TypeError, "bind takes six addresses");
+        return nullptr;
+    }
+    void* fn[6];
+    for (int i = 0; i < 6; ++i) {
         fn[i] = PyLong_AsVoidPtr(args[i]);
         if (PyErr_Occurred()) return nullptr;
     }
@@ -501,6 +564,7 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
     g_remote = reinterpret_cast<remote_fn>(fn[2]);
     g_reduce = reinterpret_cast<reduce_fn>(fn[3]);
     g_attn = reinterpret_cast<attn_fn>(fn[4]);
+    g_read = reinterpret_cast<read_fn>(fn[5]);
     Py_RETURN_NONE;
 }
 
@@ -510,6 +574,7 @@ PyMethodDef g_methods[] = {
     {"remote", (PyCFunction)(void*)remote, METH_FASTCALL, "launch (or remember) a GEMM whose C is bound to peers"},
     {"reduce", (PyCFunction)(void*)reduce, METH_FASTCALL, "launch a chunked ring reduce"},
     {"attention", (PyCFunction)(void*)attention, METH_FASTCALL, "launch (or remember) a chunked attention"},
+    {"read_tables", (PyCFunction)(void*)read_tables, METH_FASTCALL, "the words of four small tables in device memory"},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_native", "steady-state launches", -1, g_methods, nullptr, nullptr, nullptr, nullptr};

@@ -360,6 +360,25 @@ __global__ void __launch_bounds__(256) where_kernel(uint32_t* out, int dwell) {
     }
 }
 
+// Up to four small tables into host memory, one behind the other, and then `seq` into the word the host looks at.  One workgroup:
+// the tables of a launch are a few hundred words, and what is waited for is the way to the host, 3 us from an idle queue
+// (a gathering kernel, a copy and a wait for the stream took the host 35).
+struct ReadTables {
+    const int32_t* table[4];
+    int32_t count[4];
+};
+__global__ void __launch_bounds__(256) read_tables_kernel(const ReadTables t, int32_t* words, uint64_t* flag, uint64_t seq) {
+    int at = 0;
+    for (int i = 0; i < 4; ++i) {
+        for (int k = threadIdx.x; k < t.count[i]; k += 256)
+            __hip_atomic_store(words + at + k, t.table[i][k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        at += t.count[i];
+    }
+    __builtin_amdgcn_s_waitcnt(0);       // every lane's stores are acknowledged in front of the barrier
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ void __launch_bounds__(64) delay_kernel(int64_t ticks) {
     if (threadIdx.x == 0) {
         const uint64_t t0 = wall_clock64();
@@ -506,6 +525,20 @@ int syn_flag_wait(const uint64_t* flag, uint64_t value, int64_t spin_timeout_us,
     hipLaunchKernelGGL(syn::flag_wait_kernel, dim3(1), dim3(64), 0,
                        reinterpret_cast<hipStream_t>(stream), flag, value,
                        syn::timeout_ticks(spin_timeout_us), status);
+    return (int)hipGetLastError();
+}
+
+int syn_read_tables_async(const int32_t* const* tables, const int32_t* counts, int32_t n, int32_t* host_words, uint64_t* host_flag,
+                          uint64_t seq, syn_stream_t stream) {
+    if (!tables || !counts || n < 1 || n > 4 || !host_words || !host_flag) return SYN_EINVAL;
+    syn::ReadTables t = {};
+    for (int i = 0; i < n; ++i) {
+        if (counts[i] < 0 || (counts[i] > 0 && !tables[i])) return SYN_EINVAL;
+        t.table[i] = tables[i];
+        t.count[i] = counts[i];
+    }
+    hipLaunchKernelGGL(syn::read_tables_kernel, dim3(1), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), t, host_words, host_flag,
+                       seq);
     return (int)hipGetLastError();
 }
 

@@ -194,3 +194,26 @@ def test_reduce_is_launched_or_refused(hip, monkeypatch, acc_mode):
         module.ring_reduce(received, out, local.float(), 1, acc_mode=acc_mode)
     with pytest.raises(_lib.SyncopateHipError):
         module.ring_reduce(received, out, local, 3, acc_mode=acc_mode)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 3, 64, 341])
+def test_tables_are_read_at_their_place_in_the_stream(hip, rows):
+    native = _lib.native()
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    offsets, sizes = (torch.randint(-9, 2 ** 30, (4 * rows,), device="cuda", generator=g, dtype=torch.int32) for _ in range(2))
+    cums, signals = (torch.randint(-9, 2 ** 30, (rows,), device="cuda", generator=g, dtype=torch.int32) for _ in range(2))
+    for stream in (torch.cuda.current_stream(), torch.cuda.Stream()):
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            for round in range(12):
+                torch.cuda._sleep(100_000 if round % 4 else 20_000_000)      # behind work that takes 40 us, or 10 ms
+                cums.add_(1)
+                got = native.read_tables(offsets.view(-1, 4), sizes, cums, signals)
+                want = torch.cat([offsets, sizes, cums, signals]).cpu()
+                assert got == want.numpy().tobytes()
+        stream.synchronize()
+    assert native.read_tables(offsets, sizes, cums, signals.long()) is None
+    assert native.read_tables(offsets, sizes, cums, signals.cpu()) is None
+    assert native.read_tables(offsets[1:], sizes, cums, signals) is None
+    assert native.read_tables(torch.cat([offsets] * 8192)[:8192], sizes, cums, signals) is None if rows >= 3 else True
