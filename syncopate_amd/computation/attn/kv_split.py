@@ -27,8 +27,9 @@ BLOCK_US, SEGMENT_US, STEP_US = 3.6, 14.0, 8.0
 # segment, and the second kernel (its launch, and 136 KB of every part stored and loaded; 256 parts 6.8 us, 16 4.1).
 # Measured: 32 pairs of 64 blocks as 1, 2, 4, 7, 8 parts 201, 112, 69, 54 and 51 us, 48 pairs of 48 as 2, 4, 5 90, 59 and 55.
 DEAL_BLOCK_US, DEAL_FULL_US, DEAL_SEGMENT_US, DEAL_ADD_US, DEAL_ADD_FULL_US = 2.8, 0.9, 13.0, 4.0, 5.0
-# What the host takes for a launch of two kernels and their slots: tiles that take less stay single.
-DEAL_HOST_US = 38.0
+DEAL_BURST_US, DEAL_BURST_BLOCK_US = 20.0, 2.4         # 200 programs of 4 blocks 44 us, 154 of 2 36, 84 of 2 30
+# Tiles that take less than the two launches of a cut table, with what lies around them, stay single.
+DEAL_HOST_US = 24.0
 MERGE_US = 5.0
 MIN_GAIN_US = 10.0        # (the words and slots of the parts cost the host 3 us a launch, which small ones wait for)
 RESERVED_UNITS = 32       # compute units that launches which wait leave to the copies that raise their flags
@@ -53,11 +54,14 @@ def _steps(parts: int) -> int:
     return (parts - 1).bit_length()
 
 
-def _deal_us(pairs: int, parts: int, blocks: int, units: int) -> float:
-    """What `pairs` of `blocks` kv blocks take, dealt to `parts` programs each."""
+def _deal_us(pairs: int, parts: int, blocks: int, units: int, burst: bool = True) -> float:
+    """What `pairs` of `blocks` kv blocks take, dealt to `parts` programs each (`burst`: these are all the blocks there are)."""
     programs = pairs * parts
     share = min(programs / units, 1.0)
-    us = -(-programs // units) * (-(-blocks // parts) * (DEAL_BLOCK_US + DEAL_FULL_US * share) + DEAL_SEGMENT_US)
+    each = -(-blocks // parts)
+    us = -(-programs // units) * (each * (DEAL_BLOCK_US + DEAL_FULL_US * share) + DEAL_SEGMENT_US)
+    if parts > 1 and burst:              # the sums of short parts go to memory all at once
+        us += share * max(DEAL_BURST_US - DEAL_BURST_BLOCK_US * each, 0.0)
     return us + (DEAL_ADD_US + DEAL_ADD_FULL_US * programs / units if parts > 1 else 0.0)
 
 
@@ -137,7 +141,7 @@ def _split_chain(waves, signal_offsets: Sequence[int], units: int, always: bool,
         if always and flagged:
             if not dealt and min(-(-total // parts), flagged[-1]) * BLOCK_US + SEGMENT_US + 2.0 * _steps(parts) > last_us:
                 continue
-            us += max(_deal_us(pairs, parts, flagged[-1], units) - last_us, 0.0) if dealt else 0.0
+            us += max(_deal_us(pairs, parts, flagged[-1], units, burst=False) - last_us, 0.0) if dealt else 0.0
         whole_us = whole_us or us
         if best is None or us < best_us:
             best, best_us = parts, us
