@@ -137,8 +137,12 @@ def host_copy(t: torch.Tensor) -> torch.Tensor:
 
 
 def host_copies(tables: Sequence[torch.Tensor]) -> List[torch.Tensor]:
-    """CPU copies of int32 device tables, read back together: one wait for the stream instead of one per table."""
-    flat = torch.cat([t.detach().reshape(-1) for t in tables]).cpu()
+    """CPU copies of up to four int32 device tables, read back together: one wait for the stream instead of one per table."""
+    words = _lib.native().read_tables(*tables)       # None for what are not a few small tables in plain tensors
+    if words is not None:
+        flat = torch.frombuffer(bytearray(words), dtype=torch.int32)
+    else:
+        flat = torch.cat([t.detach().reshape(-1) for t in tables]).cpu()
     return [part.view(t.shape) for t, part in zip(tables, flat.split([t.numel() for t in tables]))]
 
 

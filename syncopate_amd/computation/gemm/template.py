@@ -26,6 +26,7 @@ from .._launch import (
     already_checked,
     as_device_table,
     flag_buffer,
+    host_copies,
     host_copy,
     host_ptr,
     launches_on_stream,
@@ -112,7 +113,7 @@ def _launch(
     caller_owned = all(isinstance(t, torch.Tensor) and t.is_cuda
                        for t in (cur_wave_size, wave_offset, signal_offsets))
     if not (caller_owned and already_checked(tables, params)):
-        hs, ho, hg = host_copy(sizes), host_copy(offsets), host_copy(signals)
+        hs, ho, hg = host_copies((sizes, offsets, signals))
         _lib.check(
             "syn_gemm_check_waves",
             lib.syn_gemm_check_waves(host_ptr(hs), host_ptr(ho), host_ptr(hg), num_waves, M, N, K,

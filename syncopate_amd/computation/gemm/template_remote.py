@@ -26,7 +26,7 @@ from typing import Optional, Sequence
 import torch
 
 from ... import _lib
-from .._launch import (TableLike, compute_units, device_scope, acquire_always, as_device_table, host_copy, host_ptr, launches_on_stream, recall_note,
+from .._launch import (TableLike, compute_units, device_scope, acquire_always, as_device_table, host_copies, host_copy, host_ptr, launches_on_stream, recall_note,
                        remember_note, require_cuda, status_words)
 from .template import RESERVED_UNITS
 from .tile_policy import choose_kernel_tile
@@ -69,7 +69,7 @@ def _prepare_binding(lib, sizes, offsets, signals, flags, num_waves, M, N, K, bl
                      a_list, a_target_rank, c_list, target_rank, dst_offsets, atomic_add, k_ranges, dev):
     """The host's share of a bound launch: table checks, and the device tables the kernel reads (pointer tables,
     ranks, destination offsets, k ranges).  Returns the fields of the remote descriptor and the tensors they point into."""
-    hs, ho, hg = host_copy(sizes), host_copy(offsets), host_copy(signals)
+    hs, ho, hg = host_copies((sizes, offsets, signals))
     _lib.check("syn_gemm_check_waves",
                lib.syn_gemm_check_waves(host_ptr(hs), host_ptr(ho), host_ptr(hg), num_waves, M, N, K,
                                         block_m, block_n, block_k, int(cum_tiles), flags.numel()))

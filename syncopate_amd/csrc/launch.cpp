@@ -487,14 +487,15 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
     CATCH
 }
 
-// read_tables(offsets, sizes, cums, signals) -> their words as bytes, as they are at this point of the current stream, or None
+// read_tables(table, ...) -> the words of one to four small int32 tables as bytes, as they are at this point of the current
+// stream, or None
 //
 // The words go to pinned memory that this call has to itself (from a bounded list that is never freed: the process may end
 // in any order) and the host looks at the word behind them.  Work in front of it that takes long is waited for asleep.
 constexpr int64_t kReadWords = 4096;
 PyObject* read_tables(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TRY
-    NEED(n == 4 && !modes_active());
+    NEED(n >= 1 && n <= 4 && !modes_active());
     const at::Tensor* first = plain(args[0]);
     NEED(first);
     const int dev = first->device().index();
@@ -502,15 +503,14 @@ PyObject* read_tables(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int32_t* tables[4];
     int32_t counts[4];
     int64_t words = 0;
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < (int)n; ++i) {
         const at::Tensor* t = plain(args[i], dev);
-        NEED(t && t->scalar_type() == at::kInt && t->is_contiguous() && t->numel() <= kReadWords &&
-             (i < 2 ? t->numel() % 4 == 0 : t->dim() == 1));
+        NEED(t && t->scalar_type() == at::kInt && t->is_contiguous() && t->numel() <= kReadWords);
         tables[i] = static_cast<const int32_t*>(t->data_ptr());
         counts[i] = (int32_t)t->numel();
         words += counts[i];
     }
-    NEED(words <= kReadWords);
+    NEED(words > 0 && words <= kReadWords);
     static auto* const spare = new std::vector<at::Tensor>;
     static uint64_t last = 0;
     at::Tensor buffer;
@@ -527,7 +527,7 @@ PyObject* read_tables(PyObject*, PyObject* const* args, Py_ssize_t n) {
     int rc;
     bool there = false;
     Py_BEGIN_ALLOW_THREADS
-    rc = g_read(tables, counts, 4, out, flag, seq, reinterpret_cast<syn_stream_t>(stream));
+    rc = g_read(tables, counts, (int32_t)n, out, flag, seq, reinterpret_cast<syn_stream_t>(stream));
     if (rc == 0) {
         for (int i = 0; i < 20000 && !(there = __atomic_load_n(flag, __ATOMIC_ACQUIRE) == seq); ++i) __builtin_ia32_pause();
         if (!there) {
