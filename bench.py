@@ -1134,7 +1134,7 @@ def main():
     flop = 2.0 * M * N * K
     value = flop / (wall_ms * 1e-3) / 1e12
     kernel_tflops = flop / (gated_ms * 1e-3) / 1e12
-    kernel_name = (f"gemm_wave_kernel<bf16, {'EarlyPipe16' if (BM, BN) in ((256, 256), (256, 224)) else 'SlabPipe<3 stages>'}, "
+    kernel_name = (f"gemm_wave_kernel<bf16, {'RollPipe<2 stages>' if (BM, BN) in ((256, 256), (256, 224)) else 'RollPipe<3 stages>'}, "
                    f"{BM}x{BN}, {8 if EIGHT_WAVES else 4} wavefronts, consumer>")
     traffic = _traffic().get("gemm_consumer_256x256_224_programs", {}) if (BM, BN, NUM_SMS) == (256, 256, 224) else {}
     line = {

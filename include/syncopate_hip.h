@@ -78,6 +78,9 @@ extern "C" {
 
 #define SYN_GEMM_CUT_TILE 128u      /* cut_m and cut_n hold; without it they are not read (a descriptor may
                                        then end behind `options`, as it did before version 200)   */
+#define SYN_GEMM_CUT_TAIL 256u      /* tiles that do not fill a round may run as 128x128 ones: same results bit
+                                       for bit; a producer then counts a wave's pieces, so its counters end
+                                       at a multiple of the wave's tiles                          */
 
 typedef void* syn_stream_t;        /* hipStream_t */
 

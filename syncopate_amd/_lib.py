@@ -35,6 +35,7 @@ SYN_GEMM_TWO_STAGE = 16
 SYN_GEMM_MFMA_32X32 = 32
 SYN_GEMM_ACQUIRE_ALWAYS = 64
 SYN_GEMM_CUT_TILE = 128
+SYN_GEMM_CUT_TAIL = 256
 SYN_ATTN_PAIR_Q_BLOCKS = 1
 SYN_ATTN_XCD_REMAP = 2
 SYN_ATTN_CHAIN_Q_BLOCKS = 4

@@ -210,7 +210,7 @@ def _launch(
         | (_lib.SYN_GEMM_TWO_STAGE if two_stage else 0) | (_lib.SYN_GEMM_MFMA_32X32 if mfma_32x32 else 0)
         | (_lib.SYN_GEMM_ACQUIRE_ALWAYS
            if acquire_always(wait_signal_buffer if wait_signal_buffer is not None else signal_buffer) else 0)
-        | (_lib.SYN_GEMM_CUT_TILE if cut != (0, 0) else 0),
+        | (_lib.SYN_GEMM_CUT_TILE if cut != (0, 0) else 0) | (0 if counts_seen else _lib.SYN_GEMM_CUT_TAIL),
         cut_m=cut[0], cut_n=cut[1],
     )
     with device_scope(dev):

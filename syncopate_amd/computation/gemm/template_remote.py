@@ -254,7 +254,7 @@ def gemm_remote(
         group_m=GROUP_SIZE_M, num_sms=num_gemm_sms, cum_tiles=int(cum_tiles), spin_timeout_us=0,
         options=(_lib.SYN_GEMM_XCD_REMAP if xcd_remap else 0) | (_lib.SYN_GEMM_EIGHT_WAVES if eight_waves else 0)
         | (_lib.SYN_GEMM_ACQUIRE_ALWAYS if signal_ptr is not None and acquire_always(signal_ptr) else 0)
-        | (_lib.SYN_GEMM_CUT_TILE if cut != (0, 0) else 0),
+        | (_lib.SYN_GEMM_CUT_TILE if cut != (0, 0) else 0) | _lib.SYN_GEMM_CUT_TAIL,
         cut_m=cut[0], cut_n=cut[1],
     )
     with device_scope(dev):

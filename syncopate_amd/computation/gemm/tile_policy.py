@@ -22,7 +22,8 @@ from typing import Iterable, Optional, Tuple
 
 # Cost of one round of tiles of each shape (K = 8192, microseconds; only the ratios matter).
 # RESIDENT_COST: every program busy - from the resident 8192 x 8192 x 3584 GEMM on 224 programs (256x256: 2 rounds in
-# 326 us; 128x256 / 256x128: 4 rounds in 376 / 367 us; 128x128: 8 rounds in 540 us).
+# 326 us; 128x256 / 256x128: 4 rounds in 376 / 367 us; 128x128: 8 rounds in 540 us).  (128x128 on 32x32x16 MFMAs and with
+# a prologue a tile; it takes about 15 % less since tiles run on from one to the next, the others 2 to 5.)
 # LAST_ROUND_COST: the round that is left when the last chunk lands - measured as the step's time beyond the
 # producer's with one link's delay per chunk (209 / 88 / 85 / 92 us, of which ~20 us are the flag's way to the
 # kernel, the epilogue and the stream join).  Half-empty rounds run faster than full ones: the idle compute units

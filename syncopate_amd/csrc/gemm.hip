@@ -30,6 +30,7 @@
 #include <cstddef>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 
@@ -69,6 +70,7 @@ struct GemmParams {
     // whose partial products are added into C); null: every wave takes all of K
     const int32_t* wave_k;
     int32_t cut_m, cut_n;        // the caller's tile is 2^cut_m x 2^cut_n of the kernel's
+    int32_t tail_tiles;          // TAIL kernels: the last so many tiles run as 128x128 ones
 };
 
 // kernel modes
@@ -136,6 +138,11 @@ __device__ __forceinline__ void mfma_result_wait_states(f32x4_t (&acc)[R][C]) {
         asm volatile("" : "+a"(x[i]), "+a"(x[i + 1]), "+a"(x[i + 2]), "+a"(x[i + 3]), "+a"(x[i + 4]), "+a"(x[i + 5]), "+a"(x[i + 6]),
                           "+a"(x[i + 7]));
 }
+
+template <typename P>
+struct type_tag {
+    typedef P type;
+};
 
 template <typename T>
 __device__ __forceinline__ uint2 pack4(float x0, float x1, float x2, float x3) {
@@ -620,7 +627,8 @@ struct EarlyPipe : SlabPipe<T, BM, BN, WGM, WGN, 2> {
 // and 115 -> 107; 256x256, 2 rounds of K = 2048 106.6 -> 103.6; one round the same to 1.5 %.  128x128, which ran on
 // 32x32x16 MFMAs with a k16 step (128 cycles) of look-ahead for its LDS reads: one round of K = 4096 36.2 -> 32.6, four 140.8 -> 118.8.
 // With power no limit (zeros) a 128x256 slab takes 1190 cycles for 1030 of MFMAs, with random operands 1.53 PFLOP/s.
-template <typename T, int BM, int BN, int WGM, int WGN, int NST_>
+// (HOME: the pipeline whose stages this one uses, in the same kernel)
+template <typename T, int BM, int BN, int WGM, int WGN, int NST_, typename HOME = void>
 struct RollPipe : SlabPipe<T, BM, BN, WGM, WGN, NST_> {
     typedef SlabPipe<T, BM, BN, WGM, WGN, NST_> Base;
     using Base::TM;
@@ -725,9 +733,15 @@ struct RollPipe : SlabPipe<T, BM, BN, WGM, WGN, NST_> {
     static __device__ __forceinline__ void enter(Stream& at, const Source& t) { at.turn = at.a - t.a >= (ptrdiff_t)((size_t)t.rot * ROW) ? 0 : 1; }
 
     // the stages, one behind the other: which of them a slab lives in is counted at run time
+    static constexpr int kStageBytes = NST * STAGE;
     static __device__ __forceinline__ unsigned char* stages() {
-        __shared__ __attribute__((aligned(1024))) unsigned char st[NST * STAGE];
-        return st;
+        if constexpr (std::is_void<HOME>::value) {
+            __shared__ __attribute__((aligned(1024))) unsigned char st[NST * STAGE];
+            return st;
+        } else {
+            static_assert(NST * STAGE <= HOME::kStageBytes, "the stages fit the other pipeline's");
+            return HOME::stages();
+        }
     }
     static __device__ __forceinline__ int behind(int stage) { return stage + 1 == NST ? 0 : stage + 1; }
 
@@ -1037,7 +1051,9 @@ __device__ __forceinline__ void atomic_add2<_Float16>(_Float16* dst, unsigned v)
     __builtin_amdgcn_global_atomic_fadd_v2f16((gptr)dst, __builtin_bit_cast(v2, v));
 }
 
-template <typename T, typename Pipe, int BM, int BN, int WGM, int WGN, int MODE>
+// TAIL: the tiles that do not fill a round run as 128x128 ones at the end, two or four of a tile, on a pipeline of their own in the
+// same stages.  72 of 520 tiles of 128x256, K = 2048, on 224 programs kept 72 of these busy for a third round: 72.6 us, as 144 65.6.
+template <typename T, typename Pipe, int BM, int BN, int WGM, int WGN, int MODE, bool TAIL = false>
 __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmParams p) {
     constexpr bool PRODUCER = MODE == kProducer;
     constexpr bool REMOTE = MODE == kRemote || MODE == kRemoteAtomic;
@@ -1062,7 +1078,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
 
     const int pid = logical_program_id((int)blockIdx.x, (int)gridDim.x, p.xcd_remap != 0);
     const int num_sms = p.num_sms;
-    const int num_tiles = p.num_tiles;
+    const int num_tiles = TAIL ? p.num_tiles - p.tail_tiles : p.num_tiles;
     const int tiles_here = num_tiles / num_sms + (pid < num_tiles % num_sms ? 1 : 0);
 
     const int K = p.K, N = p.N;
@@ -1182,6 +1198,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
         if (!wait_flag()) return;
     }
 
+    // how many of the smallest tiles make one of the caller's
+    constexpr int kShares = TAIL ? BM * BN / (128 * 128) : 1;
     const T* __restrict__ A = reinterpret_cast<const T*>(p.a);
     const T* __restrict__ B = reinterpret_cast<const T*>(p.b);
     T* __restrict__ C = reinterpret_cast<T*>(p.c);
@@ -1258,11 +1276,12 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
     auto panel_b = [&](const Tile& t) { return t.b_panel; };
 
     constexpr bool M16 = Pipe::kMfma16;                   // 16x16x32 MFMAs: 2 TM x 2 TN accumulators of four floats
-    constexpr int AR = M16 ? 2 * TM : TM, AC = M16 ? 2 * TN : TN, AE = M16 ? 4 : 16;
     typedef typename std::conditional<M16, f32x4_t, f32x16_t>::type acc_t;
 
-    // the C tile leaves, and with it the count of a producer's wave
-    auto store_tile = [&](const acc_t (&acc)[AR][AC], const Tile& tile) __attribute__((always_inline)) {
+    // the C tile leaves, and with it the count of a producer's wave (of `share` for every tile of the caller's)
+    auto store_tile = [&](auto pipe, const auto& acc, const Tile& tile, const int share) __attribute__((always_inline)) {
+        typedef typename decltype(pipe)::type P;
+        constexpr int WM = P::WM, WN = P::WN, TM = P::TM, TN = P::TN;
         // Epilogue.  With B as the first MFMA operand a lane holds, for column m = lane % 32 of
         // D', rows n = 8g + 4*(lane/32) + 0..3: four consecutive elements of one row of C.
         {
@@ -1357,22 +1376,22 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
                 __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, true));
                 __syncthreads();
                 if (tid == 0) {
-                    const int done = __hip_atomic_fetch_add(p.counters + tile.wave, 1, __ATOMIC_RELAXED,
+                    const int done = __hip_atomic_fetch_add(p.counters + tile.wave, share, __ATOMIC_RELAXED,
                                                             __HIP_MEMORY_SCOPE_AGENT);
-                    if (done == tile.wave_tiles - 1)
+                    if (done == tile.wave_tiles * kShares - share)
                         __hip_atomic_store(p.flags + tile.sig, 1ull, __ATOMIC_RELEASE,
                                            __HIP_MEMORY_SCOPE_SYSTEM);
                 }
             }
         }
     };
-    auto clear = [&](acc_t (&acc)[AR][AC]) __attribute__((always_inline)) {
+    auto clear = [&](auto& acc) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < AR; ++i)
+        for (auto& row : acc)
 #pragma unroll
-            for (int j = 0; j < AC; ++j)
+            for (auto& x : row)
 #pragma unroll
-                for (int e = 0; e < AE; ++e) acc[i][j][e] = 0.f;
+                for (int e = 0; e < (int)(sizeof(x) / sizeof(float)); ++e) x[e] = 0.f;
     };
 
     if (tiles_here == 0) return;
@@ -1383,52 +1402,76 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
     Tile tile = locate(pid);
 
     if constexpr (Pipe::kRolls) {
-        auto source = [&](const Tile& t) __attribute__((always_inline)) { return Pipe::source(t.a_panel, t.b_panel, t.k_len, t.k_rot); };
-        typename Pipe::Source here = source(tile);
-        int stage = 0;
-        bool primed = false;
-        typename Pipe::frag_t fa[2][Pipe::RM], fb[2][Pipe::RN];
-        typename Pipe::Stream at = Pipe::prologue(here, stage, row_bytes, lane, wave);
-        for (int it = 0; it < tiles_here; ++it) {
-            // The next tile is worked out in front of this one's K loop, which goes on into it - unless it opens a wave whose flag
-            // was not up when flags were last read (nothing of a chunk may be read before its flag), or one of them is short.
-            bool has_next = it + 1 < tiles_here, gated = false, chained = false;
-            const int next_id = pid + (it + 1) * num_sms;
-            Tile next = tile;
-            typename Pipe::Source there = here;
-            if (has_next) {
-                gated = uniform(advance(next_id));
-                if (uniform(cur_wave) < 0) {
-                    has_next = false;
-                } else if (!gated) {
-                    next = locate(next_id);
-                    there = source(next);
-                    chained = here.slabs >= Pipe::kChainSlabs && there.slabs >= Pipe::kChainSlabs;
+        // The tiles first, first + step, .. (`count` of them) on pipeline P; at(id): the tile, with the wave of its caller's tile entered.
+        auto walk = [&](auto pipe, const int first, const int count, const int shares, auto at_id, Tile tile) __attribute__((always_inline)) {
+            typedef typename decltype(pipe)::type P;
+            auto source = [&](const Tile& t) __attribute__((always_inline)) { return P::source(t.a_panel, t.b_panel, t.k_len, t.k_rot); };
+            typename P::Source here = source(tile);
+            int stage = 0;
+            bool primed = false;
+            typename P::frag_t fa[2][P::RM], fb[2][P::RN];
+            typename P::Stream at = P::prologue(here, stage, row_bytes, lane, wave);
+            for (int it = 0; it < count; ++it) {
+                // The next tile is worked out in front of this one's K loop, which goes on into it - unless it opens a wave whose flag
+                // was not up when flags were last read (nothing of a chunk may be read before its flag), or one of them is short.
+                bool has_next = it + 1 < count, gated = false, chained = false;
+                const int next_id = first + (it + 1) * num_sms;
+                Tile next = tile;
+                typename P::Source there = here;
+                if (has_next) {
+                    gated = uniform(advance(shares == 1 ? next_id : num_tiles + next_id / shares));
+                    if (uniform(cur_wave) < 0) {
+                        has_next = false;
+                    } else if (!gated) {
+                        next = at_id(next_id);
+                        there = source(next);
+                        chained = here.slabs >= P::kChainSlabs && there.slabs >= P::kChainSlabs;
+                    }
                 }
+                acc_t acc[P::RM][P::RN];
+                clear(acc);
+                P::main(acc, fa, fb, stage, at, here, there, chained, primed, row_bytes, lane, wave);
+                if (has_next && !gated && !chained) at = P::prologue(there, stage, row_bytes, lane, wave);
+                primed = chained;
+                if (chained) P::enter(at, there);
+                store_tile(pipe, acc, tile, kShares / shares);
+                if (!has_next) return uniform(cur_wave) >= 0;
+                if (gated) {
+                    if (!wait_flag()) return false;
+                    next = at_id(next_id);
+                    there = source(next);
+                    at = P::prologue(there, stage, row_bytes, lane, wave);
+                }
+                tile = next;
+                here = there;
             }
-            acc_t acc[AR][AC];
-            clear(acc);
-            Pipe::main(acc, fa, fb, stage, at, here, there, chained, primed, row_bytes, lane, wave);
-            if (has_next && !gated && !chained) at = Pipe::prologue(there, stage, row_bytes, lane, wave);
-            primed = chained;
-            if (chained) Pipe::enter(at, there);
-            store_tile(acc, tile);
-            if (!has_next) return;
-            if (gated) {
+            return true;
+        };
+        const bool on = walk(type_tag<Pipe>{}, pid, tiles_here, 1, locate, tile);
+        if constexpr (TAIL) {
+            typedef RollPipe<T, 128, 128, WGM, WGN, 3, Pipe> Small;
+            const int small_tiles = p.tail_tiles * kShares;
+            if (!on || pid >= small_tiles) return;      // (the loop of a last tile has drained: the stages are free)
+            auto part = [&](int id) __attribute__((always_inline)) {
+                Tile t = locate(num_tiles + id / kShares);
+                const int sub = id % kShares, sub_m = sub / (BN / 128), sub_n = sub % (BN / 128);
+                t.a_panel += (size_t)(sub_m * 128) * row_bytes;
+                t.b_panel += (size_t)(sub_n * 128) * row_bytes;
+                t.c_tile += (size_t)(sub_m * 128) * t.ldc + sub_n * 128;
+                return t;
+            };
+            if (advance(num_tiles + pid / kShares)) {
                 if (!wait_flag()) return;
-                next = locate(next_id);
-                there = source(next);
-                at = Pipe::prologue(there, stage, row_bytes, lane, wave);
             }
-            tile = next;
-            here = there;
+            if (cur_wave < 0) return;
+            walk(type_tag<Small>{}, pid, (small_tiles - pid + num_sms - 1) / num_sms, kShares, part, part(pid));
         }
         return;
     } else {
     Pipe::prologue(panel_a(tile), panel_b(tile), row_bytes, tile.k_len, tile.k_rot, lane, wave);
 
     for (int it = 0; it < tiles_here; ++it) {
-        acc_t acc[AR][AC];
+        acc_t acc[M16 ? 2 * TM : TM][M16 ? 2 * TN : TN];
         clear(acc);
         Pipe::main(acc, panel_a(tile), panel_b(tile), row_bytes, tile.k_len, tile.k_rot, lane, wave);
 
@@ -1448,7 +1491,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
             }
         }
 
-        store_tile(acc, tile);
+        store_tile(type_tag<Pipe>{}, acc, tile, 1);
 
         if (has_next && gated) {
             if (!wait_flag()) return;
@@ -1471,6 +1514,12 @@ template <typename T, template <typename, int, int, int, int> class PipeT, int B
           int MODE>
 static int launch_gemm(const GemmParams& p, int grid, hipStream_t stream) {
     typedef PipeT<T, BM, BN, WGM, WGN> Pipe;
+    if constexpr (Pipe::kRolls && WGM == 2 && WGN == 2 && BM % 128 == 0 && BN % 128 == 0 && BM * BN > 128 * 128) {
+        if (p.tail_tiles > 0) {
+            hipLaunchKernelGGL((gemm_wave_kernel<T, Pipe, BM, BN, WGM, WGN, MODE, true>), dim3(grid), dim3(64 * WGM * WGN), 0, stream, p);
+            return (int)hipGetLastError();
+        }
+    }
     hipLaunchKernelGGL((gemm_wave_kernel<T, Pipe, BM, BN, WGM, WGN, MODE>), dim3(grid),
                        dim3(64 * WGM * WGN), 0, stream, p);
     return (int)hipGetLastError();
@@ -1511,6 +1560,20 @@ static int dispatch_pipe(const GemmParams& p, int bm, int bn, bool eight, bool r
 }
 
 __global__ void __launch_bounds__(256) clear_words_kernel(int32_t* words, int n);
+
+// How many tiles, those beyond full rounds, run as 128x128 ones (SYN_GEMM_CUT_TAIL): behind at least one full round, and where they
+// take less then.  Measured on 224 programs, whole -> cut, K = 512 / 1024 / 2048 / 4096: 64 tiles of 128x256 behind a round 19.0 /
+// 29.7 / 50.3 / 93.0 -> 19.0 (not cut) / 25.9 / 42.5 / 75.5 us, 112 of them 30.4 / 51.9 / 94.4 -> 28.4 / 45.1 / 78.5; 16 of
+// 256x256 29.1 / 44.7 / 77.8 / 144.6 -> 25.1 / 36.1 / 59.1 / 107.5; but 64 of these, as two rounds, 28.8 / 44.8 / 78.5 / 145.3 ->
+// 30.5 / 47.4 / 75.7 / 134.9.  That is 0.667 and 1.04 us a slab of the last round's whole tiles, 0.41 of the 128x128 ones, and
+// 2.5 us a round of these for the first fills and the epilogue.
+static int gemm_tail_tiles(int tiles, int programs, int bm, int bn, int K) {
+    const int shares = bm * bn / (128 * 128), rest = tiles % programs;
+    if (bm % 128 || bn % 128 || (shares != 2 && shares != 4) || tiles <= programs || rest == 0) return 0;
+    const int rounds = (int)(((int64_t)rest * shares + programs - 1) / programs);
+    const double slabs = K / 64, whole = slabs * (shares == 2 ? 0.667 : 1.04), cut = rounds * (slabs * 0.41 + 2.5);
+    return cut < whole ? rest : 0;
+}
 
 // the tile shapes dispatch_tile has kernels for
 static bool gemm_tile_shape_built(int bm, int bn, bool eight) {
@@ -1595,6 +1658,10 @@ static int gemm_entry(const syn_gemm_desc* d, hipStream_t stream, int mode,
         p.cut_n = d->cut_n;
     }
     const bool eight = (d->options & SYN_GEMM_EIGHT_WAVES) != 0;
+    p.tail_tiles = 0;
+    if ((d->options & SYN_GEMM_CUT_TAIL) && !d->visit_log &&
+        !(d->options & (SYN_GEMM_EIGHT_WAVES | SYN_GEMM_RING_PIPE | SYN_GEMM_TWO_STAGE | SYN_GEMM_MFMA_32X32)))
+        p.tail_tiles = gemm_tail_tiles((int)tiles, grid, d->block_m, d->block_n, remote && remote->k_ranges ? 64 : d->K);
     // the ring needs whole groups of four 32-deep slabs (and does not exist for 224-wide tiles)
     const bool ring = (d->options & SYN_GEMM_RING_PIPE) && d->K % 128 == 0 && d->block_n != 224;
 
