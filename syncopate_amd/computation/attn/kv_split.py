@@ -6,8 +6,9 @@ whose sums are added up in 32 bits at the end.  Host logic on plain integers, li
 
 Two kinds of tables can be cut:
 
-* consumer tables whose waves all list the same (z, h, q) ranges (the all-gather table): the kv blocks of all waves in a row
-  are dealt to the parts one by one, and a second kernel adds the parts up (SYN_ATTN_SPLIT_DEAL);
+* consumer tables whose waves all list the same (z, h, q) ranges (the all-gather table): the parts are cut out of the kv
+  blocks of all waves in a row, in wave order; or the blocks are dealt to the parts one by one, and a second kernel adds the
+  parts up (SYN_ATTN_SPLIT_DEAL), for tables that would otherwise be single tiles;
 * producer tables that visit every pair of q blocks once (attention that feeds an exchange), causal or not.
 """
 
@@ -19,9 +20,9 @@ BLOCK = 128
 MAX_WAVES = 256           # wave-table rows that the kernel holds in LDS
 MAX_PARTS = 16
 MAX_SLOTS = 1024          # partial results in memory at a time: 136 KB each
-# Microseconds, from kernel traces (256 programs of 16 blocks and one step 80, of 8 blocks and three steps 62): a kv block of a
-# pair, what a segment costs beyond its blocks (launch, Q, first fills, epilogue), and a step of the tree in which a
-# producer's parts are added (136 KB stored, handed over and loaded).
+# Microseconds, from kernel traces (256 programs of 8 blocks and three steps 66, 192 of 12 blocks and two steps 68, 256 of
+# 16 blocks and one step 80): a kv block of a pair, what a segment costs beyond its blocks (launch, Q, first fills,
+# epilogue), and a step of the tree that adds the parts (136 KB stored, handed over and loaded).
 BLOCK_US, SEGMENT_US, STEP_US = 3.6, 14.0, 8.0
 # The same where the blocks are dealt: a kv block on a nearly idle chip and what it takes longer where all units are busy, a
 # segment, and the second kernel (its launch, and 136 KB of every part stored and loaded; 256 parts 6.8 us, 16 4.1).
@@ -77,17 +78,20 @@ def plan_kv_split(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Se
     waves = _real_waves(wave_offsets, wave_sizes, cum_wave_sizes, causal=causal, producer=producer)
     if not waves:
         return None
-    return _split_visits(waves, causal, units) if producer else _split_chain(waves, signal_offsets, units, always, dealt=False)
+    return _split_visits(waves, causal, units) if producer else _split_runs(waves, signal_offsets, units, always)
 
 
 def plan_kv_deal(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Sequence[int]], cum_wave_sizes: Sequence[int],
                  signal_offsets: Sequence[int], *, units: int) -> Optional[KvSplit]:
-    """The split of a consumer's tables that wait for flags and that `plan_kv_split` leaves to the kernel with one tile per
-    program: there a late chunk is looked at as if its blocks were one part's, here as the parts share it."""
+    """The split of a consumer's tables that `plan_kv_split` leaves to the kernel with one tile per program, as blocks that are dealt
+    to the parts: there a late chunk is looked at as if its blocks were one part's, here as the parts share it.  (Tables that
+    both would cut stay with the parts in wave order: a part that meets other blocks first rounds its probabilities against
+    another running maximum, and the results of tables that were always cut do not change.  48 pairs of 48 blocks take 73
+    us dealt and 79 in wave order.)"""
     if len(cum_wave_sizes) > MAX_WAVES:
         return None
     waves = _real_waves(wave_offsets, wave_sizes, cum_wave_sizes, causal=False, producer=False)
-    return _split_chain(waves, signal_offsets, units, True, dealt=True) if waves else None
+    return _split_dealt(waves, signal_offsets, units) if waves else None
 
 
 def _real_waves(wave_offsets, wave_sizes, cum_wave_sizes, *, causal: bool, producer: bool):
@@ -104,7 +108,7 @@ def _real_waves(wave_offsets, wave_sizes, cum_wave_sizes, *, causal: bool, produ
     return waves
 
 
-def _split_chain(waves, signal_offsets: Sequence[int], units: int, always: bool, dealt: bool) -> Optional[KvSplit]:
+def _split_runs(waves, signal_offsets: Sequence[int], units: int, always: bool) -> Optional[KvSplit]:
     size = waves[0][1]
     pairs = size[0] * size[1] * size[2] // (2 * BLOCK)
     lengths = [s[3] // BLOCK for _, s in waves]
@@ -118,42 +122,64 @@ def _split_chain(waves, signal_offsets: Sequence[int], units: int, always: bool,
     flagged = [n for n, signal in zip(lengths, signal_offsets) if signal >= 0]
     room = (always or pairs < units) and bool(flagged)
     best, best_us, whole_us = None, None, None
-    most = min(MAX_PARTS, total)
+    for parts in range(1, min(MAX_PARTS, total) + 1):
+        programs = pairs * parts
+        if pairs * (parts - 1) > MAX_SLOTS or (room and (always or parts > 1) and programs > units - RESERVED_UNITS):
+            continue
+        # What is left to do when the last chunk arrives late: its blocks, on the one part of a pair that has them, and the
+        # steps whose other sides are long there, against one round of its tiles.  (8 heads x 1024 rows, a chunk of 8 blocks
+        # every 10 us: as 7 parts 41 us behind the last flag, as tiles 25; 2 heads, 16 blocks, as 16 parts 49 and 40.)
+        if always and flagged and (min(-(-total // parts), flagged[-1]) * BLOCK_US + SEGMENT_US + 2.0 * _steps(parts) >
+                                   _tiles_us(2 * pairs, flagged[-1], units)):
+            continue
+        us = -(-programs // units) * (-(-total // parts) * BLOCK_US + SEGMENT_US + STEP_US * _steps(parts))
+        whole_us = whole_us or us
+        if best is None or us < best_us:
+            best, best_us = parts, us
     if always:
         tiles = 2 * pairs * len(waves)
         # visits to a q block that end at the same time are merged one after the other
         merges = min(len(waves), units // pairs) - 1 if tiles <= 2 * units else 0
         tiles_us = _tiles_us(tiles, -(-total // len(waves)), units) + MERGE_US * merges
-        if tiles_us < DEAL_HOST_US:
+        if best is None or best_us >= tiles_us:
             return None
-        if flagged:
-            last_us = _tiles_us(2 * pairs, flagged[-1], units)
-            if not dealt and min(-(-total // most), flagged[-1]) * BLOCK_US + SEGMENT_US > last_us:
-                return None                      # (however many parts)
-    for parts in range(1, most + 1):
-        programs = pairs * parts
-        if (parts > 1 and programs > MAX_SLOTS) or (room and (always or parts > 1) and programs > units - RESERVED_UNITS):
-            break
-        us = _deal_us(pairs, parts, total, units)
-        # What is left to do when the last chunk arrives late, against one round of its tiles.  Without `dealt` only tables
-        # that would end as early if one part had all its blocks; with it, the share of a part and the second kernel, and
-        # where that takes longer, the launch has to gain as much with every chunk there.
-        if always and flagged:
-            if not dealt and min(-(-total // parts), flagged[-1]) * BLOCK_US + SEGMENT_US + 2.0 * _steps(parts) > last_us:
-                continue
-            us += max(_deal_us(pairs, parts, flagged[-1], units, burst=False) - last_us, 0.0) if dealt else 0.0
-        whole_us = whole_us or us
-        if best is None or us < best_us:
-            best, best_us = parts, us
-    if always:
-        if best is None:
-            return None
-        # Whole pairs that leave units idle (135 of 28 blocks 102 us, as tiles 89), a gain within what the two models are off
-        # (560 whole pairs of 22 blocks 259 us, as tiles 225; 75 of 172 as two parts 295 and 277).  Over 1000 tables drawn anew (500 of them producers') four
+        # Whole pairs that leave units idle (135 of 28 blocks 102 us, as tiles 89), or whose gain is within what the two
+        # models are off (560 of 22 blocks 259 us, as tiles 225).  Over 1000 tables drawn anew (500 of them producers') four
         # lose more than 3 %, the most 7 % (324 pairs of 28 blocks), and the medians gain 20 to 39 %.
-        if (best == 1 and 8 * pairs < 7 * units) or 1.05 * best_us >= tiles_us:
+        if best == 1 and (8 * pairs < 7 * units or 1.05 * best_us >= tiles_us):
             return None
     elif best_us > min(0.85 * whole_us, whole_us - MIN_GAIN_US):
+        return None
+    return KvSplit(True, pairs, best, -(-total // best))
+
+
+def _split_dealt(waves, signal_offsets: Sequence[int], units: int) -> Optional[KvSplit]:
+    size = waves[0][1]
+    pairs = size[0] * size[1] * size[2] // (2 * BLOCK)
+    lengths = [s[3] // BLOCK for _, s in waves]
+    total = sum(lengths)
+    tiles = 2 * pairs * len(waves)
+    merges = min(len(waves), units // pairs) - 1 if tiles <= 2 * units else 0          # as in _split_runs
+    tiles_us = _tiles_us(tiles, -(-total // len(waves)), units) + MERGE_US * merges
+    if tiles_us < DEAL_HOST_US:
+        return None
+    flagged = [n for n, signal in zip(lengths, signal_offsets) if signal >= 0]
+    last_us = _tiles_us(2 * pairs, flagged[-1], units) if flagged else 0.0
+    best, best_us = None, None
+    for parts in range(1, min(MAX_PARTS, total) + 1):
+        programs = pairs * parts
+        if (parts > 1 and programs > MAX_SLOTS) or (flagged and programs > units - RESERVED_UNITS):
+            break
+        us = _deal_us(pairs, parts, total, units)
+        # What is left to do when the last chunk arrives late - the share of a part and the second kernel - against one round
+        # of its tiles: where that takes longer, the launch has to gain as much with every chunk there.
+        if flagged:
+            us += max(_deal_us(pairs, parts, flagged[-1], units, burst=False) - last_us, 0.0)
+        if best is None or us < best_us:
+            best, best_us = parts, us
+    # Whole pairs that leave units idle (135 of 28 blocks 102 us, as tiles 89), and a gain within what the two models are off (75
+    # of 172 as two parts 295 and 277).
+    if best is None or (best == 1 and 8 * pairs < 7 * units) or 1.05 * best_us >= tiles_us:
         return None
     return KvSplit(True, pairs, best, -(-total // best))
 

@@ -1,11 +1,11 @@
-"""Pairs of q blocks whose kv blocks are dealt to several programs one by one (SYN_ATTN_SPLIT_DEAL): the plan of tables that
-wait for flags (host), and launches at the sizes where the deal goes round differently."""
+"""Pairs of q blocks whose kv blocks are dealt to several programs one by one (SYN_ATTN_SPLIT_DEAL): the plan (host), which
+tables keep their parts in wave order instead, and launches at the sizes where the deal goes round differently."""
 
 import pytest
 import torch
 
 from oracle import numerics
-from syncopate_amd.computation.attn.kv_split import BLOCK, KvSplit, plan_kv_deal
+from syncopate_amd.computation.attn.kv_split import BLOCK, KvSplit, plan_kv_deal, plan_kv_split
 
 
 def _tables(Z, H, Sq, lengths, signals):
@@ -35,6 +35,70 @@ def test_plans_of_tables_that_wait():
     assert plan_kv_deal([[0, 0, 0, 0]], [[1, 1, 256, 128]], [0], [-1], units=256) is None
 
 
+@pytest.mark.parametrize("H,Sq,lengths,always,split", [
+    (49, 2816, [18 * 128] * 8, True, (539, 2)),       # more parts than slots, one of each pair's in registers
+    (50, 3072, [30 * 128] * 4, True, (600, 2)),
+    (8, 1024, [1024] * 8, True, (32, 8)),
+    (8, 1536, [1536] * 4, False, (48, 4)),            # the template's own call
+])
+def test_cut_in_wave_order(H, Sq, lengths, always, split):
+    """Tables whose parts have always been added in 32 bits: the parts in wave order that they had."""
+    got = plan_kv_split(*_tables(1, H, Sq, lengths, [-1] * len(lengths)), causal=False, producer=False, units=256, always=always)
+    assert (got.pairs, got.parts) == split and got.blocks == -(-sum(lengths) // (128 * split[1]))
+
+
+def _parts_by_hand(q, k, v, scale, parts):
+    """[rows, 128] of one head: each part's blocks in the order given, probabilities rounded against the maximum so far, and the
+    parts' sums added neighbour to neighbour."""
+    sums = []
+    for blocks in parts:
+        m, l, o = torch.full((len(q), 1), -3e38), torch.zeros(len(q), 1), torch.zeros(len(q), 128)
+        for b in blocks:
+            s = q.float() @ k[b * BLOCK:(b + 1) * BLOCK].float().T * (scale * 1.4426950408889634)
+            top = torch.maximum(m, s.max(dim=1, keepdim=True).values)
+            p = torch.exp2(s - top)
+            l = l * torch.exp2(m - top) + p.sum(dim=1, keepdim=True)
+            o = o * torch.exp2(m - top) + p.to(v.dtype).float() @ v[b * BLOCK:(b + 1) * BLOCK].float()
+            m = top
+        sums.append((m, l, o))
+    while len(sums) > 1:
+        pairs = [sums[i:i + 2] for i in range(0, len(sums), 2)]
+        sums = [pair[0] if len(pair) == 1 else _add(*pair) for pair in pairs]
+    return (sums[0][2] / sums[0][1]).to(q.dtype)
+
+
+def _add(a, b):
+    top = torch.maximum(a[0], b[0])
+    wa, wb = torch.exp2(a[0] - top), torch.exp2(b[0] - top)
+    return top, a[1] * wa + b[1] * wb, a[2] * wa + b[2] * wb
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lengths,parts,form", [([128 * 12], 4, "explicit"), ([128 * 5, 128 * 3, 128 * 7], 3, "auto"), ([128 * 9], 7, "auto")])
+def test_parts_in_wave_order_keep_their_results(hip, monkeypatch, lengths, parts, form):
+    """A table that `plan_kv_split` cuts gives the results of parts that are runs of blocks, whichever program adds them."""
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.attn import attention_forward
+
+    offsets, sizes, cums, signals = _tables(1, 1, 256, lengths, [-1] * len(lengths))
+    total = sum(lengths) // BLOCK
+    g = torch.Generator().manual_seed(11)
+    q, k, v = (torch.randn(1, 1, s, 128, generator=g).bfloat16() for s in (256, total * BLOCK, total * BLOCK))
+    each = -(-total // parts)
+    monkeypatch.setattr("syncopate_amd.computation.attn.template.plan_kv_split", lambda *args, **kwargs: KvSplit(True, 1, parts, each))
+    o = attention_forward(q.cuda(), k.cuda(), v.cuda(), 128 ** -0.5, wave_offsets=offsets, wave_sizes=sizes, cum_wave_sizes=cums,
+                          signal_offsets=signals, signal_ptr=torch.ones(1, dtype=torch.int64, device="cuda"), cum_tiles=cums[-1],
+                          form=form)
+    check_status()
+    real = -(-total // each)
+    runs = [range(total * i // real, total * (i + 1) // real) for i in range(real)]
+    want = _parts_by_hand(q[0, 0], k[0, 0], v[0, 0], 128 ** -0.5, runs)
+    # The same roundings of every probability, sums in 32 bits in another order: scores 2^-21 apart move one probability in 1000
+    # to the other side of a rounding and with it one result in 100 or 200.  Blocks met in another order round most of them
+    # anew and a third of the results.
+    assert (o[0, 0].cpu() == want).float().mean() >= 0.97
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout", ["bhsd", "bshd"])
 @pytest.mark.parametrize("Z,H,Sq,lengths,parts", [
@@ -55,7 +119,8 @@ def test_dealt_blocks_add_up(hip, monkeypatch, Z, H, Sq, lengths, parts, layout)
     g = torch.Generator().manual_seed(5)
     q, k, v = (torch.randn(Z, H, s, 128, generator=g).bfloat16() for s in (Sq, Skv, Skv))
     lay = lambda t: t if layout == "bhsd" else t.permute(0, 2, 1, 3).contiguous()
-    monkeypatch.setattr("syncopate_amd.computation.attn.template.plan_kv_split",
+    monkeypatch.setattr("syncopate_amd.computation.attn.template.plan_kv_split", lambda *args, **kwargs: None)
+    monkeypatch.setattr("syncopate_amd.computation.attn.template.plan_kv_deal",
                         lambda *args, **kwargs: KvSplit(True, Z * H * Sq // 256, parts, -(-Skv // (BLOCK * parts))))
     flags = torch.ones(waves, dtype=torch.int64, device="cuda")
     o, lse = attention_forward(lay(q).cuda(), lay(k).cuda(), lay(v).cuda(), 128 ** -0.5, wave_offsets=offsets + [[0] * 4],
