@@ -86,14 +86,14 @@ def zeroed_int32(shape, device: torch.device) -> torch.Tensor:
 
 
 def launches_on_stream(fn):
-    """Decorator of a launcher with a `stream` argument: the whole call - wave tables built
+    """Decorator of a launcher with a `stream` argument, by name or among its `**kwargs`: the whole call - wave tables built
     from lists or CPU tensors, zeroed counters, locks, outputs, and the kernel launch - runs
     with `stream` as torch's current stream.  The temporaries' fills are then ordered in front
     of the kernel, and the caching allocator hands their memory on only behind it."""
     parameters = inspect.signature(fn).parameters
-    if "stream" not in parameters:
-        return fn
-    positional = parameters["stream"].kind is inspect.Parameter.POSITIONAL_OR_KEYWORD
+    if "stream" not in parameters and not any(p.kind is inspect.Parameter.VAR_KEYWORD for p in parameters.values()):
+        raise TypeError(f"{fn.__name__} takes no stream")
+    positional = "stream" in parameters and parameters["stream"].kind is inspect.Parameter.POSITIONAL_OR_KEYWORD
     index = list(parameters).index("stream") if positional else None
 
     # (where `stream` stands is worked out once: binding the arguments on every call took 10 us, half of what a

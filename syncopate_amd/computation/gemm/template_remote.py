@@ -64,7 +64,6 @@ def _no_signals(num_waves: int, device_index: int):
                 torch.tensor([0], dtype=torch.int64, device=torch.device("cuda", device_index)))
 
 
-@launches_on_stream
 def _prepare_binding(lib, sizes, offsets, signals, flags, num_waves, M, N, K, block_m, block_n, block_k, cum_tiles,
                      a_list, a_target_rank, c_list, target_rank, dst_offsets, atomic_add, k_ranges, dev):
     """The host's share of a bound launch: table checks, and the device tables the kernel reads (pointer tables,
@@ -125,6 +124,7 @@ def _prepare_binding(lib, sizes, offsets, signals, flags, num_waves, M, N, K, bl
     return fields, keep
 
 
+@launches_on_stream
 def gemm_remote(
     a,
     b: torch.Tensor,
@@ -266,6 +266,7 @@ def gemm_remote(
     del keep, prepared
 
 
+@launches_on_stream
 def gemm_ag_direct_read(
     a,
     b,
@@ -299,6 +300,7 @@ def gemm_ag_direct_read(
                 a_target_rank=target_rank, cum_tiles=c.shape[0] * c.shape[1], **kwargs)
 
 
+@launches_on_stream
 def gemm_rs_producer_persistent(
     a,
     b,
@@ -342,6 +344,7 @@ def gemm_rs_producer_persistent(
                 dst_offsets=dst, atomic_add=True, cum_tiles=m * b.shape[0], **kwargs)
 
 
+@launches_on_stream
 def gemm_splitk(
     a: torch.Tensor,
     b: torch.Tensor,

@@ -85,6 +85,65 @@ def test_gemm_second_launch(hip, monkeypatch, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("launcher", ["gemm_consumer", "gemm_producer", "gemm_rs_producer_persistent", "gemm_remote", "gemm_splitk",
+                                      "gemm_ag_direct_read", "ring_reduce", "attention_forward"])
+def test_given_stream(hip, launcher):
+    """Calls with `stream`, after one without and again on the same operands: ordered with what was queued there in front of them,
+    the operand that arrives late and the zeroing of a C that is added to."""
+    from syncopate_amd.computation import attn, gemm, reduce
+    from syncopate_amd.computation._launch import check_status
+
+    g = torch.Generator(device="cuda").manual_seed(3)
+    randn = lambda *shape: (0.1 * torch.randn(shape, device="cuda", generator=g)).bfloat16()
+    m, n, k = 512, 512, 128
+    a, b, c = randn(m, k), randn(n, k), torch.zeros(m, n, dtype=torch.bfloat16, device="cuda")
+    sizes, offsets, waves = _table([[256, n]] * 2), _table([[0, 0], [256, 0]]), _table([0, 1])
+    flags = torch.ones(2, dtype=torch.int64, device="cuda")
+    halves, late, out = list(c.view(2, 256, n)), a, c
+    if launcher == "gemm_consumer":
+        call = lambda **kw: gemm.gemm_consumer(a, b, c, flags, sizes, offsets, waves, 2, 64, 128, 128, 64, 8, cum_tiles=m * n, **kw)
+    elif launcher == "gemm_producer":
+        call = lambda **kw: gemm.gemm_producer(a, b, c, flags, sizes, offsets, waves, 64, 128, 128, 64, 8, cum_tiles=m * n, **kw)
+    elif launcher == "gemm_rs_producer_persistent":
+        call = lambda **kw: gemm.gemm_rs_producer_persistent(a, b, halves, sizes, offsets, waves, 2, 2, 64, 128, 128, 64, 8, **kw)
+    elif launcher == "gemm_remote":
+        rows = _table([[0, 0], [0, 0]])
+        call = lambda **kw: gemm.gemm_remote(a, b, halves, 64, 128, 128, 64, 8, cur_wave_sizes=sizes, wave_offsets=offsets, M=m,
+                                             target_rank=waves, dst_offsets=rows, **kw)
+    elif launcher == "gemm_splitk":
+        boxes = _table([[m, n, 64]] * 2), _table([[0, 0, 0], [0, 0, 64]])
+        call = lambda **kw: gemm.gemm_splitk(a, b, c, 2, 64, 128, 128, 64, 8, cur_wave_sizes=boxes[0], wave_offsets=boxes[1],
+                                             cum_tiles=2 * m * n, **kw)
+    elif launcher == "gemm_ag_direct_read":
+        call = lambda **kw: gemm.gemm_ag_direct_read(list(a.view(2, 256, k)), b, c, sizes, offsets, waves, 2, 2, 64,
+                                                     BLOCK_SIZE_N=128, **kw)
+    elif launcher == "ring_reduce":
+        late, out = randn(2, 256, n), torch.zeros(256, n, dtype=torch.bfloat16, device="cuda")
+        call = lambda **kw: reduce.ring_reduce(late, out, c, 0, **kw)
+    else:
+        q, late, out = randn(1, 1, 256, 128), randn(1, 1, 256, 128), torch.zeros(1, 1, 256, 128, dtype=torch.bfloat16, device="cuda")
+        tables = dict(wave_offsets=_table([[0, 0, 0, 0]]), wave_sizes=_table([[1, 1, 256, 256]]), cum_wave_sizes=_table([256]),
+                      signal_offsets=_table([0]), cum_tiles=256)
+        call = lambda **kw: attn.attention_forward(q, late, late, 0.1, signal_ptr=flags, output_buffer=out, **tables, **kw)
+    call()
+    torch.cuda.synchronize()
+    want, real, lib = out.clone(), late.clone(), _lib.load()
+    assert want.abs().max() > 0 or launcher == "ring_reduce"
+    side = torch.cuda.Stream()
+    for _ in range(3):
+        late.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            _lib.check("syn_delay_us", lib.syn_delay_us(5000, _lib.stream_handle(side)))
+            late.copy_(real)
+            out.zero_()
+        call(stream=side)
+        side.synchronize()
+        check_status()
+        assert torch.equal(out, want)
+
+
+@pytest.mark.gpu
 def test_threads_and_streams(hip):
     """Producers of two threads on streams of their own, more launches than a pool of counters has areas."""
     from syncopate_amd.computation._launch import check_status
