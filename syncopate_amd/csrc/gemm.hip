@@ -1117,6 +1117,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
     __syncthreads();
     int waves_up = uniform(s_waves_up);
     if (p.acquire_always && uniform(s_spun)) acquire_fence_agent();
+    __syncthreads();       // wait_flag writes both words: only when everyone has read them
 
     // --- wave walk state (uniform across the workgroup) ---
     int cur_wave = -1, past_tiles = 0, cur_tiles = 0;
