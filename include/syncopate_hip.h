@@ -382,7 +382,7 @@ typedef struct syn_attn_desc {
  * block b (counted over all waves in a row) to part b % split_parts, so that every program goes through all chunks and a
  * chunk that comes late is spread over all of them.  split_blocks and split_nodes are not read.  split_parts > 1: every part
  * leaves its sums in a slot of its own, split_partials holds pairs * split_parts of them, and a second kernel of the same
- * call adds them up in the order of the parts.  Workgroup b works on part b % split_parts of pair b / split_parts (dealt
+ * call adds them up in the order of the parts (a pair of which a part gave up, see status, is left as it was).  Workgroup b works on part b % split_parts of pair b / split_parts (dealt
  * to the XCDs within rounds of 256 workgroups).  No counterpart in the reference. */
 #define SYN_ATTN_SPLIT_DEAL 64u
 #define SYN_ATTN_SPLIT_SLOT_BYTES 139264

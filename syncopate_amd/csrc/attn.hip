@@ -808,6 +808,11 @@ __device__ __forceinline__ void store_partial(unsigned char* slot, const f32x4_t
     store16(dst + 16 * 1024, f32x4_t{m[0], m[1], l[0], l[1]});
 }
 
+// In a slot whose part has not stored (yet), for attn_add_parts_kernel: row sums of -1, which no part has.
+__device__ __forceinline__ void mark_partial_missing(unsigned char* slot, int wave8, int lane) {
+    *reinterpret_cast<f32x4_t*>(slot + (((size_t)wave8 * kPartialRecords + 16) * 64 + lane) * 16) = f32x4_t{0.f, 0.f, -1.f, -1.f};
+}
+
 // The sum of two partial results.  Each product is rounded by itself (no fused multiply-add), so that a + b and b + a are
 // the same bits: which of two programs arrives second, and adds, does not show in the result.
 __device__ __forceinline__ void add_partial(const unsigned char* slot, f32x4_t (&o_acc)[8][2], float (&m)[2], float (&l)[2],
@@ -964,6 +969,13 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
     const unsigned char* __restrict__ V = reinterpret_cast<const unsigned char*>(p.v);
     T* __restrict__ O = reinterpret_cast<T*>(p.o);
 
+    const int program = kSplitChain ? (int)blockIdx.x
+                        : kSplit    ? logical_program_id_by_rounds((int)blockIdx.x, (int)gridDim.x, kUnits, p.xcd_remap != 0)
+                                    : logical_program_id((int)blockIdx.x, (int)gridDim.x, p.xcd_remap != 0);
+    if constexpr (kDeal) {
+        if (p.split_parts > 1) mark_partial_missing(p.split_partials + (size_t)program * kPartialSlotBytes, wave8, lane);
+    }
+
     const int pairs_per_wave = p.cum_wave_sizes[0] / kBlockM / 2;
     const int num_pairs = MODE == kPairChainWaves || kSplitChain || kDeal ? pairs_per_wave : p.num_tiles / 2;
     if (kSplit && (int)gridDim.x != num_pairs * p.split_parts) {
@@ -974,9 +986,6 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
         if (tid == 0) report_status(p.status, SYN_STATUS_BAD_CHAIN, 0, (int)blockIdx.x, pairs_per_wave);
         return;
     }
-    const int program = kSplitChain ? (int)blockIdx.x
-                        : kSplit    ? logical_program_id_by_rounds((int)blockIdx.x, (int)gridDim.x, kUnits, p.xcd_remap != 0)
-                                    : logical_program_id((int)blockIdx.x, (int)gridDim.x, p.xcd_remap != 0);
 
     // where the program stands: the next pair of the table (kPairTiles, kPairChainWaves) or the entry of its list
     int pair = program;
@@ -1855,7 +1864,9 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
 
 // What follows kPairSplitDeal: the sum of a pair's parts, in the order of the parts, written as whole rows.  A workgroup per
 // wavefront of the pair (32 q rows); each of its own eight wavefronts takes the 16 rows of one half and 32 columns, reads the
-// parts' statistics and two records of each part, four parts at a time, and writes 64 bytes of a row.
+// parts' statistics and two records of each part, four parts at a time, and writes 64 bytes of a row.  A pair of which a part
+// has not stored (the first kernel found the table another than the launch was planned for, or gave up on a flag, and has said so) and
+// rows outside the result are left alone.
 template <typename T>
 __global__ void __launch_bounds__(kPairThreads) attn_add_parts_kernel(const AttnParams p) {
     typedef T vec4_t __attribute__((ext_vector_type(4)));
@@ -1868,6 +1879,7 @@ __global__ void __launch_bounds__(kPairThreads) attn_add_parts_kernel(const Attn
     const unsigned char* const src = p.split_partials + (size_t)pair * parts * kPartialSlotBytes +
                                      ((size_t)wave8 * kPartialRecords * 64 + lane) * 16;
 
+    bool missing = false;
     float top = -FLT_MAX, l = 0.f;
     f32x4_t sum[2] = {};
     for (int first = 0; first < parts; first += kAtOnce) {
@@ -1882,6 +1894,7 @@ __global__ void __launch_bounds__(kPairThreads) attn_add_parts_kernel(const Attn
         float m[kAtOnce], new_top = top;
 #pragma unroll
         for (int i = 0; i < kAtOnce; ++i) {
+            missing = missing || stats[i][2 + b] < 0.f;
             m[i] = stats[i][b];
             new_top = fmaxf(new_top, m[i]);
         }
@@ -1900,10 +1913,13 @@ __global__ void __launch_bounds__(kPairThreads) attn_add_parts_kernel(const Attn
         }
     }
 
+    // (looked at here, behind the loads, which lie in the slots whatever the table says)
     const int size_h = p.wave_sizes[1], nq = p.wave_sizes[2] / kBlockM;
+    if (missing || (int)gridDim.x != p.cum_wave_sizes[0] / kBlockM / 2 * 8 || size_h <= 0 || nq <= 0) return;
     const int tile = 2 * pair + (wave8 >> 2);
     const int z = tile / (nq * size_h) + p.wave_offsets[0], h = (tile / nq) % size_h + p.wave_offsets[1];
     const int row = (tile % nq + p.wave_offsets[2] / kBlockM) * kBlockM + (wave8 & 3) * 32 + 16 * b + c16;
+    if ((unsigned)z >= (unsigned)p.Z || (unsigned)h >= (unsigned)p.H || (unsigned)row >= (unsigned)p.Sq) return;
     const float inv_l = 1.0f / l;
     T* const out = reinterpret_cast<T*>(p.o) + z * p.o_st[0] + h * p.o_st[1] + row * p.o_st[2] + 16 * t0 + 4 * g;
 #pragma unroll

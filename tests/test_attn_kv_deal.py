@@ -167,3 +167,41 @@ def test_chunks_that_come_late(hip, trusted):
             _lib.check("syn_flag_set", lib.syn_flag_set(flags.data_ptr() + 8 * ((first + 2 * i) % 7), 1, _lib.stream_handle(side)))
         check_status()
         assert torch.equal(o, resident)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["fewer pairs", "other rows", "flag that stays down", "flag of the last wave"])
+def test_refused_launch_writes_nothing(hip, monkeypatch, what):
+    """A table that is not the one the launch was planned for, or a flag that does not come: the first kernel says so, and the second
+    leaves the result as it was."""
+    from syncopate_amd import _lib
+    from syncopate_amd.computation._launch import FlagWaitTimeout, check_status
+    from syncopate_amd.computation.attn import attention_forward, template
+
+    H, parts = 2, 3
+    offsets, sizes, cums, signals = _tables(1, H, 256, [512, 512], [-1, -1])
+    flags = torch.ones(2, dtype=torch.int64, device="cuda")
+    pairs, timeout = H, {}
+    if what == "fewer pairs":
+        pairs = 2 * H
+    elif what == "other rows":
+        offsets[1][2] = 256
+    else:
+        signals = [0, 1] if what == "flag that stays down" else [-1, 1]
+        flags[signals[0] if signals[0] >= 0 else 1] = 0
+        timeout = dict(spin_timeout_us=2000)
+    monkeypatch.setattr(template, "plan_kv_split", lambda *args, **kwargs: None)
+    monkeypatch.setattr(template, "plan_kv_deal", lambda *args, **kwargs: KvSplit(True, pairs, parts, -(-8 // parts)))
+    monkeypatch.setattr(template, "already_checked", lambda *args: True)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q, k, v = (torch.randn(1, H, s, 128, device="cuda", generator=g).bfloat16() for s in (512, 1024, 1024))
+    # results of another launch where the allocator will put the parts
+    stale = torch.full((pairs * parts * _lib.SYN_ATTN_SPLIT_SLOT_BYTES,), 1, dtype=torch.uint8, device="cuda")
+    del stale
+    table = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    out = torch.full_like(q, 7.0)
+    attention_forward(q, k, v, 0.1, wave_offsets=table(offsets), wave_sizes=table(sizes), cum_wave_sizes=table(cums),
+                      signal_offsets=table(signals), signal_ptr=flags, cum_tiles=cums[-1], out=out, **timeout)
+    with pytest.raises(FlagWaitTimeout if timeout else RuntimeError, match="timed out" if timeout else rf"\[{_lib.SYN_STATUS_BAD_CHAIN}, "):
+        check_status()
+    assert bool((out == 7.0).all())
