@@ -74,6 +74,21 @@ def table_visits(wave_offsets: Sequence[Sequence[int]], wave_sizes: Sequence[Seq
     return visits
 
 
+def chains_visits(visits: Sequence[Visit], num_programs: int) -> bool:
+    """Whether `plan_attention_work` with "fair" segments keeps the sums of two visits to a pair in registers: it does where two visits in
+    a row are no longer than a program's fair share (cutting from the last visit on, the later one begins a piece that the
+    earlier one fits, or is in a longer one already)."""
+    fair = sum(v.kv_blocks for v in visits) / num_programs
+    before: Dict[Tuple[int, int, int], int] = {}
+    for v in visits:
+        if v.kv_blocks == 0:
+            continue
+        if before.get(v.key, fair) + v.kv_blocks <= fair:
+            return True
+        before[v.key] = v.kv_blocks
+    return False
+
+
 def plan_attention_work(wave_offsets, wave_sizes, cum_wave_sizes, *, causal: bool, num_programs: int,
                         max_visits: Optional[int] = None, max_blocks: Optional[float] = None,
                         group_heads: bool = True, list_masked_visits: bool = False,
