@@ -930,7 +930,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
             const int sg = lane < p.num_waves && p.cum_wave_sizes[lane] != 0 ? p.signal_offsets[lane] : -1;
             const bool up = sg < 0 || __hip_atomic_load(p.flags + sg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 1ull;
             const unsigned long long down = ~__builtin_amdgcn_ballot_w64(up);
-            if (lane == 0) s_waves_up = down == 0 ? 64 : (int)__builtin_ctzll(down);
+            if (lane == 0) s_waves_up = p.acquire_always ? 0 : down == 0 ? 64 : (int)__builtin_ctzll(down);
         }
     }
 
@@ -1093,10 +1093,11 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
         return ok;
     };
     // kPairSplitDeal: a part enters a wave every few blocks.  The flags of the next 64 waves are read at once, one per lane, and
-    // those in a row that are up are not looked at again (a flag goes up once per launch).
+    // those in a row that are up are not looked at again (a flag goes up once per launch; under SYN_ATTN_ACQUIRE_ALWAYS, whose
+    // caller need not promise that, each wave's flag is read when the wave is entered).
     int waves_up = 0, real_waves = 0;
     auto wait_for_wave = [&](const int wv) __attribute__((always_inline)) -> bool {
-        if (wv < waves_up) return true;
+        if (wv < waves_up || (p.acquire_always && __builtin_amdgcn_readfirstlane(s_row[wv][7]) < 0)) return true;
         if (wave8 == 0) {
             const int idx = wv + lane;
             const int sg = idx < real_waves ? s_row[idx][7] : -1;
@@ -1104,7 +1105,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
             const unsigned long long down = ~__builtin_amdgcn_ballot_w64(up);
             if (lane == 0) {
                 s_spun = (int)(down & 1);
-                s_waves_up = wv + (down == 0 ? 64 : max((int)__builtin_ctzll(down), 1));
+                s_waves_up = wv + (p.acquire_always ? 1 : down == 0 ? 64 : max((int)__builtin_ctzll(down), 1));
                 if (s_spun && !spin_until_equal(p.flags + sg, 1ull, p.timeout_ticks)) {
                     report_status(p.status, SYN_STATUS_SPIN_TIMEOUT, wv, (int)blockIdx.x, sg);
                     s_abort = 1;
@@ -1160,7 +1161,6 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
         parts = p.split_parts;
         part_left = before > part ? (before - part + parts - 1) / parts : 0;
         waves_up = __builtin_amdgcn_readfirstlane(s_waves_up);
-        if (p.acquire_always && waves_up > 0) acquire_fence_agent();
     }
 
     for (; pending(); advance()) {

@@ -1097,7 +1097,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
     if (tid == 0) s_abort = 0;
     // Which waves need not be waited for.  Flags are read for 64 waves at a time, a lane each - here for the first ones, beside the
     // table, and whenever a wave has to be waited for - and those in a row that are up are not looked at again: a flag goes up
-    // once per launch, and a program visits the waves in order.  With every chunk there, no program stops at a wave.
+    // once per launch, and a program visits the waves in order.  With every chunk there, no program stops at a wave.  Under
+    // SYN_GEMM_ACQUIRE_ALWAYS, whose caller need not promise that, each wave's flag is read when the wave is entered.
     // Wavefront 0: flag index per wave, -1: none.
     auto wait_index = [&](int w) -> int {
         if (w >= p.num_waves) return -1;
@@ -1107,17 +1108,12 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
     if (wave == 0) {
         const int sig = wait_index(lane);
         const bool up = sig < 0 || __hip_atomic_load(wait_on + sig, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 1ull;
-        const unsigned long long down = ~__builtin_amdgcn_ballot_w64(up), flagged = __builtin_amdgcn_ballot_w64(sig >= 0);
-        if (lane == 0) {
-            const int row = down == 0 ? 64 : (int)__builtin_ctzll(down);
-            s_waves_up = row;
-            s_spun = (flagged & (row == 64 ? ~0ull : (1ull << row) - 1)) != 0;
-        }
+        const unsigned long long down = ~__builtin_amdgcn_ballot_w64(up);
+        if (lane == 0) s_waves_up = p.acquire_always ? 0 : down == 0 ? 64 : (int)__builtin_ctzll(down);
     }
     __syncthreads();
     int waves_up = uniform(s_waves_up);
-    if (p.acquire_always && uniform(s_spun)) acquire_fence_agent();
-    __syncthreads();       // wait_flag writes both words: only when everyone has read them
+    __syncthreads();       // wait_flag writes the word: only when everyone has read it
 
     // --- wave walk state (uniform across the workgroup) ---
     int cur_wave = -1, past_tiles = 0, cur_tiles = 0;
@@ -1168,7 +1164,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
             const bool up = sig < 0 || __hip_atomic_load(wait_on + sig, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 1ull;
             const unsigned long long down = ~__builtin_amdgcn_ballot_w64(up);
             if (lane == 0) {
-                s_waves_up = cur_wave + (down == 0 ? 64 : max((int)__builtin_ctzll(down), 1));
+                s_waves_up = cur_wave + (p.acquire_always ? 1 : down == 0 ? 64 : max((int)__builtin_ctzll(down), 1));
                 s_spun = (int)(down & 1);
                 if (s_spun && !spin_until_equal(wait_on + sig, 1ull, p.timeout_ticks)) {
                     report_status(p.status, SYN_STATUS_SPIN_TIMEOUT, cur_wave, pid, sig);
