@@ -24,7 +24,8 @@ def status_words(device: torch.device) -> torch.Tensor:
     idx = device.index if device.index is not None else torch.cuda.current_device()
     buf = _status.get(idx)
     if buf is None:
-        buf = torch.zeros(_lib.SYN_STATUS_WORDS, dtype=torch.int32, device=torch.device("cuda", idx))
+        with torch.inference_mode(False):        # (written to outside the mode of the first launch, too)
+            buf = torch.zeros(_lib.SYN_STATUS_WORDS, dtype=torch.int32, device=torch.device("cuda", idx))
         _status[idx] = buf
     return buf
 
@@ -76,7 +77,9 @@ def zeroed_int32(shape, device: torch.device) -> torch.Tensor:
     if pool is None:
         if len(_ZERO_POOLS) > 64:
             _ZERO_POOLS.clear()       # (the allocator hands a dropped pool's memory on in stream order)
-        pool = _ZERO_POOLS[key] = [torch.zeros((ZERO_POOL_SLICES,) + shape, dtype=torch.int32, device=device), 0]
+        # (a pool outlives the mode that the first launch came in: an inference tensor could not be filled again outside of it)
+        with torch.inference_mode(False):
+            pool = _ZERO_POOLS[key] = [torch.zeros((ZERO_POOL_SLICES,) + shape, dtype=torch.int32, device=device), 0]
     elif pool[1] >= ZERO_POOL_SLICES:
         pool[0].zero_()
         pool[1] = 0

@@ -13,6 +13,7 @@
 #include <ATen/TensorSubclassLikeUtils.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/zeros.h>
+#include <c10/core/InferenceMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
@@ -156,6 +157,8 @@ struct Pool {
 std::map<std::tuple<int, void*, int64_t, std::thread::id>, Pool> g_pools;
 
 int32_t* zeroed(int dev, int64_t words, at::Tensor* keep) {
+    // (the areas outlive the mode that the first launch came in: an inference tensor could not be filled again outside of it)
+    const c10::InferenceMode ordinary(false);
     void* stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream();
     const auto key = std::make_tuple(dev, stream, words, std::this_thread::get_id());
     auto found = g_pools.find(key);

@@ -144,6 +144,28 @@ def test_given_stream(hip, launcher):
 
 
 @pytest.mark.gpu
+def test_first_launches_inside_inference_mode(hip):
+    """The pools of zeroed words, of the native launches and of the launchers, are made inside the mode and filled again outside."""
+    from syncopate_amd.computation._launch import ZERO_POOL_SLICES, check_status, zeroed_int32
+
+    run, want, *_ = _gemm_case("producer")
+    with torch.cuda.stream(torch.cuda.Stream()):
+        torch.cuda.current_stream().wait_stream(torch.cuda.default_stream())
+        run()                                            # (remembers the tables; a pool of this stream is still to be made)
+        with torch.inference_mode():
+            assert (run().float() - want).abs().max() <= 4e-3 * want.abs().max()
+        for _ in range(20):
+            assert (run().float() - want).abs().max() <= 4e-3 * want.abs().max()
+        with torch.inference_mode():
+            zeroed_int32((7,), torch.device("cuda", 0))
+        for _ in range(ZERO_POOL_SLICES + 1):
+            words = zeroed_int32((7,), torch.device("cuda", 0))
+            assert not words.any()
+            words.fill_(1)
+    check_status()
+
+
+@pytest.mark.gpu
 def test_threads_and_streams(hip):
     """Producers of two threads on streams of their own, more launches than a pool of counters has areas."""
     from syncopate_amd.computation._launch import check_status
