@@ -80,6 +80,8 @@ int64_t as_int(PyObject* obj, bool* ok) {
     return (int64_t)v;
 }
 
+int64_t stream_of(int dev) { return reinterpret_cast<int64_t>(c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream()); }
+
 // the launch of `fn` on the current stream, without the interpreter's lock
 template <typename F>
 int launch(int dev, F&& fn) {
@@ -101,48 +103,55 @@ bool capturing(int dev) {
 
 // ---------------------------------------------------------------- what is known about a set of tables
 
+// A launch is known by its kind, the tables' objects and what `params` lists: sizes, options, for C bound to buffers their addresses,
+// and the stream, so that the device tables a record keeps are given back in the order of the stream that reads them.
 struct Known {
     std::vector<c10::weak_intrusive_ptr<c10::TensorImpl>> tables;
     std::vector<int64_t> versions;
-    std::vector<int64_t> params;
     at::Tensor status;
     std::vector<at::Tensor> keep;            // device tables the descriptor points into
     syn_gemm_desc gemm = {};
     syn_gemm_remote remote = {};
     syn_attn_desc attn = {};
     int64_t lock_words = 0, node_words = 0, partial_bytes = 0;
+
+    // (a weak reference keeps its address from being handed out again: the same address and alive is the same tensor)
+    bool alive() const {
+        for (const auto& t : tables)
+            if (t.expired()) return false;
+        return true;
+    }
 };
-// by kind of launch and the tables' objects
-typedef std::vector<const void*> Key;
+typedef std::vector<int64_t> Key;
 std::map<Key, Known> g_known;
 
-Key key_of(int64_t kind, const std::vector<const at::Tensor*>& tables) {
+Key key_of(int64_t kind, const std::vector<const at::Tensor*>& tables, const std::vector<int64_t>& params) {
     Key key;
-    key.reserve(tables.size() + 1);
-    key.push_back(reinterpret_cast<const void*>(kind));
-    for (const at::Tensor* t : tables) key.push_back(t->unsafeGetTensorImpl());
+    key.reserve(1 + tables.size() + params.size());
+    key.push_back(kind);
+    for (const at::Tensor* t : tables) key.push_back(reinterpret_cast<int64_t>(t->unsafeGetTensorImpl()));
+    key.insert(key.end(), params.begin(), params.end());
     return key;
 }
 
 const Known* recall(int64_t kind, const std::vector<const at::Tensor*>& tables, const std::vector<int64_t>& params) {
-    const auto found = g_known.find(key_of(kind, tables));
-    if (found == g_known.end()) return nullptr;
-    const Known& k = found->second;
-    if (k.params != params) return nullptr;
-    for (size_t i = 0; i < tables.size(); ++i) {
-        // (a weak reference keeps its address from being handed out again: the same address and alive is the same tensor)
-        if (k.tables[i].expired() || (int64_t)tables[i]->_version() != k.versions[i]) return nullptr;
-    }
-    return &k;
+    const auto found = g_known.find(key_of(kind, tables, params));
+    if (found == g_known.end() || !found->second.alive()) return nullptr;
+    for (size_t i = 0; i < tables.size(); ++i)
+        if ((int64_t)tables[i]->_version() != found->second.versions[i]) return nullptr;
+    return &found->second;
 }
 
-void remember(int64_t kind, const std::vector<const at::Tensor*>& tables, Known&& k) {
+void remember(int64_t kind, const std::vector<const at::Tensor*>& tables, const std::vector<int64_t>& params, Known&& k) {
     for (const at::Tensor* t : tables) {
         k.tables.emplace_back(t->getIntrusivePtr());
         k.versions.push_back((int64_t)t->_version());
     }
-    if (g_known.size() >= kMaxRecords) g_known.clear();
-    g_known[key_of(kind, tables)] = std::move(k);
+    if (g_known.size() >= kMaxRecords) {
+        for (auto i = g_known.begin(); i != g_known.end();) i = i->second.alive() ? std::next(i) : g_known.erase(i);
+        if (g_known.size() >= kMaxRecords) g_known.clear();
+    }
+    g_known[key_of(kind, tables, params)] = std::move(k);
 }
 
 // ---------------------------------------------------------------- zeroed work areas
@@ -232,8 +241,8 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     NEED(flag_words(*flags));
     bool ok = true;
     const bool producer = as_int(args[15], &ok) != 0, acquire = as_int(args[16], &ok) != 0;
-    std::vector<int64_t> params = {g.M, g.N, g.K, g.dtype, g.dev, flags->numel()};
-    params.reserve(16);
+    std::vector<int64_t> params = {g.M, g.N, g.K, g.dtype, g.dev, stream_of(g.dev), flags->numel()};
+    params.reserve(18);
     for (int i = 7; i < 15; ++i) params.push_back(as_int(args[i], &ok));
     NEED(ok);
     for (const at::Tensor* t : tables) params.push_back(t->numel());
@@ -243,9 +252,8 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
         NEED(status && PyBytes_Check(args[17]) && PyBytes_GET_SIZE(args[17]) == (Py_ssize_t)sizeof(syn_gemm_desc));
         Known k;
         memcpy(&k.gemm, PyBytes_AS_STRING(args[17]), sizeof k.gemm);
-        k.params = std::move(params);
         k.status = *status;
-        remember(kind, tables, std::move(k));
+        remember(kind, tables, params, std::move(k));
         Py_RETURN_NONE;
     }
     const Known* k = recall(kind, tables, params);
@@ -285,10 +293,10 @@ PyObject* remote(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     bool ok = true;
     const Py_ssize_t buffers = PyList_GET_SIZE(args[2]);
-    std::vector<int64_t> params = {g.M, g.N, g.K, g.dtype, g.dev};
-    params.reserve(18 + 3 * (size_t)buffers);
+    std::vector<int64_t> params = {g.M, g.N, g.K, g.dtype, g.dev, stream_of(g.dev)};
+    params.reserve(20 + 3 * (size_t)buffers);
     for (int i = 7; i < 17; ++i) params.push_back(as_int(args[i], &ok));
-    NEED(ok && params[12] == g.M);
+    NEED(ok && params[13] == g.M);
     for (const at::Tensor* t : tables) params.push_back(t->numel());
     for (Py_ssize_t i = 0; i < buffers; ++i) {
         const at::Tensor* c = plain(PyList_GET_ITEM(args[2], i), g.dev);
@@ -310,9 +318,8 @@ PyObject* remote(PyObject*, PyObject* const* args, Py_ssize_t n) {
             NEED(t);
             k.keep.push_back(*t);
         }
-        k.params = std::move(params);
         k.status = *status;
-        remember(kKindRemote, tables, std::move(k));
+        remember(kKindRemote, tables, params, std::move(k));
         Py_RETURN_NONE;
     }
     const Known* k = recall(kKindRemote, tables, params);
@@ -386,7 +393,7 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     bool ok = true;
     std::vector<int64_t> params;
-    params.reserve(16);
+    params.reserve(20);
     for (int i = 9; i < 14; ++i) params.push_back(as_int(args[i], &ok));      // num_waves, cum_tiles, causal, bshd, auto
     const bool return_lse = as_int(args[16], &ok) != 0, acquire = as_int(args[17], &ok) != 0;
     const double scale = PyFloat_AsDouble(args[3]);
@@ -403,7 +410,7 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
         counters = plain(args[14], dev);
         NEED(counters && counters->scalar_type() == at::kInt && counters->is_contiguous());
     }
-    for (const int64_t x : {Z, H, Sq, Skv, flags->numel(), (int64_t)dev, (int64_t)(counters != nullptr)}) params.push_back(x);
+    for (const int64_t x : {Z, H, Sq, Skv, flags->numel(), (int64_t)dev, stream_of(dev), (int64_t)(counters != nullptr)}) params.push_back(x);
     for (const at::Tensor* t : tables) params.push_back(t->numel());
 
     if (n == 24) {
@@ -420,9 +427,8 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
         r.node_words = as_int(args[22], &ok);
         r.partial_bytes = as_int(args[23], &ok);
         NEED(ok);
-        r.params = std::move(params);
         r.status = *status;
-        remember(kKindAttn, tables, std::move(r));
+        remember(kKindAttn, tables, params, std::move(r));
         Py_RETURN_NONE;
     }
     const Known* known = recall(kKindAttn, tables, params);

@@ -144,6 +144,44 @@ def test_given_stream(hip, launcher):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("differ", ["buffers", "programs", "tile", "stream"])
+def test_launches_in_turn_on_one_set_of_tables(hip, monkeypatch, differ):
+    """Launches that share their tables and differ in something else are known side by side."""
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.gemm import gemm_consumer, gemm_rs_producer_persistent, template, template_remote
+
+    m, n, k = 512, 512, 192
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a, b = ((0.1 * torch.randn(s, k, device="cuda", generator=g)).bfloat16() for s in (m, n))
+    sizes, offsets, waves = _table([[256, n]] * 2), _table([[0, 0], [256, 0]]), _table([0, 1])
+    flags = torch.ones(2, dtype=torch.int64, device="cuda")
+    results = [torch.zeros(2, 256, n, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    bound, streams = [list(c) for c in results], [torch.cuda.current_stream(), torch.cuda.Stream()]
+    general, convert = [], template.as_device_table
+    for module in (template, template_remote):
+        monkeypatch.setattr(module, "as_device_table", lambda *args: general.append(1) or convert(*args))
+    want = (a.float() @ b.float().T).view(2, 256, n)
+    for turn in range(6):
+        which = turn % 2
+        into, programs, bn = which if differ == "buffers" else 0, 48 + 16 * (differ == "programs" and which), 128 << (differ == "tile" and which)
+        results[into].zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[which if differ == "stream" else 0]):
+            gemm_rs_producer_persistent(a, b, bound[into], sizes, offsets, waves, 2, 2, programs, 128, bn, 64, 8)
+            torch.cuda.synchronize()
+            # one rounding of the result (2^-9 relative), sums in 32 bits
+            assert (results[into].float() - want).abs().max() <= 4e-3 * want.abs().max()
+            results[into].zero_()
+            gemm_consumer(a, b, results[into].view(m, n), flags, sizes, offsets, waves, 2, programs, 128, bn, 64, 8, cum_tiles=m * n)
+            torch.cuda.synchronize()
+            assert (results[into].float() - want).abs().max() <= 4e-3 * want.abs().max()
+        if turn == 1:
+            general.clear()
+    check_status()
+    assert not general
+
+
+@pytest.mark.gpu
 def test_first_launches_inside_inference_mode(hip):
     """The pools of zeroed words, of the native launches and of the launchers, are made inside the mode and filled again outside."""
     from syncopate_amd.computation._launch import ZERO_POOL_SLICES, check_status, zeroed_int32
