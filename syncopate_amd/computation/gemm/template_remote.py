@@ -64,6 +64,16 @@ def _no_signals(num_waves: int, device_index: int):
                 torch.tensor([0], dtype=torch.int64, device=torch.device("cuda", device_index)))
 
 
+def _read_here(tables: Sequence[torch.Tensor], streams: set, dev: torch.device) -> None:
+    """Notes that the current stream reads `tables`, which are kept with the caller's: their memory is handed on behind what it reads.
+    `streams`: those for which that is done.  (A captured launch reads its tables whenever its graph is replayed.)"""
+    here = _lib.current_stream_handle(dev.index)
+    if here not in streams and not torch.cuda.is_current_stream_capturing():
+        for t in tables:
+            t.record_stream(torch.cuda.current_stream(dev))
+        streams.add(here)
+
+
 def _prepare_binding(lib, sizes, offsets, signals, flags, num_waves, M, N, K, block_m, block_n, block_k, cum_tiles,
                      a_list, a_target_rank, c_list, target_rank, dst_offsets, atomic_add, k_ranges, dev):
     """The host's share of a bound launch: table checks, and the device tables the kernel reads (pointer tables,
@@ -219,15 +229,15 @@ def gemm_remote(
     params = (M, N, K, BLOCK_SIZE_M, BLOCK_SIZE_N, BLOCK_SIZE_K, int(cum_tiles), flags.numel(), bool(atomic_add),
               None if a_list is None else tuple((t.data_ptr(), t.shape[0]) for t in a_list),
               None if c_list is None else tuple((t.data_ptr(), tuple(t.shape)) for t in c_list))
-    note = f"remote binding, stream {_lib.current_stream_handle(dev.index)}"      # (its tables are read, and given back, in that order)
-    prepared = recall_note(given, note) if caller_owned else None
+    prepared = recall_note(given, "remote binding") if caller_owned else None
     if prepared is None or prepared[0] != params:
         prepared = (params, _prepare_binding(lib, sizes, offsets, signals, flags, num_waves, M, N, K, BLOCK_SIZE_M, BLOCK_SIZE_N,
                                              BLOCK_SIZE_K, cum_tiles, a_list, a_target_rank, c_list, target_rank, dst_offsets,
-                                             atomic_add, k_ranges, dev))
+                                             atomic_add, k_ranges, dev), set())
         if caller_owned:
-            remember_note(given, note, prepared)
+            remember_note(given, "remote binding", prepared)
     fields, keep = prepared[1]
+    _read_here(keep, prepared[2], dev)
     remote = _lib.GemmRemote()
     for name, value in fields.items():
         setattr(remote, name, value)
@@ -334,13 +344,12 @@ def gemm_rs_producer_persistent(
     # rows are wave-local in the owner's buffer, columns keep their global position
     # (template_rs.py:157-166: offs_cm from the wave-local pid_m, offs_bn from the global pid_n)
     owned = isinstance(wave_offset, torch.Tensor) and wave_offset.is_cuda
-    note = f"owner slot offsets, stream {_lib.current_stream_handle(a.device.index)}"
-    dst = recall_note([wave_offset], note) if owned else None
+    dst = recall_note([wave_offset], "owner slot offsets") if owned else None
     if dst is None:
         dst = as_device_table(wave_offset, a.device, 2).clone()
         dst[:, 0] = 0
         if owned:
-            remember_note([wave_offset], note, dst)      # the same tensor next time: gemm_remote's notes hold
+            remember_note([wave_offset], "owner slot offsets", dst)      # the same tensor next time: gemm_remote's notes hold
     gemm_remote(a, b, bufs, num_gemm_sms, BLOCK_SIZE_M, BLOCK_SIZE_N, BLOCK_SIZE_K, GROUP_SIZE_M, STAGES,
                 cur_wave_sizes=cur_wave_size, wave_offsets=wave_offset, M=m, target_rank=target_rank,
                 dst_offsets=dst, atomic_add=True, cum_tiles=m * b.shape[0], **kwargs)
@@ -380,15 +389,15 @@ def gemm_splitk(
         raise ValueError("wave size and offset tables disagree on the number of waves")
     # the two-column tables gemm_remote takes, kept with the caller's three-column ones (so that its notes hold too)
     owned = all(isinstance(t, torch.Tensor) and t.is_cuda for t in (cur_wave_sizes, wave_offsets))
-    note = f"split-k tables, stream {_lib.current_stream_handle(dev.index)}"
-    split = recall_note([cur_wave_sizes, wave_offsets], note) if owned else None
+    split = recall_note([cur_wave_sizes, wave_offsets], "split-k tables") if owned else None
     if split is None:
         split = (sizes3[:, :2].contiguous(), offsets3[:, :2].contiguous(),
                  torch.zeros(num_waves, dtype=torch.int32, device=dev),
-                 torch.stack([offsets3[:, 2], sizes3[:, 2]], dim=1).contiguous())
+                 torch.stack([offsets3[:, 2], sizes3[:, 2]], dim=1).contiguous(), set())
         if owned:
-            remember_note([cur_wave_sizes, wave_offsets], note, split)
-    sizes2, offsets2, ranks, k_ranges = split
+            remember_note([cur_wave_sizes, wave_offsets], "split-k tables", split)
+    sizes2, offsets2, ranks, k_ranges, streams = split
+    _read_here((sizes2, offsets2), streams, dev)
     gemm_remote(a, b, [c], num_gemm_sms, BLOCK_SIZE_M, BLOCK_SIZE_N, BLOCK_SIZE_K, GROUP_SIZE_M, STAGES,
                 cur_wave_sizes=sizes2, wave_offsets=offsets2, M=a.shape[0], target_rank=ranks, dst_offsets=offsets2,
                 atomic_add=True, k_ranges=k_ranges, signal_ptr=signal_ptr, signal_offsets=signal_offsets,

@@ -104,7 +104,7 @@ bool capturing(int dev) {
 // ---------------------------------------------------------------- what is known about a set of tables
 
 // A launch is known by its kind, the tables' objects and what `params` lists: sizes, options, for C bound to buffers their addresses,
-// and the stream, so that the device tables a record keeps are given back in the order of the stream that reads them.
+// and the stream, on which the launcher has marked the device tables that a record keeps as read.
 struct Known {
     std::vector<c10::weak_intrusive_ptr<c10::TensorImpl>> tables;
     std::vector<int64_t> versions;

@@ -182,6 +182,43 @@ def test_launches_in_turn_on_one_set_of_tables(hip, monkeypatch, differ):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form", ["direct", "split k"])
+def test_captured_behind_a_launch_on_another_stream(hip, form):
+    """What an eager launch has prepared serves the capture, whose stream is another one; replays among eager launches."""
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.gemm import gemm_rs_producer_persistent, gemm_splitk
+
+    m, n, k = 512, 512, 128
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a, b = ((0.1 * torch.randn(s, k, device="cuda", generator=g)).bfloat16() for s in (m, n))
+    c = torch.zeros(m, n, dtype=torch.bfloat16, device="cuda")
+    sizes, offsets, waves = _table([[256, n]] * 2), _table([[0, 0], [256, 0]]), _table([0, 1])
+    boxes, halves = (_table([[m, n, 64]] * 2), _table([[0, 0, 0], [0, 0, 64]])), list(c.view(2, 256, n))
+
+    def launch():
+        c.zero_()
+        if form == "direct":
+            gemm_rs_producer_persistent(a, b, halves, sizes, offsets, waves, 2, 2, 64, 128, 128, 64, 8)
+        else:
+            gemm_splitk(a, b, c, 2, 64, 128, 128, 64, 8, cur_wave_sizes=boxes[0], wave_offsets=boxes[1], cum_tiles=2 * m * n)
+
+    launch()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        launch()
+    for turn in range(4):
+        a.mul_(-1)
+        launch()
+        want = c.clone()
+        c.fill_(7)
+        graph.replay()
+        torch.cuda.synchronize()
+        check_status()
+        assert torch.equal(c, want) and want.any()
+
+
+@pytest.mark.gpu
 def test_first_launches_inside_inference_mode(hip):
     """The pools of zeroed words, of the native launches and of the launchers, are made inside the mode and filled again outside."""
     from syncopate_amd.computation._launch import ZERO_POOL_SLICES, check_status, zeroed_int32
