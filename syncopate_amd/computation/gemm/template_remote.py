@@ -20,8 +20,7 @@ allocations.  Everything else (tables in elements, B stored [N, K]) is as in ``t
 from __future__ import annotations
 
 import ctypes
-import functools
-from typing import Optional, Sequence
+from typing import Dict, Optional, Sequence, Tuple
 
 import torch
 
@@ -55,13 +54,23 @@ def _check_ranks(name: str, ranks: torch.Tensor, count: int, num_waves: int) -> 
         raise ValueError(f"{name} names a rank outside 0..{count - 1}")
 
 
-@functools.lru_cache(maxsize=64)
-def _no_signals(num_waves: int, device_index: int):
-    """Signal offsets and a flag array for waves that wait for nothing, read by every such launch and written by none (copied
-    from the host, so that they are there for whichever stream launches)."""
-    with torch.inference_mode(False):
-        return (torch.tensor([-1] * num_waves, dtype=torch.int32, device=torch.device("cuda", device_index)),
-                torch.tensor([0], dtype=torch.int64, device=torch.device("cuda", device_index)))
+_NO_SIGNALS: Dict[Tuple[int, int], Tuple[torch.Tensor, torch.Tensor]] = {}
+
+
+def _no_signals(num_waves: int, device: torch.device) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Signal offsets and a flag array for waves that wait for nothing, read by every such launch and written by none.  Those of the
+    first 64 numbers of waves are kept for good (copied from the host, so that they are there for whichever stream launches); a
+    captured launch has its own, which lie in its graph's memory."""
+    key = (num_waves, device.index)
+    tables = _NO_SIGNALS.get(key)
+    capturing = torch.cuda.is_current_stream_capturing()
+    if tables is None and not capturing and len(_NO_SIGNALS) < 64:
+        with torch.inference_mode(False):
+            tables = _NO_SIGNALS[key] = (torch.tensor([-1] * num_waves, dtype=torch.int32, device=device),
+                                         torch.tensor([0], dtype=torch.int64, device=device))
+    if tables is None or capturing:
+        tables = (torch.full((num_waves,), -1, dtype=torch.int32, device=device), torch.zeros((1,), dtype=torch.int64, device=device))
+    return tables
 
 
 def _read_here(tables: Sequence[torch.Tensor], streams: set, dev: torch.device) -> None:
@@ -210,7 +219,7 @@ def gemm_remote(
     if offsets.shape[0] != num_waves:
         raise ValueError("wave size and offset tables disagree on the number of waves")
     if signal_offsets is None:
-        signals, flags = _no_signals(num_waves, dev.index)
+        signals, flags = _no_signals(num_waves, dev)
         if signal_ptr is not None:
             flags = signal_ptr
     else:
@@ -271,7 +280,8 @@ def gemm_remote(
     with device_scope(dev):
         _lib.check("syn_gemm_remote_binding",
                    lib.syn_gemm_remote_binding(ctypes.byref(desc), ctypes.byref(remote), _lib.stream_handle(stream)))
-    if steady is not None and caller_owned and sizes is cur_wave_sizes and offsets is wave_offsets:
+    if steady is not None and caller_owned and sizes is cur_wave_sizes and offsets is wave_offsets \
+            and not torch.cuda.is_current_stream_capturing():
         _lib.native().remote(*steady, bytes(desc), bytes(remote), status_words(dev),
                              [signals, flags] + [t for t in keep if t is not target_rank and t is not dst_offsets])
     del keep, prepared

@@ -323,7 +323,7 @@ PyObject* remote(PyObject*, PyObject* const* args, Py_ssize_t n) {
         Py_RETURN_NONE;
     }
     const Known* k = recall(kKindRemote, tables, params);
-    NEED(k != nullptr);
+    NEED(k != nullptr && !capturing(g.dev));      // (a graph must not point into what a record keeps)
     syn_gemm_desc d = k->gemm;
     syn_gemm_remote r = k->remote;
     const std::vector<at::Tensor> keep = k->keep;

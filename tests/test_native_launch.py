@@ -219,6 +219,49 @@ def test_captured_behind_a_launch_on_another_stream(hip, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("warm", [True, False])
+def test_captured_launch_has_tables_of_its_own(hip, monkeypatch, warm):
+    """The tables of waves that wait for nothing, in a captured launch: not those that eager launches share and a record keeps, whether
+    the captured number of waves was seen before or not."""
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.gemm import gemm_remote, template_remote
+
+    m, n, k, waves = 512, 512, 128, 4 if warm else 2
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a, b = ((0.1 * torch.randn(s, k, device="cuda", generator=g)).bfloat16() for s in (m, n))
+    c = torch.zeros(m, n, dtype=torch.bfloat16, device="cuda")
+    sizes, offsets = _table([[m // waves, n]] * waves), _table([[i * m // waves, 0] for i in range(waves)])
+    owners, bound = _table([0] * waves), [c]
+    launch = lambda: gemm_remote(a, b, bound, 64, 128, 128, 64, 8, cur_wave_sizes=sizes, wave_offsets=offsets, M=m, target_rank=owners,
+                                 dst_offsets=offsets)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        launch()                                         # prepared, and a record of this stream
+        launch()
+        torch.cuda.synchronize()
+        if not warm:
+            monkeypatch.setattr(template_remote, "_NO_SIGNALS", {})
+        kept = dict(template_remote._NO_SIGNALS)
+        made, full = [], torch.full
+        monkeypatch.setattr(torch, "full", lambda shape, *args, **kw: made.append(shape) or full(shape, *args, **kw))
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            launch()
+        assert made == [(waves,)] and template_remote._NO_SIGNALS == kept
+    a.mul_(-1)
+    want = a.float() @ b.float().T
+    for _ in range(3):
+        c.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        check_status()
+        # one rounding of the result (2^-9 relative), sums in 32 bits
+        assert (c.float() - want).abs().max() <= 4e-3 * want.abs().max()
+        launch()
+
+
+@pytest.mark.gpu
 def test_first_launches_inside_inference_mode(hip):
     """The pools of zeroed words, of the native launches and of the launchers, are made inside the mode and filled again outside."""
     from syncopate_amd.computation._launch import ZERO_POOL_SLICES, check_status, zeroed_int32
