@@ -80,7 +80,7 @@ def _launch(
         # operands and tables of a launch that came this way before: launched without the interpreter
         steady = (a, b, c, signal_buffer, cur_wave_size, wave_offset, signal_offsets, num_gemm_sms, BLOCK_SIZE_M, BLOCK_SIZE_N,
                   BLOCK_SIZE_K, GROUP_SIZE_M, cum_tiles, -1 if xcd_remap is None else bool(xcd_remap),
-                  id(choose_kernel_tile), producer, acquire_always(signal_buffer))
+                  choose_kernel_tile, producer, acquire_always(signal_buffer))
         code = _lib.native().gemm(*steady)
         if code is not None:
             _lib.check("syn_gemm_producer" if producer else "syn_gemm_consumer", code)

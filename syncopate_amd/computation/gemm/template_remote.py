@@ -189,7 +189,7 @@ def gemm_remote(
         # operands and tables of a launch that came this way before: launched without the interpreter
         steady = (a, b, c_list, cur_wave_sizes, wave_offsets, target_rank, dst_offsets, num_gemm_sms, BLOCK_SIZE_M, BLOCK_SIZE_N,
                   BLOCK_SIZE_K, GROUP_SIZE_M, cum_tiles, bool(xcd_remap), M, bool(atomic_add),
-                  id(choose_kernel_tile))
+                  choose_kernel_tile)
         code = _lib.native().remote(*steady)
         if code is not None:
             _lib.check("syn_gemm_remote_binding", code)

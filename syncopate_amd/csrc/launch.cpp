@@ -21,6 +21,7 @@
 
 #include <array>
 #include <map>
+#include <set>
 #include <thread>
 #include <tuple>
 #include <vector>
@@ -219,10 +220,17 @@ bool gemm_operands(PyObject* pa, PyObject* pb, GemmOperands* g) {
     return true;
 }
 
+// A launch holds for the rule (a function) that chose its kernel tile.  Those that a record was made under are kept, so that another
+// one does not come to the same address.
+int64_t rule_of(PyObject* rule, bool keep) {
+    static auto* const kept = new std::set<PyObject*>;
+    if (keep && kept->insert(rule).second) Py_INCREF(rule);
+    return reinterpret_cast<int64_t>(rule);
+}
+
 // gemm(a, b, c, signal, sizes, offsets, signals, num_sms, bm, bn, bk, group_m, cum_tiles, xcd_remap, rule, producer, acquire
 // [, desc, status])
-// With a descriptor (bytes) the launch it came from is remembered; else a remembered one is launched.  `rule` says which rule chose
-// the kernel's tile.
+// With a descriptor (bytes) the launch it came from is remembered; else a remembered one is launched.
 constexpr int kKindGemm = 0, kKindProducer = 1, kKindRemote = 2, kKindAttn = 3;
 
 PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -243,7 +251,8 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const bool producer = as_int(args[15], &ok) != 0, acquire = as_int(args[16], &ok) != 0;
     std::vector<int64_t> params = {g.M, g.N, g.K, g.dtype, g.dev, stream_of(g.dev), flags->numel()};
     params.reserve(18);
-    for (int i = 7; i < 15; ++i) params.push_back(as_int(args[i], &ok));
+    for (int i = 7; i < 14; ++i) params.push_back(as_int(args[i], &ok));
+    params.push_back(rule_of(args[14], n == 19));
     NEED(ok);
     for (const at::Tensor* t : tables) params.push_back(t->numel());
     const int kind = producer ? kKindProducer : kKindGemm;
@@ -295,8 +304,9 @@ PyObject* remote(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const Py_ssize_t buffers = PyList_GET_SIZE(args[2]);
     std::vector<int64_t> params = {g.M, g.N, g.K, g.dtype, g.dev, stream_of(g.dev)};
     params.reserve(20 + 3 * (size_t)buffers);
-    for (int i = 7; i < 17; ++i) params.push_back(as_int(args[i], &ok));
+    for (int i = 7; i < 16; ++i) params.push_back(as_int(args[i], &ok));
     NEED(ok && params[13] == g.M);
+    params.push_back(rule_of(args[16], n == 21));
     for (const at::Tensor* t : tables) params.push_back(t->numel());
     for (Py_ssize_t i = 0; i < buffers; ++i) {
         const at::Tensor* c = plain(PyList_GET_ITEM(args[2], i), g.dev);

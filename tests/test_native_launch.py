@@ -262,6 +262,26 @@ def test_captured_launch_has_tables_of_its_own(hip, monkeypatch, warm):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form", ["consumer", "direct"])
+def test_another_rule_for_the_tile_is_asked(hip, form):
+    """Rules made and dropped one after the other, as a caller's own may be: each is asked, wherever it lies in memory."""
+    from syncopate_amd.computation._launch import check_status
+
+    run, want, _, _, module = _gemm_case(form)
+    rule, asked, places = module.choose_kernel_tile, [], set()
+    try:
+        for turn in range(4):
+            module.choose_kernel_tile = lambda *args, **kw: asked.append(turn) or rule(*args, **kw)
+            places.add(id(module.choose_kernel_tile))
+            for _ in range(2):
+                assert (run().float() - want).abs().max() <= 4e-3 * want.abs().max()
+    finally:
+        module.choose_kernel_tile = rule
+    check_status()
+    assert asked == [0, 1, 2, 3] and len(places) == 4
+
+
+@pytest.mark.gpu
 def test_first_launches_inside_inference_mode(hip):
     """The pools of zeroed words, of the native launches and of the launchers, are made inside the mode and filled again outside."""
     from syncopate_amd.computation._launch import ZERO_POOL_SLICES, check_status, zeroed_int32
