@@ -491,14 +491,14 @@ int syn_delay_us(int64_t us, syn_stream_t stream);
  * done. */
 int syn_stream_create_cu_mask(const uint32_t* mask, uint32_t words, syn_stream_t* stream);
 int syn_stream_destroy(syn_stream_t stream);
-/* Launch `workgroups` workgroups that each record where they ran: out[2 b] = hardware id word
- * (compute unit, shader array, shader engine in bits 8..15), out[2 b + 1] = XCD id, and stay for
- * `dwell` short sleeps so that the grid spreads over every compute unit the stream may use.
- * No counterpart in the reference; it is how a partition of the device is checked. */
 /* Copies `n` <= 4 small tables of 32-bit words one behind the other to `host_words` and then writes `seq` to `*host_flag`, both in
  * pinned host memory: a caller that looks at the flag has the tables as they are at this point of the stream. */
 int syn_read_tables_async(const int32_t* const* tables, const int32_t* counts, int32_t n, int32_t* host_words, uint64_t* host_flag,
                           uint64_t seq, syn_stream_t stream);
+/* Launch `workgroups` workgroups that each record where they ran: out[2 b] = hardware id word
+ * (compute unit, shader array, shader engine in bits 8..15), out[2 b + 1] = XCD id, and stay for
+ * `dwell` short sleeps so that the grid spreads over every compute unit the stream may use.
+ * No counterpart in the reference; it is how a partition of the device is checked. */
 int syn_where_async(uint32_t* out, int32_t workgroups, int32_t dwell, syn_stream_t stream);
 
 /* Measurement aid, no counterpart in the reference: `workgroups` workgroups of four wavefronts

@@ -1064,7 +1064,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
     constexpr int TM = WM / 32, TN = WN / 32;     // 32x32 MFMA tiles per wavefront
 
     __shared__ int s_abort;
-    __shared__ int s_spun, s_waves_up;
+    __shared__ int s_spun, s_waves_up;   // written by wait_flag ..
+    __shared__ int s_first_up;           // .. while others may still read this one
     // C staging of the epilogue: 32 rows x CS_COLS columns per wavefront, 64 columns where LDS allows
     constexpr int NWAVES = WGM * WGN;
     constexpr int CS_COLS = ((BN / WGN / 32) % 2 == 0 &&
@@ -1109,11 +1110,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
         const int sig = wait_index(lane);
         const bool up = sig < 0 || __hip_atomic_load(wait_on + sig, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 1ull;
         const unsigned long long down = ~__builtin_amdgcn_ballot_w64(up);
-        if (lane == 0) s_waves_up = p.acquire_always ? 0 : down == 0 ? 64 : (int)__builtin_ctzll(down);
+        if (lane == 0) s_first_up = down == 0 ? 64 : (int)__builtin_ctzll(down);
     }
     __syncthreads();
-    int waves_up = uniform(s_waves_up);
-    __syncthreads();       // wait_flag writes the word: only when everyone has read it
+    int waves_up = p.acquire_always ? 0 : uniform(s_first_up);
 
     // --- wave walk state (uniform across the workgroup) ---
     int cur_wave = -1, past_tiles = 0, cur_tiles = 0;
