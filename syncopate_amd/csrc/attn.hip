@@ -1067,8 +1067,8 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
 
     // wait for flag `sg` of the wave `wv` that is being entered; false when the wait gave up
     // A look ahead at the flag of the visit after the one being entered (thread 0): asked for here, read at the next
-    // change of visit, a kv range later.  A flag goes up once per launch, so a 1 seen early still holds then; a 0
-    // means nothing and the flag is read again.
+    // change of visit, a kv range later.  A flag goes up once per launch, so a 1 seen early still holds then (not under
+    // SYN_ATTN_ACQUIRE_ALWAYS, whose caller need not promise that); a 0 means nothing and the flag is read again.
     int peeked_sig = -1;
     unsigned long long peeked = 0;
     auto peek_flag = [&](const int sg) __attribute__((always_inline)) {
@@ -1077,7 +1077,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) attn_pair_kernel(const AttnPa
     };
     auto wait_for_flag = [&](const int sg, const int wv) __attribute__((always_inline)) -> bool {
         if (tid == 0) {
-            const bool seen_up = peeked_sig == sg && peeked == 1ull;
+            const bool seen_up = peeked_sig == sg && peeked == 1ull && !p.acquire_always;
             s_spun = !seen_up && __hip_atomic_load(p.flags + sg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 1ull;
             if (s_spun && !spin_until_equal(p.flags + sg, 1ull, p.timeout_ticks)) {
                 report_status(p.status, SYN_STATUS_SPIN_TIMEOUT, wv, (int)blockIdx.x, sg);

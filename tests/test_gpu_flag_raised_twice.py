@@ -53,13 +53,15 @@ def test_gemm(hip, block_n):
     assert torch.equal(got, c)
 
 
-def test_dealt_attention(hip, monkeypatch):
+@pytest.mark.parametrize("form", ["dealt", "parts", "chained", "tiles"])
+def test_attention(hip, monkeypatch, form):
     from syncopate_amd.computation.attn import attention_forward, template
     from syncopate_amd.computation.attn.kv_split import KvSplit
 
-    blocks = 2000                                        # of 2.8 us each, on one program
-    monkeypatch.setattr(template, "plan_kv_split", lambda *args, **kwargs: None)
-    monkeypatch.setattr(template, "plan_kv_deal", lambda *args, **kwargs: KvSplit(True, 1, 1, blocks + 1))
+    blocks = 2000                                        # of 2.4 or 2.8 us each, on one or two programs
+    whole = KvSplit(True, 1, 1, blocks + 1)
+    monkeypatch.setattr(template, "plan_kv_split", lambda *args, **kwargs: whole if form == "parts" else None)
+    monkeypatch.setattr(template, "plan_kv_deal", lambda *args, **kwargs: whole if form == "dealt" else None)
     g = torch.Generator(device="cuda").manual_seed(1)
     q, k, v = (torch.randn(1, 1, s, 128, device="cuda", generator=g).bfloat16() for s in (256, 128 * (blocks + 1), 128 * (blocks + 1)))
     v[:, :, 128 * blocks:] = 0
@@ -68,7 +70,8 @@ def test_dealt_attention(hip, monkeypatch):
     tables = dict(wave_offsets=table([[0, 0, 0, 0], [0, 0, 0, 128 * blocks]]), wave_sizes=table([[1, 1, 256, 128 * blocks], [1, 1, 256, 128]]),
                   cum_wave_sizes=table([256, 512]), signal_offsets=table([0, 1]), cum_tiles=512)
     flags = torch.ones(2, dtype=torch.int64, device="cuda")
-    launch = lambda: attention_forward(q, k, v, 128 ** -0.5, signal_ptr=flags, **tables)
+    options = dict(chained=dict(pair_q_blocks=True, chain_q_blocks=True), tiles=dict(num_programs=2)).get(form, {})
+    launch = lambda: attention_forward(q, k, v, 128 ** -0.5, signal_ptr=flags, **tables, **options)
     got = _again(launch, flags, lambda: v[:, :, 128 * blocks:].copy_(new))
     assert torch.equal(got, launch())
     check_status()
