@@ -923,9 +923,9 @@ def run_attention_slot(device, launches=10):
 
 
 def _host_cpu():
-    """What the CPU baselines ran on: the model string, the cores the host shows and the threads used.  A one-GPU box
-    of the pool gives a job 16 cores whatever the host shows (OMP_NUM_THREADS is 16 there), so the baselines use
-    at most that many threads."""
+    """What the CPU baselines ran on: the model string, the cores the host shows and the threads used.  A job with
+    one GPU has 16 cores whatever the host shows (OMP_NUM_THREADS is 16 there), so the baselines use at most that
+    many threads."""
     model = ""
     try:
         with open("/proc/cpuinfo") as f:
@@ -937,7 +937,7 @@ def _host_cpu():
         pass
     threads = min(16, os.cpu_count() or 1)
     return {"cpu_model": model, "host_cores": os.cpu_count(), "threads": threads,
-            "threads_note": "capped at the 16 cores a one-GPU job of this pool is given"}
+            "threads_note": "capped at 16 cores for one GPU"}
 
 
 def cpu_baseline(state):

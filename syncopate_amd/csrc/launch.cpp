@@ -150,7 +150,7 @@ void remember(int64_t kind, const std::vector<const at::Tensor*>& tables, const 
     }
     if (g_known.size() >= kMaxRecords) {
         for (auto i = g_known.begin(); i != g_known.end();) i = i->second.alive() ? std::next(i) : g_known.erase(i);
-        if (g_known.size() >= kMaxRecords) g_known.clear();
+        if (g_known.size() >= kMaxRecords / 4 * 3) g_known.clear();      // (or the next ones would be looked through again soon)
     }
     g_known[key_of(kind, tables, params)] = std::move(k);
 }
