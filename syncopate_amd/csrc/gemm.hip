@@ -648,7 +648,7 @@ struct RollPipe : SlabPipe<T, BM, BN, WGM, WGN, NST_> {
     static constexpr int NST = NST_, kChainSlabs = 3;
     static constexpr int RM = 2 * TM, RN = 2 * TN;          // 16-row blocks of A and of B per wavefront
     static constexpr int PA = (FILLS + 2) / 3, PB = (FILLS - PA + 1) / 2, PC = FILLS - PA - PB;
-    static_assert(RM % 2 == 0, "two quarters of row blocks");
+    static_assert(RM % 2 == 0 && RN % 2 == 0, "two quarters of row blocks, columns two at a time");
 
     struct Lane16 {
         int a_rd, b_rd, quad, swz;
@@ -681,17 +681,24 @@ struct RollPipe : SlabPipe<T, BM, BN, WGM, WGN, NST_> {
     // One quarter: row blocks HALF * RM/2 .. of A against all column blocks, `between(g)` after MFMA g.  The MFMAs
     // are volatile assembly, so the memory operations that `between` issues stay where the source puts them.
     // B is the first operand: acc[i][j] holds D'[n][m] of rows m = 16 i .. and columns n = 16 j .. of the wavefront's
-    // part, lane l the four consecutive n = 4 (l / 16) + 0..3 of row m = l % 16
+    // part, lane l the four consecutive n = 4 (l / 16) + 0..3 of row m = l % 16.
+    // The order: two columns at a time, down the rows and up again, so that from one MFMA to the next ONE operand changes, A and B
+    // in turn.  What the operand latches and multipliers switch is power, and on operands other than zeros the board's
+    // power limit is the clock: bare MFMAs on random registers run at 2064 TFLOP/s in this order, 2049 to and fro along whole rows,
+    // 2000 row after row (which changes both at the end of each), 1942 with both changed every time (zeros: 2409 in any).  Against
+    // row after row: 8192 x 3584 x 8192 on 256x256 tiles 333.4 -> 329.4 us, 8192 x 8192 x 3584 and its reduce 356.3 -> 353.6, 128x128
+    // tiles, 8192 x 2048 x 4096, 121.9 -> 119.8, 128x256, n = 4096, 211.0 -> 209.0.
     template <int HALF, typename F>
     static __device__ __forceinline__ void quarter(f32x4_t (&acc)[RM][RN], const frag_t (&fa)[RM], const frag_t (&fb)[RN],
                                                    F&& between) {
+        constexpr int R = RM / 2;
 #pragma unroll
-        for (int i = 0; i < RM / 2; ++i)
-#pragma unroll
-            for (int j = 0; j < RN; ++j) {
-                Mfma16<T>::run(fb[j], fa[HALF * (RM / 2) + i], acc[HALF * (RM / 2) + i][j]);
-                between(i * RN + j);
-            }
+        for (int g = 0; g < R * RN; ++g) {
+            const int pair = g / (2 * R), row = g % (2 * R) / 2;
+            const int i = pair % 2 == 0 ? row : R - 1 - row, j = 2 * pair + (g % 2 ^ row % 2);
+            Mfma16<T>::run(fb[j], fa[HALF * R + i], acc[HALF * R + i][j]);
+            between(g);
+        }
     }
 
     // Where a tile's slabs come from: the first rows of its panels, the number of slabs, and the one it begins with.
