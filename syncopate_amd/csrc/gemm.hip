@@ -73,6 +73,13 @@ struct GemmParams {
     int32_t tail_tiles;          // TAIL kernels: the last so many tiles run as 128x128 ones
 };
 
+// what a wave of a remote binding is bound to: its peer's A and / or C (null: the launch's own), where its tiles go in C, its K range
+struct Bound {
+    const void* a;
+    void* c;
+    int dst_m, dst_n, k0, k_len;
+};
+
 // kernel modes
 constexpr int kConsumer = 0, kProducer = 1, kRemote = 2, kRemoteAtomic = 3;   // kRemoteAtomic: kRemote whose C tiles are added
 
@@ -1102,6 +1109,26 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
         s_waves[w][3] = p.wave_offsets[2 * w + 1] / BN;
         s_waves[w][4] = p.signal_offsets[w];
     }
+    // What a wave is bound to.  Looked up for the wave of a tile, where the tile is worked out: a peer's address is two loads one after
+    // the other, and looked up for every wave that the walk passes on the way, in front of each tile, the walk waited for them
+    // all (four waves to a tile of eight owners' 8192 x 8192 x 3584, added: 391 -> 386 us; one wave each, 1024 x 1024 x 1024, 12.7 ->
+    // 12.4, where nothing needs the address before the last product now).  Copied to LDS with the wave table, 384 and 13.0.
+    auto bound_to = [&](int w) -> Bound {
+        Bound b = {nullptr, nullptr, 0, 0, 0, p.K};
+        // the wave's peer: A rows are read from its shard and / or C tiles go into its buffer,
+        // both addressed by wave-local rows (template_ag.py:151-161, template_rs.py:140-166)
+        if (p.a_peers) b.a = p.a_peers[p.a_target[w]];
+        if (p.c_peers) {
+            b.c = p.c_peers[p.c_target[w]];
+            b.dst_m = p.c_dst_offsets[2 * w];
+            b.dst_n = p.c_dst_offsets[2 * w + 1];
+        }
+        if (p.wave_k) {
+            b.k0 = p.wave_k[2 * w];
+            b.k_len = p.wave_k[2 * w + 1];
+        }
+        return b;
+    };
     if (tid == 0) s_abort = 0;
     // Which waves need not be waited for.  Flags are read for 64 waves at a time, a lane each - here for the first ones, beside the
     // table, and whenever a wave has to be waited for - and those in a row that are up are not looked at again: a flag goes up
@@ -1126,10 +1153,6 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
     int cur_wave = -1, past_tiles = 0, cur_tiles = 0;
     int cur_m = 0, cur_n = 0, off_m = 0, off_n = 0, cur_sig = -1;
     int cur_wait = -1;            // flag index the wave waits for: its own signal (consumer), the second table's (producer)
-    const T* a_base = nullptr;
-    T* c_base = nullptr;
-    int dst_m = 0, dst_n = 0;
-    int cur_k0 = 0, cur_klen = p.K;
     auto enter_wave = [&](int w) {
         cur_wave = w;
         if (w < kLdsWaves) {
@@ -1147,20 +1170,6 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
         }
         cur_wait = PRODUCER ? (p.wait_offsets != nullptr ? p.wait_offsets[w] : -1) : cur_sig;
         cur_tiles = cur_m * cur_n;
-        if (REMOTE) {
-            // the wave's peer: A rows are read from its shard and / or C tiles go into its buffer,
-            // both addressed by wave-local rows (template_ag.py:151-161, template_rs.py:140-166)
-            a_base = p.a_peers ? reinterpret_cast<const T*>(p.a_peers[p.a_target[w]]) : nullptr;
-            if (p.c_peers) {
-                c_base = reinterpret_cast<T*>(p.c_peers[p.c_target[w]]);
-                dst_m = p.c_dst_offsets[2 * w];
-                dst_n = p.c_dst_offsets[2 * w + 1];
-            }
-            if (p.wave_k) {
-                cur_k0 = p.wave_k[2 * w];
-                cur_klen = p.wave_k[2 * w + 1];
-            }
-        }
     };
     enter_wave(0);
 
@@ -1252,11 +1261,16 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
         t.b_panel = reinterpret_cast<const unsigned char*>(B + (size_t)pid_n * BN * K);
         t.c_tile = C + (size_t)pid_m * BM * N + (size_t)pid_n * BN;
         t.ldc = (size_t)N;
-        if (REMOTE) {
+        Bound bound = {};
+        if constexpr (REMOTE) {
+            bound = bound_to(cur_wave);
+            const T* const a_base = static_cast<const T*>(bound.a);
+            T* const c_base = static_cast<T*>(bound.c);
             if (a_base) t.a_panel = reinterpret_cast<const unsigned char*>(a_base + (size_t)pid_m_local * BM * K);
             if (c_base) {
                 t.ldc = (size_t)p.c_ld;
-                t.c_tile = c_base + ((size_t)dst_m + (size_t)pid_m_local * BM) * t.ldc + dst_n + (size_t)pid_n_local * BN;
+                t.c_tile = c_base + ((size_t)bound.dst_m + (size_t)pid_m_local * BM) * t.ldc + bound.dst_n +
+                           (size_t)pid_n_local * BN;
             }
         }
         // Tiles walk K cyclically, neighbouring tiles starting 128 elements apart.  With a
@@ -1267,9 +1281,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
         t.k_rot = p.k_stagger ? (((pid_m >> p.cut_m) + (pid_n >> p.cut_n)) & 3) * (128 / Pipe::BK) : 0;
         t.k_len = K;
         if (REMOTE) {
-            t.a_panel += (size_t)cur_k0 * sizeof(T);
-            t.b_panel += (size_t)cur_k0 * sizeof(T);
-            t.k_len = cur_klen;
+            const int k0 = bound.k0;
+            t.a_panel += (size_t)k0 * sizeof(T);
+            t.b_panel += (size_t)k0 * sizeof(T);
+            t.k_len = bound.k_len;
         }
         t.wave = cur_wave;
         t.sig = cur_sig;
