@@ -171,6 +171,13 @@ __device__ __forceinline__ const unsigned char* uniform(const unsigned char* ptr
     return reinterpret_cast<const unsigned char*>(lo | hi << 32);
 }
 
+// An entry of a table that nothing writes during the launch, at an address that is the same in every lane, by a scalar load.  (The
+// compiler, which cannot tell that the kernel's own stores leave the table alone, makes vector loads of it.)
+template <typename U>
+__device__ __forceinline__ U table_entry(const U* table, int i) {
+    return *(const __attribute__((address_space(4))) U*)(uintptr_t)(table + i);
+}
+
 typedef __attribute__((address_space(3))) void* lds_void_ptr;
 typedef const __attribute__((address_space(1))) void* global_void_ptr;
 
@@ -1109,23 +1116,28 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_wave_kernel(const GemmPar
         s_waves[w][3] = p.wave_offsets[2 * w + 1] / BN;
         s_waves[w][4] = p.signal_offsets[w];
     }
-    // What a wave is bound to.  Looked up for the wave of a tile, where the tile is worked out: a peer's address is two loads one after
-    // the other, and looked up for every wave that the walk passes on the way, in front of each tile, the walk waited for them
-    // all (four waves to a tile of eight owners' 8192 x 8192 x 3584, added: 391 -> 386 us; one wave each, 1024 x 1024 x 1024, 12.7 ->
-    // 12.4, where nothing needs the address before the last product now).  Copied to LDS with the wave table, 384 and 13.0.
+    // What a wave is bound to.  Looked up for the wave of a tile, where the tile is worked out, and by scalar loads.  A peer's address
+    // is two loads one after the other.  Looked up for every wave that the walk passes, the walk waited for two such pairs a tile where
+    // 256 programs on 256x256 tiles go through eight owners' 8192 x 8192 x 3584; by vector loads for every tile, each wait
+    // was also one for the last tile's stores and the next one's fills, which end in order with them.  Adding form, us, entering each
+    // wave (and the products row after row, see RollPipe::quarter) / vector loads for each tile / this: 386.4 / 379.9 / 379.8 there; tiles that stay in a wave, 2 owners, 224 programs: 128x256,
+    // 8192 x 4096 x 512, 69.2 / 70.4 / 68.7, 128x128, 2048 x 8192 x 256, 33.4 / 34.2 / 33.4 (storing, the former: 52.2 / 52.4 / 50.0);
+    // a tile a program, 1024 x 1024 x 1024: 11.08 / 10.65 / 10.76.  Kept in registers until the wave changes, by
+    // vector loads, the 256x256 kernels spill 87 registers for 23 (391 -> 398); in scalar ones, no faster than this.
     auto bound_to = [&](int w) -> Bound {
         Bound b = {nullptr, nullptr, 0, 0, 0, p.K};
+        w = uniform(w);
         // the wave's peer: A rows are read from its shard and / or C tiles go into its buffer,
         // both addressed by wave-local rows (template_ag.py:151-161, template_rs.py:140-166)
-        if (p.a_peers) b.a = p.a_peers[p.a_target[w]];
+        if (p.a_peers) b.a = table_entry(p.a_peers, table_entry(p.a_target, w));
         if (p.c_peers) {
-            b.c = p.c_peers[p.c_target[w]];
-            b.dst_m = p.c_dst_offsets[2 * w];
-            b.dst_n = p.c_dst_offsets[2 * w + 1];
+            b.c = table_entry(p.c_peers, table_entry(p.c_target, w));
+            b.dst_m = table_entry(p.c_dst_offsets, 2 * w);
+            b.dst_n = table_entry(p.c_dst_offsets, 2 * w + 1);
         }
         if (p.wave_k) {
-            b.k0 = p.wave_k[2 * w];
-            b.k_len = p.wave_k[2 * w + 1];
+            b.k0 = table_entry(p.wave_k, 2 * w);
+            b.k_len = table_entry(p.wave_k, 2 * w + 1);
         }
         return b;
     };

@@ -93,7 +93,7 @@ def test_peers_rows_and_sums(hip, bm, bn):
     sizes, offsets = _table([[rows, n]] * world), _table([[i * rows, 0] for i in order])
     log = torch.empty(18, 4, dtype=torch.int32, device="cuda")                 # (whole tiles)
     results = []
-    for programs in (256, 16, 7):                     # 18 tiles
+    for programs in (256, 16, 7, 5, 2):               # 18 tiles in waves of six: on 5 and on 2, a program's next tile may be its wave's
         for whole in (True, False):
             kw = dict(visit_log=log) if whole else {}
             c = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
