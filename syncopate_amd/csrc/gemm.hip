@@ -705,15 +705,16 @@ struct RollPipe : SlabPipe<T, BM, BN, WGM, WGN, NST_> {
     template <int HALF, typename F>
     static __device__ __forceinline__ void quarter(f32x4_t (&acc)[RM][RN], const frag_t (&fa)[RM], const frag_t (&fb)[RN],
                                                    F&& between) {
-        constexpr int R = RM / 2;
 #pragma unroll
-        for (int g = 0; g < R * RN; ++g) {
-            const int pair = g / (2 * R), row = g % (2 * R) / 2;
-            const int i = pair % 2 == 0 ? row : R - 1 - row, j = 2 * pair + (g % 2 ^ row % 2);
-            Mfma16<T>::run(fb[j], fa[HALF * R + i], acc[HALF * R + i][j]);
+        for (int g = 0; g < RM / 2 * RN; ++g) {
+            const int i = HALF * (RM / 2) + row_of(g), j = column_of(g);
+            Mfma16<T>::run(fb[j], fa[i], acc[i][j]);
             between(g);
         }
     }
+    // the accumulator of MFMA g of a quarter: its row, of RM/2, and its column
+    static constexpr int row_of(int g) { return g / RM % 2 == 0 ? g % RM / 2 : RM / 2 - 1 - g % RM / 2; }
+    static constexpr int column_of(int g) { return 2 * (g / RM) + (g % 2 ^ g % RM / 2 % 2); }
 
     // Where a tile's slabs come from: the first rows of its panels, the number of slabs, and the one it begins with.
     struct Source {
@@ -843,8 +844,11 @@ struct RollPipe : SlabPipe<T, BM, BN, WGM, WGN, NST_> {
             asm volatile("" ::: "memory");
             read_step<0>(fa[0], fb[0], st + stage * STAGE, l16);
         }
-        // (two wait states between the zeros of the first accumulators and the first MFMAs)
-        asm volatile("s_nop 1" : "+a"(acc[0][0]), "+a"(acc[0][1]), "+a"(acc[0][2]), "+a"(acc[0][3]));
+        // Two wait states between the zeros of the accumulators and the MFMAs that read them: zeros of the first four MFMAs' come in
+        // front of this statement, and what comes behind it belongs to MFMAs with more than two others in front of them.
+        static_assert(Q > 4, "further MFMAs behind the first four");
+        asm volatile("s_nop 1" : "+a"(acc[row_of(0)][column_of(0)]), "+a"(acc[row_of(1)][column_of(1)]),
+                                 "+a"(acc[row_of(2)][column_of(2)]), "+a"(acc[row_of(3)][column_of(3)]));
         int s = 0;
         do {
             const int nxt_stage = behind(stage);
