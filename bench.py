@@ -329,25 +329,27 @@ def check_ag_gemm(state):
 
 # ---------------------------------------------------------------------------- matrix-pipe ceiling
 
-def run_mfma_ceiling(device, state, launches=8):
+def run_mfma_ceiling(device, state, launches=40, warmup=20):
     """What the matrix pipes of this board sustain: a loop of nothing but the GEMM's MFMA on
     register-resident operands, one workgroup of four wavefronts per compute unit, with constant
     and with random operands (the board is power-limited: toggling operand bits cost clock);
-    and the consumer kernel itself, every chunk resident, on operands that are all zero."""
+    and the consumer kernel itself, every chunk resident, on operands that are all zero.  Behind some
+    launches of warm-up: the first few run before the power limit has set the clock."""
     from syncopate_amd import _lib
 
     lib = _lib.load()
     sink = torch.empty(256 * 256, dtype=torch.float32, device=device)
     stream = _lib.stream_handle(torch.cuda.current_stream())
     iters = 2000
-    out = {"launches": launches, "mfma": "v_mfma_f32_16x16x32_bf16, 8x8 accumulators per wavefront, 128 per round (the 256x256 tile's "
-                                          "K loop); mfma_32x32x16_*: v_mfma_f32_32x32x16_bf16, 4x4 accumulators, 64 per round",
+    out = {"launches": launches, "warmup_launches": warmup,
+           "mfma": "v_mfma_f32_16x16x32_bf16, 8x8 accumulators per wavefront, 128 per round (the 256x256 tile's "
+                   "K loop, in its order); mfma_32x32x16_*: v_mfma_f32_32x32x16_bf16, 4x4 accumulators, 64 per round",
            "rounds_per_launch": iters}
     for workgroups in (256, NUM_SMS):
         for pattern, name in ((5, "constant"), (6, "random"), (1, "mfma_32x32x16_constant"), (2, "mfma_32x32x16_random")):
             def probe(i):
                 _lib.check("syn_probe_mfma_rate", lib.syn_probe_mfma_rate(sink.data_ptr(), workgroups, iters, pattern, stream))
-            ms = _timed(probe, launches, 3)
+            ms = _timed(probe, launches, warmup)
             out[f"{name}_operands_{workgroups}_workgroups_tflops"] = workgroups * 4.0 * iters * 64 * 32768 / ms / 1e9
     if state is not None and "resident_ms_fn" in state:
         zeros_a, zeros_b = torch.zeros_like(state["a"]), torch.zeros_like(state["b"])

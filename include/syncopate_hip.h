@@ -507,8 +507,9 @@ int syn_where_async(uint32_t* out, int32_t workgroups, int32_t dwell, syn_stream
  * operands, 1: all ones, 2: pseudo-random N(0, 0.02)-like values.  flop = workgroups * 4 * iters *
  * 64 * 32768.  sink: device float[workgroups * 256].  The rate with pattern 2 is what the matrix
  * pipes sustain under the board's power limit when operand bits toggle.  pattern + 4: the same
- * operands and flop on 128 v_mfma_f32_16x16x32_bf16 per round (8 x 8 accumulators), the form of
- * the 256x256 tile's K loop. */
+ * operands and flop on 128 v_mfma_f32_16x16x32_bf16 per round (8 x 8 accumulators), the form and
+ * order of the 256x256 tile's K loop; pattern + 4 + 16, 32, 48: in another order, row after row of
+ * accumulators, rows to and fro, along diagonals. */
 int syn_probe_mfma_rate(float* sink, int32_t workgroups, int32_t iters, int32_t pattern,
                         syn_stream_t stream);
 

@@ -101,8 +101,8 @@ struct AttnMfma<_Float16> {
 
 // The paired kernel's products: v_mfma_f32_16x16x32 (A: 16 rows x 32 k, lane l holds row l % 16, k 8 (l / 16) .. + 8;
 // B: 32 k x 16 columns, lane l holds column l % 16, the same k; C: lane l holds column l % 16, rows 4 (l / 16) .. + 4).
-// Same flop per cycle as the 32x32x16 form, and on random operands 11 % less energy per flop for the bare
-// instruction (syn_probe_mfma_rate) - this kernel runs at the board's power limit, so that is speed.
+// Same flop per cycle as the 32x32x16 form, and on random operands 13 % less energy per flop for the bare
+// instruction (syn_probe_mfma_rate: 2076 TFLOP/s against 1803 at the power limit, both row after row) - this kernel runs at the board's power limit, so that is speed.
 template <typename T>
 __device__ __forceinline__ f32x4_t mfma16(typename AttnMfma<T>::frag_t a, typename AttnMfma<T>::frag_t b, f32x4_t c);
 template <>

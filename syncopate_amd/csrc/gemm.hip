@@ -697,11 +697,12 @@ struct RollPipe : SlabPipe<T, BM, BN, WGM, WGN, NST_> {
     // B is the first operand: acc[i][j] holds D'[n][m] of rows m = 16 i .. and columns n = 16 j .. of the wavefront's
     // part, lane l the four consecutive n = 4 (l / 16) + 0..3 of row m = l % 16.
     // The order: two columns at a time, down the rows and up again, so that from one MFMA to the next ONE operand changes, A and B
-    // in turn.  What the operand latches and multipliers switch is power, and on operands other than zeros the board's
-    // power limit is the clock: bare MFMAs on random registers run at 2064 TFLOP/s in this order, 2049 to and fro along whole rows,
-    // 2000 row after row (which changes both at the end of each), 1942 with both changed every time (zeros: 2409 in any).  Against
-    // row after row: 8192 x 3584 x 8192 on 256x256 tiles 333.4 -> 329.4 us, 8192 x 8192 x 3584 and its reduce 356.3 -> 353.6, 128x128
-    // tiles, 8192 x 2048 x 4096, 121.9 -> 119.8, 128x256, n = 4096, 211.0 -> 209.0.
+    // in turn.  What the operand latches and multipliers switch is power, and on operands other than zeros the board's power
+    // limit is the clock of a long launch: bare MFMAs on random registers (syn_probe_mfma_rate, once the clock has settled) run at 2130
+    // TFLOP/s in this order, 2092 to and fro along whole rows, 2076 row after row (which changes both at the end of each), 2002 with both
+    // changed every time (zeros: 2466 to 2484 in any).  Against row after row: 8192 x 3584 x 8192 on 256x256 tiles 328.7 -> 323.4 us,
+    // 8192 x 8192 x 3584 and its reduce 351.6 -> 347.7, 128x128 tiles, 8192 x 2048 x 4096, 118.2 -> 116.5, 128x256, 8192 x 4096 x 4096,
+    // 207.7 -> 205.9, 5120 x 3328 x 2112 66.4 -> 65.5; nothing on zeros (277.5 -> 277.4 for the first) and in launches of 10 us.
     template <int HALF, typename F>
     static __device__ __forceinline__ void quarter(f32x4_t (&acc)[RM][RN], const frag_t (&fa)[RM], const frag_t (&fb)[RN],
                                                    F&& between) {

@@ -1,8 +1,9 @@
 // Matrix-pipe ceiling probe for gfx950 (MI355X): a loop of nothing but the GEMM kernels' MFMA, in the GEMM's
-// register pattern, with every operand held in registers: no LDS, no memory.  One workgroup of four wavefronts
+// register pattern and order, with every operand held in registers: no LDS, no memory.  One workgroup of four wavefronts
 // per compute unit (one per SIMD), like the 256x256 GEMM tile.  Two forms: v_mfma_f32_32x32x16_bf16 (a wavefront
 // owns a 4 x 4 grid of 32x32 accumulators and multiplies four A fragments with four B fragments per k16 step) and
-// v_mfma_f32_16x16x32_bf16 (8 x 8 accumulators of 16x16, eight fragments of each operand per k32 step).
+// v_mfma_f32_16x16x32_bf16 (8 x 8 accumulators of 16x16, eight fragments of each operand per k32 step).  Both in the order of
+// the GEMM's pipelines on that MFMA: row after row the former, the latter as RollPipe::quarter, or in one of three others for comparison.
 //
 // The operands of consecutive k16 steps rotate over SETS register-resident fragment sets filled
 // with a pattern: zeros, one constant, or N(0, 0.02)-like pseudo-random bf16 values.  The rate
@@ -76,8 +77,16 @@ __global__ void __launch_bounds__(256) mfma_rate_kernel(float* sink, int iters, 
     sink[me] = total;
 }
 
+// How the 16x16x32 MFMAs of a k32 step follow each other.  What changes from one to the next is what switches:
+//   kOrderPairs     the GEMM's: two columns of accumulators at a time, down the rows and up again: A and B in turn
+//   kOrderRows      row after row: B, and A too at the end of a row
+//   kOrderToAndFro  every other row backwards: B, or A at the end of a row
+//   kOrderDiagonal  both every time
+constexpr int kOrderPairs = 0, kOrderRows = 1, kOrderToAndFro = 2, kOrderDiagonal = 3;
+
 // the same on 16x16x32 MFMAs: 128 per round, the flop of 64 of the larger ones.  The accumulators are named as AGPR
 // tuples in inline assembly, as in the GEMM's K loop.
+template <int ORDER>
 __global__ void __launch_bounds__(256) mfma16_rate_kernel(float* sink, int iters, int pattern) {
     typedef float f32x4_probe_t __attribute__((ext_vector_type(4)));
     f32x4_probe_t acc[8][8];
@@ -98,10 +107,21 @@ __global__ void __launch_bounds__(256) mfma16_rate_kernel(float* sink, int iters
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fb[s][j]), "v"(fa[s][i]));
+            for (int g = 0; g < 64; ++g) {
+                int i = g / 8, j = g % 8;
+                if (ORDER == kOrderPairs) {
+                    // a half of four rows against all columns, then the other
+                    const int h = g % 32, row = h % 8 / 2;
+                    i = 4 * (g / 32) + (h / 8 % 2 == 0 ? row : 3 - row);
+                    j = 2 * (h / 8) + (h % 2 ^ row % 2);
+                } else if (ORDER == kOrderToAndFro) {
+                    j = i % 2 == 0 ? j : 7 - j;
+                } else if (ORDER == kOrderDiagonal) {
+                    j = g % 8;
+                    i = (g / 8 + g) % 8;
+                }
+                asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fb[s][j]), "v"(fa[s][i]));
+            }
     }
     // the compiler adds no wait states behind assembly MFMAs: a matrix op of N passes needs N + 3 of them (at
     // most 19) before a vector instruction may read its result
@@ -476,13 +496,17 @@ extern "C" int syn_probe_read_streams_skewed(const void* base, int64_t stream_by
 extern "C" int syn_probe_mfma_rate(float* sink, int32_t workgroups, int32_t iters, int32_t pattern,
                                    syn_stream_t stream) {
     using namespace syn;
-    if (sink == nullptr || workgroups <= 0 || iters <= 0 || pattern < 0 || (pattern & 3) > 2 || pattern > 6) return SYN_EINVAL;
-    if (pattern & 4)
-        hipLaunchKernelGGL(mfma16_rate_kernel, dim3(workgroups), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
-                           sink, iters, pattern & 3);
-    else
-        hipLaunchKernelGGL(mfma_rate_kernel, dim3(workgroups), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), sink,
-                           iters, pattern);
+    // bits 0-1: operands; 2: the MFMA; 4-5: the order, of the 16x16x32 form
+    const int order = pattern >> 4;
+    if (sink == nullptr || workgroups <= 0 || iters <= 0 || pattern < 0 || (pattern & 3) > 2 || (pattern & 8) || order > 3)
+        return SYN_EINVAL;
+    if (order != 0 && !(pattern & 4)) return SYN_EINVAL;
+    auto* const kernel = !(pattern & 4)              ? mfma_rate_kernel
+                         : order == kOrderPairs      ? mfma16_rate_kernel<kOrderPairs>
+                         : order == kOrderRows       ? mfma16_rate_kernel<kOrderRows>
+                         : order == kOrderToAndFro   ? mfma16_rate_kernel<kOrderToAndFro>
+                                                     : mfma16_rate_kernel<kOrderDiagonal>;
+    hipLaunchKernelGGL(kernel, dim3(workgroups), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), sink, iters, pattern & 3);
     return (int)hipGetLastError();
 }
 
