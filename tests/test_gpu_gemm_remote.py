@@ -189,3 +189,43 @@ def test_split_k_argument_errors(hip):
     with pytest.raises(ValueError, match="added into"):
         gemm_remote(a, b, [c], 8, 128, 128, cur_wave_sizes=[[256, 256]], wave_offsets=[[0, 0]], M=256,
                     target_rank=[0], dst_offsets=[[0, 0]], k_ranges=[[0, 128]], **kw)      # plain stores
+
+
+@pytest.mark.parametrize("atomic_add", [False, True])
+def test_replayed_launch_reads_tables_as_they_are(hip, atomic_add):
+    """Owners that a kernel in front of each replay of a captured launch writes, as the scalar loads of the look-up find them."""
+    from syncopate_amd.computation._launch import check_status
+    from syncopate_amd.computation.gemm import gemm_remote
+
+    world, rows, N, K = 4, 256, 256, 128
+    M = world * rows
+    g = torch.Generator(device="cuda").manual_seed(6)
+    a, b = ((0.1 * torch.randn(s, K, device="cuda", generator=g)).bfloat16() for s in (M, N))
+    shards = list(a.view(world, rows, K))
+    c = torch.zeros(world, rows, N, dtype=torch.bfloat16, device="cuda")
+    table = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    sizes, offsets, dst = table([[rows, N]] * world), table([[i * rows, 0] for i in range(world)]), table([[0, 0]] * world)
+    readers, owners = table(range(world)), table(range(world))
+    kw = dict(cur_wave_sizes=sizes, wave_offsets=offsets, M=M, a_target_rank=readers, target_rank=owners, dst_offsets=dst,
+              atomic_add=atomic_add)
+    launch = lambda: gemm_remote(shards, b, list(c), 3, 128, 128, 64, 8, **kw)      # 16 tiles on 3 programs
+    launch()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        launch()
+    got = []
+    for turn in range(6):
+        c.zero_()
+        torch.remainder(readers + 1, world, out=readers)
+        torch.remainder(3 * owners + turn, world, out=owners)         # (3 and 4 have no common divisor: still one wave each)
+        graph.replay()
+        got.append((c.clone(), readers.clone(), owners.clone()))
+    torch.cuda.synchronize()
+    check_status()
+    product = torch.stack([s.float() @ b.float().T for s in shards])
+    for out, r, o in got:
+        want = torch.empty_like(product)
+        want[o.long()] = product[r.long()]
+        # one rounding of the result (2^-9 relative), sums in 32 bits
+        assert (out.float() - want).abs().max() <= 4e-3 * want.abs().max()
